@@ -131,8 +131,9 @@ WM_EXPORT int wm_route_scored(const float* logits, const float* bias, int32_t to
                               void* stream);
 /* logits[t, e] = x[t] . w[e] for bf16 x [T, H] and bf16 w [E, H], fp32 out: the
  * router linear (SparseMoE.gate, qwen4_exp.py:1000; linear_bf16,
- * Native/QwenNative/kernels.metal:18-67). 64+ tokens with hidden a multiple of 32 run on
- * bf16 MFMA (the GEMM of wm_norm_router); fewer run one wave per output. */
+ * Native/QwenNative/kernels.metal:18-67). Up to 4 tokens stream the weight
+ * rows; more, with hidden a multiple of 32 and 16-byte aligned rows, run on bf16 MFMA; other
+ * operands one wave per output. */
 WM_EXPORT int wm_linear_bf16(const void* x, const void* w, int32_t tokens, int32_t hidden, int32_t outputs,
                              float* out, void* stream);
 
@@ -206,7 +207,8 @@ WM_EXPORT int wm_combine_pairs(const void* rows, const float* weights, int32_t t
  * MLP (qwen4_exp.py:763-771) with shared_expert_gate (:1002-1003, :1045); native
  * engine.mm:2075-2079. x [T, H], gate_w / up_w [I, H], down_w [H, I], gate_vec [H], add and y
  * [T, H], all bf16 and 16-byte aligned; add (nullable) may alias y. H and I multiples of
- * 32. Fewer than 64 tokens run two GEMV kernels, more the bf16 MFMA GEMM of wm_linear_bf16.
+ * 32. Up to 4 tokens run two GEMV kernels, more the bf16 MFMA GEMM of wm_linear_bf16; at 64 or
+ * more tokens H and I are at most 9568.
  * workspace: wm_mlp_bf16_workspace_size bytes. */
 WM_EXPORT size_t wm_mlp_bf16_workspace_size(int32_t tokens, int32_t hidden, int32_t inter);
 WM_EXPORT int wm_mlp_bf16(const void* x, int32_t tokens, int32_t hidden, int32_t inter, const void* gate_w,
@@ -274,14 +276,14 @@ WM_EXPORT int wm_kernel_timing_ms(float* out2);
  * without attention). residual fp32 [T, H], y and x bf16 [T, H]. */
 WM_EXPORT int wm_residual_rmsnorm(float* residual, const void* y, int32_t tokens, int32_t hidden, float eps,
                                   void* x, void* stream);
-/* The step before the MoE fused into one launch: v = residual + y (y nullable),
+/* The step before the MoE (one launch for few tokens, the norm and a GEMM for more): v = residual + y (y nullable),
  * x = bf16(v * rsqrt(mean(v^2) + eps) * norm_weight) (norm_weight nullable: unit),
  * logits[t, e] = x[t] . router[e] (fp32 [T, E]) and shared_logit[t] = x[t] . shared_gate
  * (both nullable together). residual_out (nullable, must not overlap residual) receives v.
  * bf16 y [T, H], norm_weight [H], router [E, H], shared_gate [H]; every pointer 16-byte
  * aligned, hidden a multiple of 8. router_packed (nullable) is the same rows from
- * wm_repack_router, router_packed_bytes its size; the prefill path (16+ tokens) then reads
- * it instead of router. Replaces the norm dispatch and the router / shared-gate linears
+ * wm_repack_router, router_packed_bytes its size: accepted and checked, but the GEMM reads
+ * router, whose rows it loads as fast. Replaces the norm dispatch and the router / shared-gate linears
  * before the expert step (Native/QwenNative/engine.mm:2074-2079; SparseMoE.gate and
  * shared_expert_gate, qwen4_exp.py:1000-1003); routing follows with wm_route_softmax_topk or
  * wm_route_scored on the device. */
@@ -290,7 +292,7 @@ WM_EXPORT int wm_norm_router(const float* residual, const void* y, const void* n
                              const void* router_packed, size_t router_packed_bytes, void* x,
                              float* residual_out, float* logits, float* shared_logit, void* stream);
 /* The router rows (and the shared gate row when shared_gate is set) in the fragment order of
- * wm_norm_router's prefill GEMM: [ceil((E + gate) / 16) + gate][H / 32][64] x 16 bytes,
+ * v_mfma_f32_16x16x32_bf16: [ceil((E + gate) / 16) + gate][H / 32][64] x 16 bytes,
  * zero-padded rows (the spare group with a gate makes the size tell whether it is packed). A one-time repack, like the prefill tile layout of the experts (no reference
  * counterpart: the reference's router weight stays [E, H]). hidden a multiple of 32. */
 WM_EXPORT size_t wm_router_packed_bytes(int32_t experts, int32_t hidden, int32_t has_gate);

@@ -27,7 +27,7 @@
 #include <cmath>
 #include <mutex>
 
-#include "wm_common.h"
+#include "lds_dma.h"
 #include "moe_internal.h"
 
 namespace wm {
@@ -62,24 +62,6 @@ __device__ __forceinline__ float pow2_biased(int e) { return __uint_as_float((ui
 // ---------------------------------------------------------------------------------
 // Loads and the persistent K loop.
 
-// Direct global -> LDS loads, lane i writing LDS address lds + size * i. Written as inline
-// assembly so the compiler does not treat them as LDS stores it must wait for before every
-// LDS read (it cannot tell the ring's stages apart); the K loop's explicit vmcnt waits and
-// barriers order them instead. M0 carries the wave-uniform LDS address (nothing else in
-// these kernels uses M0); an M0 write needs wait states before an LDS DMA reads it.
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
-}
-// The global address is a wave-uniform base in scalar registers plus a 32-bit per-lane
-// offset, so no 64-bit addresses occupy vector registers.
-__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory");
-}
-__device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 1\n\tglobal_load_lds_dword %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory");
-}
 // A pointer every lane holds, moved to scalar registers and read through the constant
 // address space, so the loads through it are scalar loads (waited for through lgkmcnt,
 // outside the vmcnt count of the ring's loads). For data the kernel never writes.

@@ -6,24 +6,23 @@
 // engine runs the same three linears with a mul_silu (Native/QwenNative/engine.mm:2075-2079).
 // Weights are bf16 [I, H] (gate, up) and [H, I] (down), y = x W^T as mlx nn.Linear.
 //
-// Few tokens (decode, < 64): two HBM-bound GEMV kernels.
-//   gate_up: a wave per intermediate row streams the gate and up rows (16 bytes per lane
-//            per load) against every token's x, reduces, and writes the bf16 act; block 0
-//            also computes each token's gate value.
-//   down:    a wave per output row streams the down row against the tokens' act and writes
-//            y = add + g * d (fp32 arithmetic, one bf16 rounding).
-// 64+ tokens: the bf16 MFMA GEMM of the router (norm_router.hip) for the three linears,
-// with an elementwise SwiGLU kernel between them and the gate / add in a final kernel.
+// Up to 4 tokens (decode): two GEMV kernels, a wave per intermediate row (gate and up rows)
+// and a wave per output row, four 16-byte chunks of each row and of every token in flight.
+// More: the bf16 GEMM of gemm_bf16.hip twice, with the SwiGLU and the tokens' gate values in
+// the first launch and the gate and add in the second.
+// Measured (hidden 2560, intermediate 640): 8 tokens 24.3 us as GEMVs that looped over the
+// tokens, now 14.6; 301 tokens about 290 us as three GEMMs with separate activation, gate and
+// output passes, now 23; 2048 tokens 430, now 49.
 #include <cmath>
 
-#include "wm_common.h"
+#include "gemm_bf16.h"
 
 namespace wm {
 
-bool linear_bf16_mfma(const void* x, const void* w, int tokens, int hidden, int outputs, float* out, hipStream_t s);
-bool linear_bf16_mfma_fits(int tokens, int hidden);
+// The widths of the interface at 64 or more tokens.
+constexpr int MLP_MAX_WIDTH = 9568;
 
-constexpr int MLP_GEMV_MAX_TOKENS = 63;
+constexpr int MLP_GEMV_MAX_TOKENS = 4;
 
 // dot of 8 bf16 (one 16-byte chunk) against 8 bf16
 __device__ __forceinline__ float dot8_bf16(uint4 a, uint4 b, float acc) {
@@ -44,7 +43,43 @@ __device__ __forceinline__ float wave_gate(const uint16_t* __restrict__ xr, cons
   return 1.0f / (1.0f + __expf(-a));
 }
 
-// grid: ceil(I / 4); wave w of block b owns intermediate row i = 4 b + w.
+// Dot products of R weight rows with the rows of TMAX tokens, 64 chunks a step, UNROLL
+// steps in flight; chunks past the end read the last one and are not used.
+template <int TMAX, int R, int UNROLL>
+__device__ __forceinline__ void wave_dots(const uint4* const (&wr)[R], const uint4* __restrict__ x, int tokens,
+                                          int chunks, int lane, float (&acc)[R][TMAX]) {
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int t = 0; t < TMAX; ++t) acc[r][t] = 0.0f;
+  for (int c0 = lane; c0 - lane < chunks; c0 += 64 * UNROLL) {
+    uint4 wv[UNROLL][R], xv[UNROLL][TMAX];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int c = min(c0 + 64 * u, chunks - 1);
+#pragma unroll
+      for (int r = 0; r < R; ++r) wv[u][r] = gload16(&wr[r][c]);
+#pragma unroll
+      for (int t = 0; t < TMAX; ++t) xv[u][t] = gload16(&x[(int64_t)min(t, tokens - 1) * chunks + c]);
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if (c0 + 64 * u >= chunks) continue;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int t = 0; t < TMAX; ++t) acc[r][t] = dot8_bf16(wv[u][r], xv[u][t], acc[r][t]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int t = 0; t < TMAX; ++t) acc[r][t] = segment_sum<64>(acc[r][t]);
+}
+
+// grid: ceil(I / 4) + 1; wave w of block b owns intermediate row i = 4 b + w; the last block
+// the tokens' gate values.
+template <int TMAX>
 __global__ void __launch_bounds__(256) mlp_gate_up_gemv_kernel(const uint16_t* __restrict__ x, int tokens, int hidden,
                                                                int inter, const uint16_t* __restrict__ wg,
                                                                const uint16_t* __restrict__ wu,
@@ -52,82 +87,48 @@ __global__ void __launch_bounds__(256) mlp_gate_up_gemv_kernel(const uint16_t* _
                                                                uint16_t* __restrict__ act, float* __restrict__ gate) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int i = blockIdx.x * 4 + wave;
-  if (blockIdx.x == 0)
-    for (int t = wave; t < tokens; t += 4) {
-      const float g = wave_gate(x + (int64_t)t * hidden, gate_vec, hidden, lane);
-      if (lane == 0) gate[t] = g;
+  if (blockIdx.x == gridDim.x - 1) {
+    if (wave < tokens) {  // at most 4 tokens
+      const float g = wave_gate(x + (int64_t)wave * hidden, gate_vec, hidden, lane);
+      if (lane == 0) gate[wave] = g;
     }
-  if (i >= inter) return;
-  const uint4* gr = reinterpret_cast<const uint4*>(wg + (int64_t)i * hidden);
-  const uint4* ur = reinterpret_cast<const uint4*>(wu + (int64_t)i * hidden);
-  const int chunks = hidden / 8;
-  for (int t = 0; t < tokens; ++t) {
-    const uint4* xr = reinterpret_cast<const uint4*>(x + (int64_t)t * hidden);
-    float g = 0.0f, u = 0.0f;
-    for (int c = lane; c < chunks; c += 64) {
-      const uint4 xv = xr[c];
-      g = dot8_bf16(gr[c], xv, g);
-      u = dot8_bf16(ur[c], xv, u);
-    }
-    g = segment_sum<64>(g);
-    u = segment_sum<64>(u);
-    if (lane == 0) act[(int64_t)t * inter + i] = f32_to_bf16_bits(silu(g) * u);
+    return;
   }
+  if (i >= inter) return;
+  const uint4* rows[2] = {reinterpret_cast<const uint4*>(wg + (int64_t)i * hidden),
+                          reinterpret_cast<const uint4*>(wu + (int64_t)i * hidden)};
+  float acc[2][TMAX];
+  wave_dots<TMAX, 2, 4>(rows, reinterpret_cast<const uint4*>(x), tokens, hidden / 8, lane, acc);
+#pragma unroll
+  for (int t = 0; t < TMAX; ++t)
+    if (t < tokens && lane == 0) act[(int64_t)t * inter + i] = f32_to_bf16_bits(silu(acc[0][t]) * acc[1][t]);
 }
 
 // grid: ceil(H / 4); wave w of block b owns output row o = 4 b + w.
+template <int TMAX>
 __global__ void __launch_bounds__(256) mlp_down_gemv_kernel(const uint16_t* __restrict__ act, int tokens, int hidden,
                                                             int inter, const uint16_t* __restrict__ wd,
-                                                            const float* __restrict__ gate,
-                                                            const uint16_t* __restrict__ add,
-                                                            uint16_t* __restrict__ y) {
+                                                            const float* __restrict__ gate, const uint16_t* add,
+                                                            uint16_t* y) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int o = blockIdx.x * 4 + wave;
   if (o >= hidden) return;
-  const uint4* dr = reinterpret_cast<const uint4*>(wd + (int64_t)o * inter);
-  const int chunks = inter / 8;
-  for (int t = 0; t < tokens; ++t) {
-    const uint4* ar = reinterpret_cast<const uint4*>(act + (int64_t)t * inter);
-    float d = 0.0f;
-    for (int c = lane; c < chunks; c += 64) d = dot8_bf16(dr[c], ar[c], d);
-    d = segment_sum<64>(d);
-    if (lane == 0) {
-      float v = gate[t] * d;
+  const uint4* rows[1] = {reinterpret_cast<const uint4*>(wd + (int64_t)o * inter)};
+  float acc[1][TMAX];
+  wave_dots<TMAX, 1, 4>(rows, reinterpret_cast<const uint4*>(act), tokens, inter / 8, lane, acc);
+#pragma unroll
+  for (int t = 0; t < TMAX; ++t)
+    if (t < tokens && lane == 0) {
+      float v = gate[t] * acc[0][t];
       if (add) v += bf16_bits_to_f32(add[(int64_t)t * hidden + o]);
       y[(int64_t)t * hidden + o] = f32_to_bf16_bits(v);
     }
-  }
-}
-
-// act[t, i] = bf16(silu(g[t, i]) * u[t, i]) for the MFMA path; one thread per element.
-__global__ void __launch_bounds__(256) mlp_act_kernel(const float* __restrict__ g, const float* __restrict__ u,
-                                                      int64_t n, uint16_t* __restrict__ act) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e < n) act[e] = f32_to_bf16_bits(silu(g[e]) * u[e]);
-}
-
-// gate[t] for the MFMA path: one wave per token.
-__global__ void __launch_bounds__(64) mlp_gate_kernel(const uint16_t* __restrict__ x, int hidden,
-                                                      const uint16_t* __restrict__ gate_vec, float* __restrict__ gate) {
-  const float g = wave_gate(x + (int64_t)blockIdx.x * hidden, gate_vec, hidden, threadIdx.x);
-  if (threadIdx.x == 0) gate[blockIdx.x] = g;
-}
-
-// y[t, o] = bf16(add[t, o] + gate[t] * d[t, o]); one thread per element.
-__global__ void __launch_bounds__(256) mlp_out_kernel(const float* __restrict__ d, const float* __restrict__ gate,
-                                                      const uint16_t* __restrict__ add, int hidden, int64_t n,
-                                                      uint16_t* __restrict__ y) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (e >= n) return;
-  float v = gate[e / hidden] * d[e];
-  if (add) v += bf16_bits_to_f32(add[e]);
-  y[e] = f32_to_bf16_bits(v);
 }
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 struct MlpLayout {
-  size_t gate, act, g, u, d, total;
+  size_t gate, act, total;
 };
 
 static MlpLayout mlp_layout(int tokens, int hidden, int inter) {
@@ -136,11 +137,6 @@ static MlpLayout mlp_layout(int tokens, int hidden, int inter) {
   const size_t T = tokens > 0 ? (size_t)tokens : 1;
   p.gate = at; at += align256(sizeof(float) * T);
   p.act = at;  at += align256(sizeof(uint16_t) * T * inter);
-  if (tokens > MLP_GEMV_MAX_TOKENS) {
-    p.g = at; at += align256(sizeof(float) * T * inter);
-    p.u = at; at += align256(sizeof(float) * T * inter);
-    p.d = at; at += align256(sizeof(float) * T * hidden);
-  }
   p.total = at;
   return p;
 }
@@ -168,39 +164,51 @@ WM_EXPORT int wm_mlp_bf16(const void* x, int32_t tokens, int32_t hidden, int32_t
       if ((uintptr_t)p % 16) fail("wm_mlp_bf16: every tensor must be 16-byte aligned");
     const MlpLayout p = mlp_layout(tokens, hidden, inter);
     if (workspace_bytes < p.total) fail("wm_mlp_bf16: workspace too small");
-    // every GEMM of the MFMA path is checked before the first launch, so a shape it cannot
-    // hold launches nothing
-    if (tokens > MLP_GEMV_MAX_TOKENS && (!linear_bf16_mfma_fits(tokens, hidden) || !linear_bf16_mfma_fits(tokens, inter)))
-      fail("wm_mlp_bf16: hidden or intermediate too large for the MFMA GEMM's x tile (150 KB of LDS)");
+    if (tokens >= 64 && (hidden > MLP_MAX_WIDTH || inter > MLP_MAX_WIDTH))
+      fail("wm_mlp_bf16: hidden or intermediate too large at 64 or more tokens (at most " +
+           std::to_string(MLP_MAX_WIDTH) + ")");
     hipStream_t s = as_stream(stream);
     uint8_t* ws = (uint8_t*)workspace;
     float* gate = (float*)(ws + p.gate);
     uint16_t* act = (uint16_t*)(ws + p.act);
     const uint16_t *xb = (const uint16_t*)x, *gv = (const uint16_t*)gate_vec, *ab = (const uint16_t*)add;
     if (tokens <= MLP_GEMV_MAX_TOKENS) {
-      hipLaunchKernelGGL(mlp_gate_up_gemv_kernel, dim3((inter + 3) / 4), dim3(256), 0, s, xb, tokens, hidden, inter,
-                         (const uint16_t*)gate_w, (const uint16_t*)up_w, gv, act, gate);
-      check_launch("mlp_gate_up_gemv");
-      hipLaunchKernelGGL(mlp_down_gemv_kernel, dim3((hidden + 3) / 4), dim3(256), 0, s, act, tokens, hidden, inter,
-                         (const uint16_t*)down_w, gate, ab, (uint16_t*)y);
-      check_launch("mlp_down_gemv");
+#define WM_MLP(T)                                                                                                     \
+  do {                                                                                                                \
+    hipLaunchKernelGGL(mlp_gate_up_gemv_kernel<T>, dim3((inter + 3) / 4 + 1), dim3(256), 0, s, xb, tokens, hidden,    \
+                       inter, (const uint16_t*)gate_w, (const uint16_t*)up_w, gv, act, gate);                         \
+    check_launch("mlp_gate_up_gemv");                                                                                 \
+    hipLaunchKernelGGL(mlp_down_gemv_kernel<T>, dim3((hidden + 3) / 4), dim3(256), 0, s, act, tokens, hidden, inter,  \
+                       (const uint16_t*)down_w, gate, ab, (uint16_t*)y);                                              \
+    check_launch("mlp_down_gemv");                                                                                    \
+  } while (0)
+      if (tokens <= 1) WM_MLP(1);
+      else if (tokens <= 2) WM_MLP(2);
+      else WM_MLP(4);
+#undef WM_MLP
       return;
     }
-    float* g = (float*)(ws + p.g);
-    float* u = (float*)(ws + p.u);
-    float* d = (float*)(ws + p.d);
-    if (!linear_bf16_mfma(x, gate_w, tokens, hidden, inter, g, s) || !linear_bf16_mfma(x, up_w, tokens, hidden, inter, u, s))
-      fail("wm_mlp_bf16: the gate/up GEMM does not support this shape");
-    const int64_t ni = (int64_t)tokens * inter, nh = (int64_t)tokens * hidden;
-    hipLaunchKernelGGL(mlp_act_kernel, dim3((unsigned)((ni + 255) / 256)), dim3(256), 0, s, g, u, ni, act);
-    check_launch("mlp_act");
-    hipLaunchKernelGGL(mlp_gate_kernel, dim3(tokens), dim3(64), 0, s, xb, hidden, gv, gate);
-    check_launch("mlp_gate");
-    if (!linear_bf16_mfma(act, down_w, tokens, inter, hidden, d, s))
-      fail("wm_mlp_bf16: the down GEMM does not support this shape");
-    hipLaunchKernelGGL(mlp_out_kernel, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, s, d, gate, ab, hidden, nh,
-                       (uint16_t*)y);
-    check_launch("mlp_out");
+    GemmArgs g{};
+    g.x = xb;
+    g.w = (const uint16_t*)gate_w;
+    g.w2 = (const uint16_t*)up_w;
+    g.tokens = tokens;
+    g.k = hidden;
+    g.n = inter;
+    g.out16 = act;
+    g.vec = gv;
+    g.vec_out = gate;
+    gemm_bf16(GEMM_SWIGLU, g, s);
+    GemmArgs d{};
+    d.x = act;
+    d.w = (const uint16_t*)down_w;
+    d.tokens = tokens;
+    d.k = inter;
+    d.n = hidden;
+    d.out16 = (uint16_t*)y;
+    d.gate = gate;
+    d.add = ab;
+    gemm_bf16(GEMM_DOWN, d, s);
   });
 }
 

@@ -1,31 +1,29 @@
-// The step before the MoE in one launch: the residual add and RMSNorm that produce the
+// The step before the MoE: the residual add and RMSNorm that produce the
 // expert input, with the router GEMV and the shared expert's gate GEMV fused into the
 // norm's epilogue:
 //   v = r + y (y optional),  x = bf16(v * rsqrt(mean(v^2) + eps) * w_norm)  (w_norm optional),
 //   logits[t, e] = x[t] . W_router[e],  shared_logit[t] = x[t] . g.
 // The reference runs these as separate dispatches (the norm, then linear(router),
 // linear(shared_gate): Native/QwenNative/engine.mm:2074-2079, with the norm in the
-// hyper-connection mix before it); fused, the expert input is built once per block in
-// LDS and never re-read from HBM for the GEMVs, and routing (wm_route_softmax_topk /
-// wm_route_scored) follows on the device with no host step.
+// hyper-connection mix before it). Routing (wm_route_softmax_topk / wm_route_scored) follows
+// on the device with no host step.
 //
-// Grid (row blocks, token blocks). A block owns TB tokens and RB consecutive output rows
+// Few tokens: one launch, the expert input built once per block in LDS. Grid (row blocks,
+// token blocks); a block owns TB tokens and RB consecutive output rows
 // (router rows, then the gate row as row E). Every block recomputes the norm of its TB
 // tokens (r and y are L2-resident after the first block of a token group) and keeps x as
 // a [TB][H] bf16 tile in LDS (TB up to 16, within 96 KB); row block 0 also writes x and
 // r + y to HBM. Each wave takes rows wave, wave + 4, ...: a lane streams 16-byte chunks
 // of the weight row once and
 // applies each to the TB tokens' x chunks (V_DOT2_F32_BF16), then one wave reduction
-// per token.
+// per token. More tokens: the norm and the GEMM as two launches (residual_norm_kernel).
 #include <algorithm>
 #include <cmath>
 
+#include "gemm_bf16.h"
 #include "moe_internal.h"
 
 namespace wm {
-
-typedef __bf16 nr_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float nr_f32x4 __attribute__((ext_vector_type(4)));
 
 // Statistics of v = r + y for tokens t0 .. t0 + nt, then the x tile [TB][stride] (uint4 =
 // 8 bf16; tokens past nt are zero). The writer block also stores x and v to HBM. Ends with
@@ -34,17 +32,9 @@ template <int TB>
 __device__ __forceinline__ void build_x_tile(const float* __restrict__ r, const uint16_t* __restrict__ y,
                                              const uint16_t* __restrict__ nw, int t0, int nt, int hidden, float eps,
                                              bool writer, uint16_t* __restrict__ x_out, float* __restrict__ r_out,
-                                             uint4* tile, int stride, float* inv_s,
-                                             const uint16_t* __restrict__ xin = nullptr) {
+                                             uint4* tile, int stride, float* inv_s) {
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int chunks = hidden / 8;
-  if (xin) {  // a plain linear: the tile is the given bf16 rows
-    for (int t = 0; t < TB; ++t)
-      for (int c = threadIdx.x; c < chunks; c += 256)
-        tile[t * stride + c] = t < nt ? ((const uint4*)(xin + (int64_t)(t0 + t) * hidden))[c] : make_uint4(0, 0, 0, 0);
-    __syncthreads();
-    return;
-  }
   constexpr int QU = 8;  // float4 loads in flight per lane
   const int quads = hidden / 4;
   for (int t = wave; t < nt; t += 4) {
@@ -210,16 +200,6 @@ __global__ void __launch_bounds__(256) norm_router_kernel(
   }
 }
 
-// Many tokens (prefill): the router GEMM on MFMA. A block owns TB tokens (8 or 16 columns
-// of V_MFMA_F32_16X16X32_BF16; columns past TB are zero) and every output row; the x tile
-// rows are padded by 16 bytes so the 16 tokens' reads fall on distinct banks. Wave w
-// takes 16-row groups w, w + 4, ... four at a time: per 32-wide K step, four weight
-// fragments (16 bytes per lane, loaded four steps ahead) against one x fragment.
-// Operands: lane l holds row / token l % 16 and K chunk (l / 16) of each 32-wide step (the
-// same lane-to-K map for both, so the K order inside a step cancels); the result holds
-// token l % 16 for rows 4 (l / 16) .. +3 of the group. With `packed` (wm_repack_router)
-// each fragment is one contiguous 1 KB read instead of 16 rows x 64 bytes.
-
 // The packed router: [groups][hidden / 32][64 lanes] uint4, lane l of group g and step s
 // holding row 16 g + l % 16 (router rows, then the gate row, then zeros; one spare zero
 // group follows when the gate is packed), 8 values from column 32 s + 8 (l / 16).
@@ -238,99 +218,110 @@ __global__ void __launch_bounds__(256) repack_router_kernel(const uint4* __restr
     packed[o] = v;
   }
 }
-template <int TB>
-__global__ void __launch_bounds__(256) norm_router_mfma_kernel(
-    const float* __restrict__ r, const uint16_t* __restrict__ y, const uint16_t* __restrict__ nw, int tokens,
-    int hidden, float eps, const uint16_t* __restrict__ router, int experts, const uint16_t* __restrict__ gate,
-    const uint4* __restrict__ packed, uint16_t* __restrict__ x_out, float* __restrict__ r_out,
-    float* __restrict__ logits, float* __restrict__ shared_logit, const uint16_t* __restrict__ xin) {
-  extern __shared__ uint4 x_tile[];  // [TB][hidden / 8 + 1]
-  __shared__ float inv_s[TB];
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int t0 = blockIdx.x * TB;
-  const int nt = min(TB, tokens - t0);
-  const int chunks = hidden / 8, stride = chunks + 1, steps = hidden / 32;
-  build_x_tile<TB>(r, y, nw, t0, nt, hidden, eps, xin == nullptr, x_out, r_out, x_tile, stride, inv_s, xin);
 
-  const int rows = experts + (gate ? 1 : 0);
-  const int groups = (rows + 15) / 16;
-  const int n = lane % 16, kq = lane / 16;
-  constexpr int NCOL = TB > 16 ? TB / 16 : 1;  // 16-token column blocks
-  const uint4* xb[NCOL];
-  bool has_col[NCOL];
+__device__ __forceinline__ float4 load_nt(const float4* p) {
+  const wm_f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const wm_f32x4*>(p));
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+typedef uint32_t nr_u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 load_nt(const uint2* p) {
+  const nr_u32x2 v = __builtin_nontemporal_load(reinterpret_cast<const nr_u32x2*>(p));
+  return make_uint2(v.x, v.y);
+}
+// Many tokens: the norm as a kernel of its own (a block per token), then the GEMM of
+// gemm_bf16.hip on its x. The norm passes r, y, x and r + y through memory once, which is
+// what bounds a long prompt (r and y are read once: non-temporal loads, 53.8 -> 50.7 us for
+// 4000 tokens of 2560 with 512 experts); the shared gate's dot product rides on the row in
+// registers. In one launch every block held 8 to 32 tokens' whole rows in LDS for the GEMM and
+// passed all the router rows: 120 us for the same 4000 tokens.
+// Q: float4 values per thread (hidden <= 1024 Q).
+template <int Q>
+__global__ void __launch_bounds__(256) residual_norm_kernel(const float* __restrict__ r, const uint16_t* __restrict__ y,
+                                                            const uint16_t* __restrict__ nw, int hidden, float eps,
+                                                            const uint16_t* __restrict__ gate,
+                                                            uint16_t* __restrict__ x_out, float* __restrict__ r_out,
+                                                            float* __restrict__ shared_logit) {
+  __shared__ float part[2][4];
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int quads = hidden / 4;
+  const int64_t row = (int64_t)blockIdx.x * hidden;
+  const float4* rr = (const float4*)(r + row);
+  const uint2* yy = y ? (const uint2*)(y + row) : nullptr;
+  float4 v[Q];
+  uint2 b[Q];
 #pragma unroll
-  for (int cb = 0; cb < NCOL; ++cb) {
-    has_col[cb] = 16 * cb + n < TB;
-    xb[cb] = x_tile + (has_col[cb] ? 16 * cb + n : 0) * stride + kq;
+  for (int j = 0; j < Q; ++j) {
+    const int q = min((int)threadIdx.x + 256 * j, quads - 1);
+    v[j] = load_nt(rr + q);
+    b[j] = yy ? load_nt(yy + q) : make_uint2(0, 0);
   }
-  for (int g0 = wave; g0 < groups; g0 += 16) {
-    const uint4* wp[4];
-    const int wstep = packed ? 64 : 4;  // uint4s from one K step's fragment to the next
+  float ss = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = (g0 + 4 * j) * 16 + n;
-      if (packed)  // fragment-major: group g's step-s fragment is 64 consecutive uint4, one per lane
-        wp[j] = packed + (int64_t)min(g0 + 4 * j, groups - 1) * steps * 64 + lane;
-      else
-        wp[j] = weight_row(router, gate, experts, hidden, e < rows ? e : 0) + kq;
+  for (int j = 0; j < Q; ++j) {
+    v[j].x += bf16_bits_to_f32(b[j].x & 0xffffu);
+    v[j].y += bf16_bits_to_f32(b[j].x >> 16);
+    v[j].z += bf16_bits_to_f32(b[j].y & 0xffffu);
+    v[j].w += bf16_bits_to_f32(b[j].y >> 16);
+    if ((int)threadIdx.x + 256 * j < quads) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
+  }
+  ss = segment_sum<64>(ss);
+  if (lane == 0) part[0][wave] = ss;
+  __syncthreads();
+  const float inv = rsqrtf(((part[0][0] + part[0][1]) + (part[0][2] + part[0][3])) / (float)hidden + eps);
+  float dot = 0.0f;
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const int q = threadIdx.x + 256 * j;
+    if (q >= quads) continue;
+    float f[4] = {v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv};
+    if (nw) {
+      const uint2 n = ((const uint2*)nw)[q];
+      f[0] *= bf16_bits_to_f32(n.x & 0xffffu);
+      f[1] *= bf16_bits_to_f32(n.x >> 16);
+      f[2] *= bf16_bits_to_f32(n.y & 0xffffu);
+      f[3] *= bf16_bits_to_f32(n.y >> 16);
     }
-    // four K steps of fragments in flight: set u holds step s + u
-    constexpr int PD = 4;
-    nr_f32x4 acc[4][NCOL];
-    uint4 a[PD][4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int cb = 0; cb < NCOL; ++cb) acc[j][cb] = nr_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int u = 0; u < PD; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (g0 + 4 * j < groups) a[u][j] = wp[j][wstep * (u < steps ? u : 0)];
-    for (int s = 0; s < steps; s += PD) {
-#pragma unroll
-      for (int u = 0; u < PD; ++u) {
-        if (s + u < steps) {
-          uint4 bv[NCOL];
-#pragma unroll
-          for (int cb = 0; cb < NCOL; ++cb) bv[cb] = has_col[cb] ? xb[cb][4 * (s + u)] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if (g0 + 4 * j >= groups) break;  // wave-uniform: a last batch with fewer groups
-#pragma unroll
-            for (int cb = 0; cb < NCOL; ++cb)
-              acc[j][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(nr_bf16x8, a[u][j]),
-                                                                   __builtin_bit_cast(nr_bf16x8, bv[cb]), acc[j][cb],
-                                                                   0, 0, 0);
-            if (s + u + PD < steps) a[u][j] = wp[j][wstep * (s + u + PD)];
-          }
-        }
-      }
+    const uint2 xv = make_uint2((uint32_t)f32_to_bf16_bits(f[0]) | ((uint32_t)f32_to_bf16_bits(f[1]) << 16),
+                                (uint32_t)f32_to_bf16_bits(f[2]) | ((uint32_t)f32_to_bf16_bits(f[3]) << 16));
+    ((uint2*)(x_out + row))[q] = xv;
+    if (r_out) ((float4*)(r_out + row))[q] = v[j];
+    if (gate) {
+      const uint2 g = ((const uint2*)gate)[q];
+      dot = dot2_bf16(bits_to_bf16x2(xv.x), bits_to_bf16x2(g.x), dot);
+      dot = dot2_bf16(bits_to_bf16x2(xv.y), bits_to_bf16x2(g.y), dot);
     }
-#pragma unroll
-    for (int cb = 0; cb < NCOL; ++cb) {
-      const int t = 16 * cb + n;
-      if (t >= nt) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int e = (g0 + 4 * j) * 16 + 4 * kq + i;
-          if (e < rows) store_row(logits, shared_logit, experts, t0 + t, e, acc[j][cb][i]);
-        }
-    }
+  }
+  if (gate) {
+    dot = segment_sum<64>(dot);
+    if (lane == 0) part[1][wave] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) shared_logit[blockIdx.x] = (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]);
   }
 }
 
-// The MFMA path's token block: 32 tokens (two column blocks per weight fragment) or 16 when
-// the padded x tile fits 150 KB of LDS, else 8; 0 (the dot-product path) below 16 tokens or
-// when hidden is not a multiple of 32.
-static int mfma_token_block(int tokens, int hidden) {
-  if (tokens < 16 || hidden % 32) return 0;
-  if (tokens >= 32 && (size_t)32 * (hidden / 8 + 1) * 16 + 128 <= 150 * 1024) return 32;
-  for (int tb : {16, 8})
-    if ((size_t)tb * (hidden / 8 + 1) * 16 + 64 <= 150 * 1024) return tb;
-  return 0;
+constexpr int NORM_MAX_HIDDEN = 10240;
+// Tokens from which the two launches are faster than the fused kernel below (hidden 2560, 512
+// experts: 4 tokens 10.9 us against 9.1, 8 tokens 11.6 against 15.8; hidden 7168, 256 experts, whose GEMM has half
+// the blocks: 8 tokens 18.8 against 18.0, 15 tokens 21.3 against 17.5).
+static int norm_gemm_min_tokens(int hidden) { return hidden <= 4096 ? 8 : 16; }
+
+static void residual_norm(const float* r, const uint16_t* y, const uint16_t* nw, int tokens, int hidden, float eps,
+                          const uint16_t* gate, uint16_t* x, float* r_out, float* shared_logit, hipStream_t s) {
+#define WM_RN(Q) hipLaunchKernelGGL(residual_norm_kernel<Q>, dim3(tokens), dim3(256), 0, s, r, y, nw, hidden, eps, gate, \
+                                    x, r_out, shared_logit)
+  switch ((hidden + 1023) / 1024) {
+    case 1: WM_RN(1); break;
+    case 2: WM_RN(2); break;
+    case 3: WM_RN(3); break;
+    case 4: WM_RN(4); break;
+    case 5: WM_RN(5); break;
+    case 6: WM_RN(6); break;
+    case 7: WM_RN(7); break;
+    case 8: WM_RN(8); break;
+    default: WM_RN(10); break;
+  }
+#undef WM_RN
+  check_launch("residual_norm");
 }
 
 // The dot-product path's token block: the largest whose x tile (plus the 64-byte
@@ -339,28 +330,6 @@ static int pick_token_block(int tokens, int hidden) {
   const int fit = (96 * 1024 - 64) / (hidden * 2);
   for (int tb : {16, 8, 4, 2}) if (tb <= fit && tokens >= tb) return tb;
   return 1;
-}
-
-// logits = x . w^T on the router GEMM's MFMA path (a tile of x as given, no norm), for
-// wm_linear_bf16 at 64+ tokens. False when the shape does not suit it (the caller then uses
-// the one-wave-per-output kernel).
-// Whether linear_bf16_mfma takes x [tokens, hidden] (its x tile must fit the LDS).
-bool linear_bf16_mfma_fits(int tokens, int hidden) { return tokens >= 64 && mfma_token_block(tokens, hidden) > 0; }
-
-bool linear_bf16_mfma(const void* x, const void* w, int tokens, int hidden, int outputs, float* out, hipStream_t s) {
-  const int tb = tokens >= 64 ? mfma_token_block(tokens, hidden) : 0;
-  if (!tb || ((uintptr_t)x % 16) || ((uintptr_t)w % 16)) return false;
-  const int blocks = (tokens + tb - 1) / tb;
-  const size_t lds = (size_t)tb * (hidden / 8 + 1) * 16;
-#define WM_LIN(TB) hipLaunchKernelGGL(norm_router_mfma_kernel<TB>, dim3(blocks), dim3(256), lds, s, nullptr, nullptr, \
-                                      nullptr, tokens, hidden, 0.0f, (const uint16_t*)w, outputs, nullptr, nullptr, \
-                                      nullptr, nullptr, out, nullptr, (const uint16_t*)x)
-  if (tb == 32) WM_LIN(32);
-  else if (tb == 16) WM_LIN(16);
-  else WM_LIN(8);
-#undef WM_LIN
-  check_launch("linear_bf16 (MFMA)");
-  return true;
 }
 
 }  // namespace wm
@@ -420,20 +389,17 @@ WM_EXPORT int wm_norm_router(const float* residual, const void* y, const void* n
       if (p && ((uintptr_t)p % 16)) fail("wm_norm_router: tensors must be 16-byte aligned");
     hipStream_t s = as_stream(stream);
     const int rows = experts + (shared_gate ? 1 : 0);
-    const int mfma_tb = mfma_token_block(tokens, hidden);
-    if (mfma_tb) {
-      const int blocks = (tokens + mfma_tb - 1) / mfma_tb;
-      const size_t lds = (size_t)mfma_tb * (hidden / 8 + 1) * 16;
-#define WM_NRM(TB) hipLaunchKernelGGL(norm_router_mfma_kernel<TB>, dim3(blocks), dim3(256), lds, s, residual, \
-                                      (const uint16_t*)y, (const uint16_t*)norm_weight, tokens, hidden, eps, \
-                                      (const uint16_t*)router, experts, (const uint16_t*)shared_gate, \
-                                      (const uint4*)router_packed, (uint16_t*)x, residual_out, logits, shared_logit, \
-                                      nullptr)
-      if (mfma_tb == 32) WM_NRM(32);
-      else if (mfma_tb == 16) WM_NRM(16);
-      else WM_NRM(8);
-#undef WM_NRM
-      check_launch("norm_router_mfma");
+    if (tokens >= norm_gemm_min_tokens(hidden) && hidden <= NORM_MAX_HIDDEN && gemm_bf16_fits(x, router, hidden)) {
+      residual_norm(residual, (const uint16_t*)y, (const uint16_t*)norm_weight, tokens, hidden, eps,
+                    (const uint16_t*)shared_gate, (uint16_t*)x, residual_out, shared_logit, s);
+      GemmArgs g{};
+      g.x = (const uint16_t*)x;
+      g.w = (const uint16_t*)router;
+      g.tokens = tokens;
+      g.k = hidden;
+      g.n = experts;
+      g.out = logits;
+      gemm_bf16(GEMM_F32, g, s);
       return;
     }
     const int tb = pick_token_block(tokens, hidden);

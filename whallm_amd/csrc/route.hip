@@ -3,11 +3,10 @@
 // One wave64 per token; the top-k rule and register layout are in route_device.h.
 #include <cmath>
 
+#include "gemm_bf16.h"
 #include "route_device.h"
 
 namespace wm {
-
-bool linear_bf16_mfma(const void* x, const void* w, int tokens, int hidden, int outputs, float* out, hipStream_t s);
 
 constexpr int ROUTE_MAX_K = 32;
 
@@ -190,41 +189,66 @@ __device__ __forceinline__ float dot8_bf16x(uint4 a, uint4 b, float acc) {
   return dot2_bf16(bits_to_bf16x2(a.w), bits_to_bf16x2(b.w), acc);
 }
 
-// Few tokens (<= TMAX): a wave takes LR_ROWS output rows and streams them once in 16-byte
-// chunks (non-temporal loads: the rows are read once per call, 3% off the C5 verify step); each chunk of every token's x, loaded once per wave, meets all LR_ROWS rows, so x
-// is read from the caches once per LR_ROWS rows (one x pass per row made x, not the
-// weights, the larger read at 4 tokens). grid: ceil(outputs / (4 LR_ROWS)), 4 waves a block.
+// Few tokens (<= TMAX): a wave takes ROWS output rows and streams them once in 16-byte
+// chunks; each chunk of every token's x, loaded once per wave, meets all ROWS rows.
+// grid: ceil(outputs / (4 ROWS)), 4 waves a block.
+// ROWS 4, for many outputs: x is read from the caches once per 4 rows (one x pass per row made x,
+// not the weights, the larger read at 4 tokens); non-temporal weight loads (3% off a verify step).
+// ROWS 1, below LR_MIN_OUTPUTS: a wave per row puts four times the waves on the few rows, and
+// eight chunks of the row and of every x are in flight at once: one memory round trip for 4096
+// values (512 rows of 2560, 1 token: 2.3 us against 4.9 with 4 rows and two chunks in flight).
 constexpr int LR_ROWS = 4;
-template <int TMAX>
+constexpr int LR_MIN_OUTPUTS = 4096;
+template <int TMAX, int ROWS>
 __global__ void __launch_bounds__(256) linear_rows_kernel(const uint4* __restrict__ x, const uint4* __restrict__ w,
                                                          int tokens, int chunks, int outputs, float* __restrict__ out) {
+  constexpr int UNROLL = ROWS == 1 ? 8 : 2;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int o0 = (blockIdx.x * 4 + wave) * LR_ROWS;
+  const int o0 = (blockIdx.x * 4 + wave) * ROWS;
   if (o0 >= outputs) return;
-  const uint4* wr[LR_ROWS];
+  const uint4* wr[ROWS];
 #pragma unroll
-  for (int r = 0; r < LR_ROWS; ++r) wr[r] = w + (int64_t)min(o0 + r, outputs - 1) * chunks;  // in bounds
-  float acc[LR_ROWS][TMAX];
+  for (int r = 0; r < ROWS; ++r) wr[r] = w + (int64_t)min(o0 + r, outputs - 1) * chunks;  // in bounds
+  float acc[ROWS][TMAX];
 #pragma unroll
-  for (int r = 0; r < LR_ROWS; ++r)
+  for (int r = 0; r < ROWS; ++r)
 #pragma unroll
     for (int t = 0; t < TMAX; ++t) acc[r][t] = 0.0f;
+  if constexpr (ROWS == 1) {
+    for (int c0 = lane; c0 - lane < chunks; c0 += 64 * UNROLL) {
+      uint4 wv[UNROLL], xv[UNROLL][TMAX];
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        const int c = min(c0 + 64 * u, chunks - 1);
+        wv[u] = gload16(&wr[0][c]);
+#pragma unroll
+        for (int t = 0; t < TMAX; ++t) xv[u][t] = gload16(&x[(int64_t)min(t, tokens - 1) * chunks + c]);
+      }
+#pragma unroll
+      for (int u = 0; u < UNROLL; ++u) {
+        if (c0 + 64 * u < chunks)
+#pragma unroll
+          for (int t = 0; t < TMAX; ++t) acc[0][t] = dot8_bf16x(wv[u], xv[u][t], acc[0][t]);
+      }
+    }
+  } else {
 #pragma unroll 2
-  for (int c = lane; c < chunks; c += 64) {
-    uint4 wv[LR_ROWS];
+    for (int c = lane; c < chunks; c += 64) {
+      uint4 wv[ROWS];
 #pragma unroll
-    for (int r = 0; r < LR_ROWS; ++r) wv[r] = gload16_nt(&wr[r][c]);
+      for (int r = 0; r < ROWS; ++r) wv[r] = gload16_nt(&wr[r][c]);
 #pragma unroll
-    for (int t = 0; t < TMAX; ++t) {
-      if (t < tokens) {
-        const uint4 xv = x[(int64_t)t * chunks + c];
+      for (int t = 0; t < TMAX; ++t) {
+        if (t < tokens) {
+          const uint4 xv = x[(int64_t)t * chunks + c];
 #pragma unroll
-        for (int r = 0; r < LR_ROWS; ++r) acc[r][t] = dot8_bf16x(wv[r], xv, acc[r][t]);
+          for (int r = 0; r < ROWS; ++r) acc[r][t] = dot8_bf16x(wv[r], xv, acc[r][t]);
+        }
       }
     }
   }
 #pragma unroll
-  for (int r = 0; r < LR_ROWS; ++r) {
+  for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
     for (int t = 0; t < TMAX; ++t) {
       if (t < tokens) {  // uniform
@@ -300,21 +324,35 @@ WM_EXPORT int wm_linear_bf16(const void* x, const void* w, int32_t tokens, int32
     if (tokens < 0 || outputs < 0 || hidden < 2 || hidden % 2) fail("wm_linear_bf16: bad shape");
     if (tokens == 0 || outputs == 0) return;
     if (!x || !w || !out) fail("wm_linear_bf16: null pointer");
-    // 64+ tokens: the router GEMM on MFMA (norm_router.hip); up to 16 tokens with 16-byte
-    // rows: one pass over each weight row; else one wave per output
-    if (linear_bf16_mfma(x, w, tokens, hidden, outputs, out, as_stream(stream))) return;
-    if (tokens <= 16 && hidden % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0) {
-      const dim3 grid((outputs + 4 * LR_ROWS - 1) / (4 * LR_ROWS));
+    const bool rows16 = hidden % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0;
+    const bool gemm = gemm_bf16_fits(x, w, hidden);
+    // up to 4 tokens: weight rows streamed past the tokens' x (512 rows of 2048: 1 token 2.2 us,
+    // 4 tokens 3.5, the GEMM 4.2 and 4.7; 129,280 rows of 7168: 275 and 304 us, the GEMM 315).
+    // More: the GEMM (8 tokens of the large one 432 us streamed, 312 as a GEMM).
+    if (rows16 && tokens <= (gemm ? 4 : 16)) {
       const int chunks = hidden / 8;
-#define WM_LR(T) hipLaunchKernelGGL(linear_rows_kernel<T>, grid, dim3(256), 0, as_stream(stream), (const uint4*)x, \
-                                    (const uint4*)w, tokens, chunks, outputs, out)
-      if (tokens <= 1) WM_LR(1);
-      else if (tokens <= 2) WM_LR(2);
-      else if (tokens <= 4) WM_LR(4);
-      else if (tokens <= 8) WM_LR(8);
-      else WM_LR(16);
+#define WM_LR(T, R) hipLaunchKernelGGL((linear_rows_kernel<T, R>), dim3((outputs + 4 * R - 1) / (4 * R)), dim3(256), 0, \
+                                       as_stream(stream), (const uint4*)x, (const uint4*)w, tokens, chunks, outputs, out)
+#define WM_LRT(T) do { if (outputs < LR_MIN_OUTPUTS) WM_LR(T, 1); else WM_LR(T, LR_ROWS); } while (0)
+      if (tokens <= 1) WM_LRT(1);
+      else if (tokens <= 2) WM_LRT(2);
+      else if (tokens <= 4) WM_LRT(4);
+      else if (tokens <= 8) WM_LR(8, LR_ROWS);
+      else WM_LR(16, LR_ROWS);
+#undef WM_LRT
 #undef WM_LR
       check_launch("linear_rows");
+      return;
+    }
+    if (gemm) {
+      GemmArgs g{};
+      g.x = (const uint16_t*)x;
+      g.w = (const uint16_t*)w;
+      g.tokens = tokens;
+      g.k = hidden;
+      g.n = outputs;
+      g.out = out;
+      gemm_bf16(GEMM_F32, g, as_stream(stream));
       return;
     }
     hipLaunchKernelGGL(linear_bf16_kernel, dim3((outputs + 3) / 4, tokens), dim3(256), 0, as_stream(stream),

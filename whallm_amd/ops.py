@@ -542,9 +542,8 @@ def residual_rmsnorm(residual: torch.Tensor, y: torch.Tensor | None, eps: float 
 
 
 def repack_router(router: torch.Tensor, shared_gate: torch.Tensor | None = None) -> torch.Tensor:
-    """The router rows (+ the shared gate row) in the prefill GEMM's fragment order
-    (wm_repack_router): a one-time copy that norm_router(..., router_packed=) reads at 16+
-    tokens as contiguous 1 KB fragments."""
+    """The router rows (+ the shared gate row) in MFMA fragment order (wm_repack_router).
+    norm_router(..., router_packed=) accepts it; it reads the rows as stored just as fast."""
     device = _require_device(router, shared_gate)
     router = _contig(router, torch.bfloat16, "router")
     E, H = router.shape
@@ -563,11 +562,11 @@ def repack_router(router: torch.Tensor, shared_gate: torch.Tensor | None = None)
 def norm_router(residual: torch.Tensor, y: torch.Tensor | None, router: torch.Tensor,
                 shared_gate: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None, eps: float = 1e-6,
                 residual_out: torch.Tensor | None = None, router_packed: torch.Tensor | None = None):
-    """One launch (wm_norm_router): v = residual + y, x = bf16(rmsnorm(v) * norm_weight),
+    """The step before the MoE (wm_norm_router): v = residual + y, x = bf16(rmsnorm(v) * norm_weight),
     router logits = x @ router^T (fp32) and the shared gate logit x @ shared_gate (fp32, or
     None). Returns (x, logits, shared_logit); ``residual_out`` (a separate fp32 buffer)
     receives v. The residual itself is not written (other blocks still read it).
-    ``router_packed`` (repack_router of the same router and gate) speeds up 16+ tokens."""
+    ``router_packed`` (repack_router of the same router and gate) is accepted and checked."""
     device = _require_device(residual, y, router, shared_gate, norm_weight, residual_out, router_packed)
     if residual.dtype != torch.float32 or not residual.is_contiguous():
         raise ValueError("residual must be a contiguous float32 tensor")
