@@ -11,7 +11,8 @@
 //   split   : every token row of x (bf16) becomes two E2M3 (fp6) terms, hi and lo, each
 //             with an E8M0 scale per 32 values, stored as the MFMA's B operand reads them
 //             (the GEMMs copy them to LDS unchanged).
-//   gate_up : tile = 128 permuted rows x (TW / 2 gate + the matching up weight rows); per
+//   gate_up : tile = 128 permuted rows (64 or 16 where an expert has few: grouped_stream.h) x
+//             (TW / 2 gate + the matching up weight rows); per
 //             128-wide K step each wave runs its weight tiles x 2 row tiles x 2 halves of
 //             the step x 2 terms MFMAs. SwiGLU is the epilogue, which writes act straight
 //             back as E2M3 terms (the down GEMM's B operand).
@@ -26,6 +27,7 @@
 #include <atomic>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 
 #include "lds_dma.h"
 #include "moe_internal.h"
@@ -53,8 +55,9 @@ struct Lists {
   int has_shared;
 };
 
+template <int ROWS = BM>
 __device__ __forceinline__ int active_row_tiles(const Lists& L) {
-  return L.tile_count[0] + (L.has_shared ? (L.tokens + BM - 1) / BM : 0);
+  return L.tile_count[0] + (L.has_shared ? (L.tokens + ROWS - 1) / ROWS : 0);
 }
 
 __device__ __forceinline__ float pow2_biased(int e) { return __uint_as_float((uint32_t)e << 23); }
@@ -84,19 +87,35 @@ __device__ __forceinline__ const uint8_t* uniform_u8(const uint8_t* p) {
 // it, and no memory fence.
 __device__ __forceinline__ void ring_wait_all() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The tiles of this workgroup in a persistent launch: XCD x takes the contiguous range
-// [x * share, (x + 1) * share) of the (row tile, column tile) list, and its workgroups
-// take every (gridDim / 8)-th tile of it, so the column tiles of a row tile (which read
-// the same rows) and the row tiles of an expert (the same weights) meet in one L2.
+// The tiles of this workgroup in a persistent launch: XCD x takes an eighth of the (row tile,
+// column tile) list in one run, and its workgroups take every (gridDim / 8)-th tile of it, so the
+// column tiles of a row tile (which read the same rows) and the row tiles of an expert (the same
+// weights) meet in one L2. The first `lead` tiles may follow a spacing of their own.
 struct TileRange {
   int first, stride, count;
+  int lead, lead_first, lead_stride;
+  __device__ __forceinline__ int at(int j) const {
+    return j < lead ? lead_first + lead_stride * j : first + stride * (j - lead);
+  }
 };
 __device__ __forceinline__ TileRange tile_range(int active) {
   const int xcd = blockIdx.x % XCDS, local = blockIdx.x / XCDS, per = gridDim.x / XCDS;
-  const int share = (active + XCDS - 1) / XCDS;
-  const int hi = min(xcd * share + share, active);
-  TileRange t{xcd * share + local, per, 0};
+  const int lo = (int)((int64_t)active * xcd / XCDS), hi = (int)((int64_t)active * (xcd + 1) / XCDS);
+  TileRange t{lo + local, per, 0, 0, 0, 0};
   if (t.first < hi) t.count = (hi - t.first + per - 1) / per;
+  return t;
+}
+// The tiles of a second list that the launch goes on to: the workgroups that had one tile less of the
+// first list (`before` tiles) take `extra` more of this one.
+__device__ __forceinline__ TileRange tile_range_after(int active, int before, int extra) {
+  const int xcd = blockIdx.x % XCDS, local = blockIdx.x / XCDS, per = gridDim.x / XCDS;
+  const int had = (int)((int64_t)before * (xcd + 1) / XCDS) - (int)((int64_t)before * xcd / XCDS);
+  const int heavy = had % per, light = heavy ? per - heavy : 0;  // workgroups with one more, with one less
+  const int lo = (int)((int64_t)active * xcd / XCDS), hi = (int)((int64_t)active * (xcd + 1) / XCDS);
+  const int ahead = min(light * extra, hi - lo);  // the tiles that the light ones take first
+  TileRange t{lo + ahead + local, per, 0, 0, lo + local - heavy, light};
+  if (light && local >= heavy && t.lead_first < lo + ahead) t.lead = (lo + ahead - t.lead_first + light - 1) / light;
+  t.count = t.lead + (t.first < hi ? (hi - t.first + per - 1) / per : 0);
   return t;
 }
 
@@ -285,6 +304,22 @@ __device__ __forceinline__ int fp8_term_exponent(float amax) {
   return e - 7 > 5 ? e - 7 : 5;
 }
 
+// The hi and lo terms of 4 values under f = 2^(127 - s).
+__device__ __forceinline__ void fp8_terms4(const float (&v)[4], float f, uint32_t& hi, uint32_t& lo) {
+  float h[4], l[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = v[j] * f;
+  const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[0], h[1], 0, false);
+  const uint32_t w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[2], h[3], (int)w01, true);
+  l[0] = (h[0] - __builtin_amdgcn_cvt_f32_fp8((int)w, 0)) * 16.0f;
+  l[1] = (h[1] - __builtin_amdgcn_cvt_f32_fp8((int)w, 1)) * 16.0f;
+  l[2] = (h[2] - __builtin_amdgcn_cvt_f32_fp8((int)w, 2)) * 16.0f;
+  l[3] = (h[3] - __builtin_amdgcn_cvt_f32_fp8((int)w, 3)) * 16.0f;
+  const uint32_t u01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[0], l[1], 0, false);
+  hi = w;
+  lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[2], l[3], (int)u01, true);
+}
+
 // The hi and lo E4M3 terms of one 32-value block (v in K order) as 8 words each (byte i of
 // the 32 = value i), and the hi scale byte.
 __device__ __forceinline__ void fp8_terms32(const float (&v)[32], uint32_t (&hi)[8], uint32_t (&lo)[8], int& s_hi) {
@@ -295,18 +330,8 @@ __device__ __forceinline__ void fp8_terms32(const float (&v)[32], uint32_t (&hi)
   const float f = pow2_biased(254 - s_hi);  // 2^(127 - s): exact
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    float h[4], l[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) h[j] = v[4 * q + j] * f;
-    const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[0], h[1], 0, false);
-    const uint32_t w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[2], h[3], (int)w01, true);
-    l[0] = (h[0] - __builtin_amdgcn_cvt_f32_fp8((int)w, 0)) * 16.0f;
-    l[1] = (h[1] - __builtin_amdgcn_cvt_f32_fp8((int)w, 1)) * 16.0f;
-    l[2] = (h[2] - __builtin_amdgcn_cvt_f32_fp8((int)w, 2)) * 16.0f;
-    l[3] = (h[3] - __builtin_amdgcn_cvt_f32_fp8((int)w, 3)) * 16.0f;
-    const uint32_t u01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[0], l[1], 0, false);
-    hi[q] = w;
-    lo[q] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[2], l[3], (int)u01, true);
+    const float four[4] = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    fp8_terms4(four, f, hi[q], lo[q]);
   }
 }
 
@@ -425,19 +450,20 @@ __device__ __forceinline__ int32_t scalar_i32(const int32_t* p, int idx) {
 
 // Row range and expert of logical row tile m through scalar loads only (a per-lane vector
 // load would make the compiler wait for every load in flight, the ring's included).
+template <int ROWS = BM>
 __device__ __forceinline__ bool resolve_tile_s(const Lists& L, int m, int& expert, int& begin, int& end) {
   const int routed_tiles = scalar_i32(L.tile_count, 0);
   if (m < routed_tiles) {
     expert = scalar_i32(L.tiles, 2 * m);
     begin = scalar_i32(L.tiles, 2 * m + 1);
-    end = min(begin + BM, scalar_i32(L.offsets, expert + 1));
+    end = min(begin + ROWS, scalar_i32(L.offsets, expert + 1));
     return true;
   }
   const int j = m - routed_tiles;
-  if (!L.has_shared || j * BM >= L.tokens) return false;
+  if (!L.has_shared || j * ROWS >= L.tokens) return false;
   expert = -1;
-  begin = L.pairs + j * BM;
-  end = min(begin + BM, L.pairs + L.tokens);
+  begin = L.pairs + j * ROWS;
+  end = min(begin + ROWS, L.pairs + L.tokens);
   return true;
 }
 
@@ -448,6 +474,7 @@ __device__ __forceinline__ bool resolve_tile_s(const Lists& L, int m, int& exper
 // reads). With 4 or fewer it is row-major: a row tile's column tiles run together (its
 // split rows stay in L2) while the W workgroups of an XCD still cover W / n_tiles row tiles
 // of an expert at a time (measured faster for C3's down GEMM). Scalar loads only.
+template <int ROWS = BM>
 __device__ __forceinline__ void order_tile(const Lists& L, int logical, int n_tiles, int& mt, int& nt) {
   const int m0 = logical / n_tiles;
   if (n_tiles <= 4) {
@@ -461,11 +488,11 @@ __device__ __forceinline__ void order_tile(const Lists& L, int logical, int n_ti
     const int e = scalar_i32(L.tiles, 2 * m0);
     const int begin = scalar_i32(L.tiles, 2 * m0 + 1);
     const int lo = scalar_i32(L.offsets, e), hi = scalar_i32(L.offsets, e + 1);
-    t0 = m0 - (begin - lo) / BM;
-    c = (hi - lo + BM - 1) / BM;
+    t0 = m0 - (begin - lo) / ROWS;
+    c = (hi - lo + ROWS - 1) / ROWS;
   } else {
     t0 = routed;
-    c = (L.tokens + BM - 1) / BM;
+    c = (L.tokens + ROWS - 1) / ROWS;
   }
   const int local = logical - t0 * n_tiles;
   nt = local / c;
@@ -1071,11 +1098,9 @@ __device__ __forceinline__ int table_tiled(const wm_fp8_experts& t) { return t.t
 // 32 (MI / 2) wn + [0, 32 MI / 2) (mi < MI / 2) and the same up rows (mi >= MI / 2).
 // x6 / a6: the split rows' terms (and, E4M3, x6s / a6s their scale dwords).
 template <typename F, int DA, int DB, typename Table>
-__global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) gate_up_mx_kernel(const uint8_t* __restrict__ x6,
-                                                                 const uint8_t* __restrict__ x6s,
-                                                                 const int32_t* __restrict__ row_token, Lists L,
-                                                                 Table routed, Table shared, uint8_t* __restrict__ a6,
-                                                                 uint32_t* __restrict__ a6s) {
+__device__ __forceinline__ void gate_up_mx(uint8_t* lds, const uint8_t* __restrict__ x6, const uint8_t* __restrict__ x6s,
+                                           const int32_t* __restrict__ row_token, const Lists& L, const Table& routed,
+                                           const Table& shared, uint8_t* __restrict__ a6, uint32_t* __restrict__ a6s) {
   constexpr int TG = F::TW / 2, MI = F::MI, HM = MI / 2;
   constexpr int XS = F::Terms::XS;
   const int H = routed.hidden, I = routed.inter;
@@ -1090,7 +1115,7 @@ __global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) gate_up_mx_kernel
 
   auto setup = [&](int j, Tile& t) {
     int mt = 0;
-    order_tile(L, tr.first + tr.stride * j, n_tiles, mt, t.nt);
+    order_tile(L, tr.at(j), n_tiles, mt, t.nt);
     int expert = 0, begin = 0, end = 0;
     if (!resolve_tile_s(L, mt, expert, begin, end)) return false;
     t.begin = begin;
@@ -1212,16 +1237,15 @@ __global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) gate_up_mx_kernel
     zero_acc<F>(acc);
   };
 
-  __shared__ __attribute__((aligned(16))) uint8_t lds[RingMx<F, DA, DB>::BYTES];
   persistent_tiles<F, DA, DB, Tile>(tr, H / 128, lds, setup, mfma, epilogue);
 }
 
 // down: out[row, n] = act[row] . W2[n], bf16, permuted rows (the combine applies the routing
 // weights); tile = 128 rows x TW output columns, wave wn owns columns 32 MI wn + [0, 32 MI).
 template <typename F, int DA, int DB, typename Table>
-__global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) down_mx_kernel(const uint8_t* __restrict__ a6,
-                                                              const uint8_t* __restrict__ a6s, Lists L, Table routed,
-                                                              Table shared, uint16_t* __restrict__ out) {
+__device__ __forceinline__ void down_mx(uint8_t* lds, const uint8_t* __restrict__ a6, const uint8_t* __restrict__ a6s,
+                                        const Lists& L, const Table& routed, const Table& shared,
+                                        uint16_t* __restrict__ out) {
   constexpr int MI = F::MI;
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = (H + F::TW - 1) / F::TW;
@@ -1234,7 +1258,7 @@ __global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) down_mx_kernel(co
 
   auto setup = [&](int j, Tile& t) {
     int mt = 0;
-    order_tile(L, tr.first + tr.stride * j, n_tiles, mt, t.nt);
+    order_tile(L, tr.at(j), n_tiles, mt, t.nt);
     int expert = 0, begin = 0, end = 0;
     if (!resolve_tile_s(L, mt, expert, begin, end)) return false;
     t.begin = begin;
@@ -1299,9 +1323,32 @@ __global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4) down_mx_kernel(co
     zero_acc<F>(acc);
   };
 
-  __shared__ __attribute__((aligned(16))) uint8_t lds[RingMx<F, DA, DB>::BYTES];
   persistent_tiles<F, DA, DB, Tile>(tr, I / 128, lds, setup, mfma, epilogue);
 }
+
+// 128-row tiles alone.
+template <typename F, typename Table>
+__global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4)
+    gate_up_mx_kernel(const uint8_t* __restrict__ x6, const uint8_t* __restrict__ x6s, const int32_t* __restrict__ row_token,
+                      Lists L, Table routed, Table shared, uint8_t* __restrict__ a6, uint32_t* __restrict__ a6s) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[RingMx<F, F::DA, F::DB>::BYTES];
+  gate_up_mx<F, F::DA, F::DB>(lds, x6, x6s, row_token, L, routed, shared, a6, a6s);
+}
+template <typename F, typename Table>
+__global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4)
+    down_mx_kernel(const uint8_t* __restrict__ a6, const uint8_t* __restrict__ a6s, Lists L, Table routed, Table shared,
+                   uint16_t* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[RingMx<F, F::DA, F::DB>::BYTES];
+  down_mx<F, F::DA, F::DB>(lds, a6, a6s, L, routed, shared, out);
+}
+
+}  // namespace mf
+}  // namespace wm
+
+#include "grouped_stream.h"
+
+namespace wm {
+namespace mf {
 
 // Token of every permuted row: order[p] / K for routed rows, p - P for the shared rows.
 __global__ void __launch_bounds__(256) row_tokens_kernel(const int32_t* __restrict__ order, int pairs, int k,
@@ -1463,6 +1510,7 @@ static int compute_units() {
 
 struct Layout {
   size_t permute_ws, order, inverse, offsets, tiles, tile_count, gate, row_token, x6, x6s, a6, a6s, rows, total;
+  int64_t max_tiles;
 };
 
 // Split rows take the larger of the two term formats' bytes per 128-wide K step (E4M3: 256
@@ -1471,15 +1519,16 @@ struct Layout {
 static Layout layout(int tokens, int k, int experts, int hidden, int inter, bool has_shared) {
   const int64_t pairs = (int64_t)tokens * k;
   const int64_t rows = pairs + (has_shared ? tokens : 0);
-  const int64_t max_tiles = (pairs + BM - 1) / BM + experts;
+  const int64_t max_tiles = (pairs + 15) / 16 + experts;  // of the smallest row tile; the cold list follows
   Layout p{};
   size_t at = 0;
   p.permute_ws = at; at += align256(wm_permute_workspace_size(pairs, experts));
   p.order = at;      at += align256(sizeof(int32_t) * (size_t)(pairs > 0 ? pairs : 1));
   p.inverse = at;    at += align256(sizeof(int32_t) * (size_t)(pairs > 0 ? pairs : 1));
   p.offsets = at;    at += align256(sizeof(int32_t) * (size_t)(experts + 1));
-  p.tiles = at;      at += align256(sizeof(int32_t) * 2 * (size_t)max_tiles);
-  p.tile_count = at; at += align256(sizeof(int32_t));
+  p.tiles = at;      at += align256(sizeof(int32_t) * 2 * (size_t)(max_tiles + experts));
+  p.max_tiles = max_tiles;
+  p.tile_count = at; at += align256(2 * sizeof(int32_t));
   p.gate = at;       at += align256(sizeof(float) * (size_t)(tokens > 0 ? tokens : 1));
   p.row_token = at;  at += align256(sizeof(int32_t) * (size_t)(rows > 0 ? rows : 1));
   p.x6 = at;         at += align256((size_t)tokens * (hidden / 128) * XSTEP8);
@@ -1489,6 +1538,31 @@ static Layout layout(int tokens, int k, int experts, int hidden, int inter, bool
   p.rows = at;       at += align256(sizeof(uint16_t) * (size_t)rows * hidden);
   p.total = at;
   return p;
+}
+
+// How a call's row tiles are made. ROWS_MIXED is the general one: it was the fastest or within 3%
+// of it at every size measured (us of a whole call, tiled weights, 128-row tiles alone / mixed):
+//   MXFP4 2048/512, 512 experts top 10, even routing: 64 tokens 273/202, 1200 402/294, 2048 416/376,
+//     4096 466/479, 16384 1278/1292; skewed (Zipf 1.1): 97/80, 200/198, 272/249, 441/405, 1230/1227
+//   MXFP4 5120/2304, 384 experts top 6: 64 1543/934, 2048 2684/2038, 4096 2922/2747; skewed 2231/2068
+//   FP8 7168/2048, 256 experts top 8: 64 2490/1507, 2048 3190/2882, 4096 4722/4750; skewed 4642/4279
+// Where it loses its 3% (64 to 128 rows for every expert) the host, which knows the mean and not the
+// counts, cannot tell it from the skewed call that gains 9%.
+// ROWS_16, MXFP4 at up to 8 rows an expert: mixed / 16 rows, 2048/512: 1.2 rows 202/145, 5.9 268/202
+// (skewed 80/65, 121/120; at 11.7 skewed 152/181); 5120/2304: 1.0 934/846. Tokens are bounded since
+// the shared expert's rows take tiles of 16 too.
+// The streaming kernels need two weight units a tile (FP8 256, MXFP4 384 wide); E2M3 terms have only
+// 128-row tiles.
+enum RowTiles {
+  ROWS_128,    // 128 rows of every expert
+  ROWS_MIXED,  // 128 rows of the experts with more than 64, 64 of the others
+  ROWS_16,     // 16 rows of every expert
+};
+static RowTiles row_tiles(bool e4m3, bool fp8, int tokens, int k, int experts, int hidden, int inter) {
+  const int least = fp8 ? 256 : 384;
+  if (!e4m3 || hidden < least || inter < least) return ROWS_128;
+  if (!fp8 && tokens <= 512 && (int64_t)tokens * k <= (int64_t)8 * experts) return ROWS_16;
+  return ROWS_MIXED;
 }
 
 template <typename F, typename Table>
@@ -1531,10 +1605,19 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
   L.k = k;
   L.has_shared = has_shared ? 1 : 0;
   int32_t* inverse = (int32_t*)(base + p.inverse);
-  if (wm_permute(indices, pairs, routed.experts, BM, (int32_t*)L.order, inverse, (int32_t*)L.offsets,
-                 (int32_t*)L.tiles, (int32_t*)L.tile_count, base + p.permute_ws,
-                 wm_permute_workspace_size(pairs, routed.experts), s) != 0)
-    fail(std::string("prefill permute: ") + wm_last_error());
+  const RowTiles how = row_tiles(F::Terms::E4, F::FP8, tokens, k, routed.experts, H, I);
+  const int bm = how == ROWS_16 ? 16 : BM;
+  // the cold list of ROWS_MIXED: at most one 64-row tile an expert, and the shared expert's when it fits
+  Lists cold = L;
+  cold.tiles = L.tiles + 2 * p.max_tiles;
+  cold.tile_count = L.tile_count + 1;
+  constexpr int COLD_ROWS = 64;
+  if (how == ROWS_MIXED) {
+    L.has_shared = has_shared && tokens > COLD_ROWS;
+    cold.has_shared = has_shared && tokens <= COLD_ROWS;
+  }
+  permute_tiles(indices, pairs, routed.experts, bm, how == ROWS_MIXED ? COLD_ROWS : 0, (int32_t*)L.order, inverse,
+                (int32_t*)L.offsets, (int32_t*)L.tiles, (int32_t*)cold.tiles, (int32_t*)L.tile_count, base + p.permute_ws, s);
   // the split kernel computes the shared gate when a row's blocks fit one wave in a
   // power-of-two group; otherwise a kernel of its own does
   const bool fused_gate = has_shared && shared_gate && (H / 32) <= 64 && ((H / 32) & (H / 32 - 1)) == 0;
@@ -1560,13 +1643,14 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
                        x6, fused_gate ? shared_gate : nullptr, (float*)L.shared_gate);
   check_launch("split_rows");
   const Table sh = shared ? *shared : routed;
-  const int64_t max_row_tiles = (pairs + BM - 1) / BM + routed.experts + (has_shared ? (tokens + BM - 1) / BM : 0);
-  // Persistent launches: one workgroup per CU (the LDS stages allow one), a multiple of the
-  // 8 XCDs, and no more than the work tiles can use.
+  const int64_t max_row_tiles = (pairs + bm - 1) / bm + routed.experts + (has_shared ? (tokens + bm - 1) / bm : 0);
+  // Persistent launches: as many workgroups per CU as the LDS rings allow, a multiple of the 8
+  // XCDs, and no more than the work tiles can use.
+  const int per_cu = how == ROWS_16 ? 2 : 1;
   const int cus = compute_units();
   auto grid_for = [&](int n_tiles) {
     const int64_t work = max_row_tiles * n_tiles;
-    const int64_t per_xcd = std::min<int64_t>((work + XCDS - 1) / XCDS, std::max(cus / XCDS, 1));
+    const int64_t per_xcd = std::min<int64_t>((work + XCDS - 1) / XCDS, std::max(cus / XCDS, 1) * per_cu);
     return dim3((unsigned)(per_xcd * XCDS));
   };
   uint8_t* a6 = base + p.a6;
@@ -1574,13 +1658,38 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
   uint16_t* out_rows = (uint16_t*)(base + p.rows);
   TimingEvents* te = g_timing.load() ? timing_events() : nullptr;
   if (te) check_hip(hipEventRecord(te->ev[0], s), "hipEventRecord");
-  hipLaunchKernelGGL((gate_up_mx_kernel<F, F::DA, F::DB, Table>), grid_for((I + F::TW / 2 - 1) / (F::TW / 2)),
-                     dim3(64 * F::WAVES), 0, s, x6, x6s, row_token, L, routed, sh, a6, a6s);
-  check_launch("gate_up");
-  if (te) check_hip(hipEventRecord(te->ev[1], s), "hipEventRecord");
   // unweighted rows: the combine applies the routing weights and the shared gate
-  hipLaunchKernelGGL((down_mx_kernel<F, F::DA, F::DB, Table>), grid_for((H + F::TW - 1) / F::TW), dim3(64 * F::WAVES), 0,
-                     s, a6, (const uint8_t*)a6s, L, routed, sh, out_rows);
+  auto mid = [&] {
+    check_launch("gate_up");
+    if (te) check_hip(hipEventRecord(te->ev[1], s), "hipEventRecord");
+  };
+  if constexpr (F::Terms::E4 && !F::FP8) {
+    if (how == ROWS_16) {
+      using S = StreamF<false, true, 16, 4>;
+      hipLaunchKernelGGL((stream_gate_up_kernel<S, Table>), grid_for(I / (S::TW / 2)), dim3(64 * S::WAVES), 0, s, x6, x6s,
+                         row_token, L, routed, sh, a6, (uint8_t*)a6s);
+      mid();
+      hipLaunchKernelGGL((stream_down_kernel<S, Table>), grid_for((H + S::TW - 1) / S::TW), dim3(64 * S::WAVES), 0, s, a6,
+                         (const uint8_t*)a6s, L, routed, sh, out_rows);
+    }
+  }
+  if constexpr (F::Terms::E4) {
+    if (how == ROWS_MIXED) {
+      const dim3 all((unsigned)(std::max(cus / XCDS, 1) * XCDS));
+      hipLaunchKernelGGL((mixed_gate_up_kernel<F, Table>), all, dim3(512), 0, s, x6, x6s, row_token, L, cold, routed, sh, a6,
+                         a6s);
+      mid();
+      hipLaunchKernelGGL((mixed_down_kernel<F, Table>), all, dim3(512), 0, s, a6, (const uint8_t*)a6s, L, cold, routed, sh,
+                         out_rows);
+    }
+  }
+  if (how == ROWS_128) {
+    hipLaunchKernelGGL((gate_up_mx_kernel<F, Table>), grid_for((I + F::TW / 2 - 1) / (F::TW / 2)), dim3(64 * F::WAVES), 0, s,
+                       x6, x6s, row_token, L, routed, sh, a6, a6s);
+    mid();
+    hipLaunchKernelGGL((down_mx_kernel<F, Table>), grid_for((H + F::TW - 1) / F::TW), dim3(64 * F::WAVES), 0, s, a6,
+                       (const uint8_t*)a6s, L, routed, sh, out_rows);
+  }
   check_launch("down");
   if (te) check_hip(hipEventRecord(te->ev[2], s), "hipEventRecord");
   const int32_t* shared_slots = has_shared ? shared->slots : nullptr;

@@ -1,0 +1,511 @@
+// The grouped GEMMs' tiles for few rows an expert: a part of grouped_mfma.hip (which includes it
+// after its 128-row tiles and its tile, term and scalar-load helpers).
+//
+// With up to a few dozen rows an expert the weights, each read once, bound the call. What 128-row
+// tiles spend there instead: MFMAs on empty rows (128 for 1 to 64), two load slots that wait
+// a memory round trip each K step, and, in the row layout, half a 128-byte line of every
+// MXFP4 row a step. Here:
+//
+//   tile    : BM rows of one expert x TW = 32 WAVES weight rows; wave w owns the 32-row weight tile
+//             w: for gate_up 16 gate rows and the same 16 up rows, so that a lane holds both
+//             results of a column.
+//   weights : a unit is 128 bytes of every row (two 128-wide K steps of MXFP4, one of FP8), eight
+//             whole lines of 8 rows a load, in either layout, with the non-temporal hint (a
+//             plain read of HBM: 7.0 against 5.9 TB/s).
+//   rows    : the split rows by K step, as in the 128-row tiles.
+//
+// Both go to LDS rings of three slots by direct loads, two units (steps) ahead, across tiles.
+// Two shapes: 64 rows x 256 weight rows (8 waves, 154 KB), one row tile an expert; and, for MXFP4, 16
+// rows x 128 (4 waves, 77 KB), two workgroups on a CU, one's epilogue and tile set-up under the
+// other's loads. row_tiles() says which call takes which, with times. At 2 rows an expert of
+// 7168/2048 FP8 weights (11.3 GB): 1486 us a call against 2791 with 128-row tiles, 7.6 TB/s.
+#pragma once
+
+namespace wm {
+namespace mf {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+template <bool FP8_, bool A_SCALED_, int BM_, int WAVES_>
+struct StreamF {
+  static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
+  static constexpr int BM = BM_, WAVES = WAVES_, NI = 2, TW = 32 * WAVES_;  // NI: 32-row row tiles of 64 rows
+  static constexpr int SUB = FP8_ ? 1 : 2;                 // K steps of a weight unit
+  static constexpr int BSUB = BM_ == 16 ? SUB : 1;         // K steps of a split-row slot
+  static constexpr int GRAN = SUB / BSUB;                  // split-row slots of a unit
+  static constexpr int A_FMT = FP8_ ? FMT_FP8 : FMT_FP4;
+  static constexpr int A_SLOT = TW * 128 + (A_SCALED_ ? TW * 4 * SUB : 0);
+  static constexpr int B_TERMS = BM_ * XSTEP8 * BSUB, B_SLOT = B_TERMS + BM_ * 4 * BSUB;
+  static constexpr int RINGS = 3 * (A_SLOT + B_SLOT), BYTES = RINGS + WAVES_ * BM_ * 4;  // and block maxima
+  static constexpr int NQA = 4, NQB = BM_ / 4 / WAVES_;    // 1 KB loads of a wave: a unit's, a K step's rows
+  // about how many of its tiles take as long as one 128-row tile (twice the weight rows for MXFP4, and
+  // bound by its MFMAs)
+  static constexpr int HOT_COST = FP8_ ? 1 : 3;
+  // loads of a wave: a unit's, and at least a split-row slot's (see issue_rows)
+  static constexpr int UNIT_LOADS = NQA + (A_SCALED_ ? 1 : 0), ROW_LOADS = BM_ == 16 ? BSUB + 1 : 2;
+  static_assert(BM_ == 16 ? NQB == 1 && !FP8_ : BM_ == 64 && NQB == 2, "the loader's split-row loads");
+};
+
+// Loads of one tile. Weight load i of wave w fills rows 8 (w + WAVES i) .. + 7 of the tile: lane l
+// row l / 8, LDS position l % 8 holding piece (l % 8) ^ (l / 8) of the row's 128 bytes (8 rows at
+// one piece then lie on distinct banks). The second half of a unit's pieces (the odd K step of MXFP4)
+// is `half` bytes on; a last unit of one step reads its first half twice.
+template <typename F>
+struct StreamLoads {
+  const uint8_t *w, *s, *b, *bs;
+  uint32_t woff[F::NQA], whalf, wunit, soff, shalf, sunit;
+  uint32_t boff[F::NQB], bsoff;
+
+  // rows: the region's rows, k its K; row_of(j): the region row of tile row j (8-row groups stay
+  // together)
+  template <typename RowOf>
+  __device__ __forceinline__ void weights(const uint8_t* region, const uint8_t* scales, int rows, int k, int tiled,
+                                          int wave, int lane, RowOf row_of) {
+    w = uniform_u8(region);
+    s = uniform_u8(scales);
+    const int p = (lane % 8) ^ (lane / 8);
+#pragma unroll
+    for (int i = 0; i < F::NQA; ++i) {
+      const int row = row_of(8 * (wave + F::WAVES * i) + lane / 8);
+      if (tiled)
+        woff[i] = (uint32_t)(row / 16 * (F::FP8 ? 2048 : 1024) + (F::FP8 ? p : p % 4) * 256 + row % 16 * 16);
+      else
+        woff[i] = (uint32_t)(row * (F::FP8 ? k : k / 2) + (F::FP8 ? p : p % 4) * 16);
+    }
+    const uint32_t step = tiled ? (uint32_t)rows * (F::FP8 ? 128 : 64) : (F::FP8 ? 128 : 64);
+    wunit = F::SUB * step;
+    whalf = F::FP8 || p < 4 ? 0 : step;
+    soff = shalf = sunit = 0;
+    if constexpr (F::A_SCALED && F::FP8) {  // E8M0 32 x 32 blocks: lanes 0..31, a dword a row and step
+      soff = (uint32_t)(row_of(32 * wave + lane % 32) / 32 * (k / 32));
+      sunit = 4;
+    } else if constexpr (F::A_SCALED) {  // lane l: row 32 w + l / 2, step l % 2
+      const int row = row_of(32 * wave + lane / 2);
+      const uint32_t sstep = tiled ? (uint32_t)rows * 4 : 4;
+      soff = (uint32_t)(tiled ? row * 4 : row * (k / 32));
+      sunit = 2 * sstep;
+      shalf = lane % 2 ? sstep : 0;
+    }
+  }
+  // row_index(r): the split row of tile row r (wave-uniform r). Load i of wave w fills rows
+  // 4 (w + WAVES i) .. + 3, and the scale load their dwords.
+  template <typename RowIndex>
+  __device__ __forceinline__ void rows(const uint8_t* terms, const uint8_t* scales, int k, int wave, int lane,
+                                       RowIndex row_index) {
+    b = uniform_u8(terms);
+    bs = uniform_u8(scales);
+    bsoff = 0;
+#pragma unroll
+    for (int i = 0; i < F::NQB; ++i) {
+      const int q0 = 4 * (wave + F::WAVES * i);
+      int idx[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) idx[d] = row_index(q0 + d);
+      const int d = lane / 16, e = lane % 4;
+      const int mine = d == 0 ? idx[0] : d == 1 ? idx[1] : d == 2 ? idx[2] : idx[3];
+      boff[i] = (uint32_t)mine * (uint32_t)(k / 128 * XSTEP8) + 16u * (uint32_t)((lane % 16) ^ ((q0 + d) & 15));
+      const int srow = e == 0 ? idx[0] : e == 1 ? idx[1] : e == 2 ? idx[2] : idx[3];
+      if (lane / 4 == i || F::NQB == 1) bsoff = (uint32_t)srow * (uint32_t)(k / 128 * 4);
+    }
+  }
+  // Weight unit u; whole: both its steps exist. UNIT_LOADS instructions.
+  __device__ __forceinline__ void issue_unit(uint8_t* slot, int u, bool whole, int wave, int lane) const {
+    const uint32_t at = (uint32_t)u * wunit + (whole ? whalf : 0);
+#pragma unroll
+    for (int i = 0; i < F::NQA; ++i) dma16<true>(w, woff[i] + at, lds_addr(slot + (wave + F::WAVES * i) * 1024));
+    if constexpr (F::A_SCALED) {
+      if (!F::FP8 || lane < 32)
+        dma4(s, soff + (uint32_t)u * sunit + (whole ? shalf : 0),
+             lds_addr(slot + F::TW * 128 + wave * (F::FP8 ? 128 : 256)));
+    }
+  }
+  // The split rows' K steps BSUB k .. of a tile of `n` rows into a slot: ROW_LOADS instructions or one
+  // more (the second load's rows only where the tile has them; what it leaves in LDS feeds unused
+  // columns). A step past the last reads the last again.
+  __device__ __forceinline__ void issue_rows(uint8_t* slot, int k, int steps, int n, int wave, int lane) const {
+    const int ks = min(F::BSUB * k, steps - 1);
+    if constexpr (F::BM == 16) {
+      const bool two = ks + 1 < steps;
+#pragma unroll
+      for (int h = 0; h < F::BSUB; ++h)
+        dma16(b, boff[0] + (uint32_t)(h && two ? ks + 1 : ks) * XSTEP8, lds_addr(slot + h * 16 * XSTEP8 + wave * 1024));
+      // lanes 0..3 the first step's scale dwords of rows 4 w .. + 3, lanes 4..7 the second's
+      if (lane < 4 * F::BSUB)
+        dma4(bs, bsoff + (uint32_t)(lane >= 4 && two ? ks + 1 : ks) * 4, lds_addr(slot + F::B_TERMS + 16 * F::BSUB * wave));
+    } else {
+#pragma unroll
+      for (int i = 0; i < F::NQB; ++i)
+        if (4 * F::WAVES * i < n)
+          dma16(b, boff[i] + (uint32_t)ks * XSTEP8, lds_addr(slot + (wave + F::WAVES * i) * 1024));
+      if (lane < 4 * F::NQB) dma4(bs, bsoff + (uint32_t)ks * 4, lds_addr(slot + F::B_TERMS + 16 * F::NQB * wave));
+    }
+  }
+};
+
+template <typename F>
+struct StreamTile {
+  StreamLoads<F> ld;
+  int expert, begin, end, nt;
+  float limit;
+  const_f32_ptr s0, s1;  // FP8 with fp32 blocks: the block scales of the wave's registers 0..7 and 8..15
+};
+
+// Tile `logical` of the list. With 64 rows every expert has one row tile, so the list is row tile by
+// row tile; otherwise an expert's row tiles that read the same weights run together (order_tile).
+template <typename F>
+__device__ __forceinline__ void stream_locate(const Lists& L, int logical, int n_tiles, StreamTile<F>& t) {
+  int mt = logical / n_tiles;
+  t.nt = logical - mt * n_tiles;
+  if constexpr (F::BM == 16) order_tile<F::BM>(L, logical, n_tiles, mt, t.nt);
+  resolve_tile_s<F::BM>(L, mt, t.expert, t.begin, t.end);
+}
+
+// A wave's results: 32-row weight tile x two 32-row row tiles (v_mfma_scale_f32_32x32x64), or with 16 rows
+// its two 16-row weight tiles (gate_up: the gate and the up rows) x 16 rows (16x16x128).
+template <typename F>
+struct StreamAcc {
+  v16f v[F::NI];
+  v4f q[2];
+  __device__ __forceinline__ void clear() {
+    if constexpr (F::BM == 16) {
+      q[0] = q[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    } else {
+#pragma unroll
+      for (int ni = 0; ni < F::NI; ++ni)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[ni][i] = 0.0f;
+    }
+  }
+};
+
+// acc += K step `sub` of an MXFP4 weight unit and of a split-row slot of 16 rows. Lane (c, q) holds row
+// c's E2M1 K [32 q, +32), or E4M3 K [16 q, +16) and [64 + 16 q, +16); scale lane (c, q) covers K block q.
+template <typename F>
+__device__ __forceinline__ void stream_step16(const uint8_t* wa, const uint8_t* rb, int sub, int wave, int lane,
+                                              v4f (&acc)[2]) {
+  const int c = lane % 16, q = lane / 16;
+  uint4 p[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) p[e] = *reinterpret_cast<const uint4*>(rb + sub * 16 * XSTEP8 + e4_piece(c, 4 * e + q));
+  const uint32_t sw =
+      *reinterpret_cast<const uint32_t*>(rb + F::B_TERMS + 16 * F::BSUB * (c / 4) + 16 * sub + 4 * (c % 4)) >> (8 * q);
+  const v8i hi = {(int)p[0].x, (int)p[0].y, (int)p[0].z, (int)p[0].w, (int)p[1].x, (int)p[1].y, (int)p[1].z, (int)p[1].w};
+  const v8i lo = {(int)p[2].x, (int)p[2].y, (int)p[2].z, (int)p[2].w, (int)p[3].x, (int)p[3].y, (int)p[3].z, (int)p[3].w};
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int row = 32 * wave + 16 * t + c;
+    const uint4 u = *reinterpret_cast<const uint4*>(wa + row * 128 + 16 * ((4 * sub + q) ^ (row % 8)));
+    const v8i a = {(int)u.x, (int)u.y, (int)u.z, (int)u.w, 0, 0, 0, 0};
+    const int sa = (int)(*reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + row * 8 + 4 * sub) >> (8 * q));
+    // lo scales: hi - 4 (every hi scale byte is >= 5, so the low byte takes no borrow)
+    acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, hi, acc[t], F::A_FMT, FMT_FP8, 0, sa, 0, (int)sw);
+    acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, lo, acc[t], F::A_FMT, FMT_FP8, 0, sa, 0, (int)(sw - 4));
+  }
+}
+
+// acc += K step `sub` of a weight unit x a step of split rows.
+template <typename F>
+__device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb, int sub, int rows, int wave, int lane,
+                                            float f0, float f1, v16f (&acc)[F::NI]) {
+  const int r = lane % 32, g = lane / 32;
+  const uint8_t* arow = wa + (32 * wave + r) * 128;
+  uint32_t sa = 127;
+  if constexpr (F::A_SCALED)
+    sa = *reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + (32 * wave + r) * 4 * F::SUB + 4 * sub);
+  v8i a[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    auto piece = [&](int p) { return *reinterpret_cast<const uint4*>(arow + 16 * (p ^ (r % 8))); };
+    if constexpr (F::FP8) {
+      const uint4 u = piece(4 * h + g), v = piece(4 * h + 2 + g);
+      a[h] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
+    } else {
+      const uint4 u = piece(4 * sub + 2 * h + g);
+      a[h] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, 0, 0, 0, 0};
+    }
+  }
+#pragma unroll
+  for (int ni = 0; ni < F::NI; ++ni) {
+    if (32 * ni >= rows) break;  // no rows in this row tile (uniform)
+    const int row = 32 * ni + r;
+    // where the loader put the row's scale dword
+    const uint32_t sw = *reinterpret_cast<const uint32_t*>(
+        rb + F::B_TERMS + 4 * (8 * (row / 4 % F::WAVES) + 4 * (row / (4 * F::WAVES)) + row % 4));
+    v16f blk;
+    if constexpr (F::BLOCK_F32) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) blk[i] = 0.0f;
+    }
+    v16f& sum = F::BLOCK_F32 ? blk : acc[ni];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int sh = 8 * g + 16 * h;
+      v8i t[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint4 u = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + g));
+        const uint4 v = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + 2 + g));
+        t[e] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
+      }
+      const int ws = F::A_SCALED ? (int)(sa >> sh) : 127;
+      sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[h], t[0], sum, F::A_FMT, FMT_FP8, 0, ws, 0, (int)(sw >> sh));
+      sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[h], t[1], sum, F::A_FMT, FMT_FP8, 0, ws, 0,
+                                                            (int)((sw - 0x04040404u) >> sh));
+    }
+    if constexpr (F::BLOCK_F32) {  // the fp32 block scale cannot ride on the MFMA's E8M0 scales
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[ni][i] = fmaf(i < 8 ? f0 : f1, blk[i], acc[ni][i]);
+    }
+  }
+}
+
+// The tiles of this workgroup as one sequence of split-row slots, GRAN to a weight unit (a tile's
+// last unit counts whole; its missing K step is skipped). At the top of slot step g: wait until its
+// rows and its unit have landed, a barrier (which also frees the slots of step g - 1), then the
+// loads of the rows of step g + 2 and, on a unit's first step, of the unit two on, the next tile's
+// where this one ends. Issue order is ..., rows g, unit g / GRAN + 1 (first steps), rows g + 1, so
+// UNIT_LOADS + ROW_LOADS may stay in flight while those were issued. The epilogue's stores count
+// too: they may complete out of order with loads, but loads do not among themselves, so at most that
+// many of the youngest loads are outstanding. At least two units a tile.
+// locate(j, tile) finds a tile (at the start of the one before it, so that its scalar loads'
+// round trips are not where the loads of its first unit wait), setup(tile) its addresses.
+template <typename F, typename Locate, typename Setup, typename Epilogue>
+__device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uint8_t* lds, int wave, int lane, Locate locate,
+                                             Setup setup, Epilogue epilogue) {
+  if (tr.count == 0) return;
+  const int units = (steps + F::SUB - 1) / F::SUB, n = units * F::GRAN;
+  auto wslot = [&](int u) { return lds + u % 3 * F::A_SLOT; };
+  auto rslot = [&](int g) { return lds + 3 * F::A_SLOT + g % 3 * F::B_SLOT; };
+  auto unit = [&](const StreamTile<F>& t, int at, int u) {
+    t.ld.issue_unit(wslot(at), u, F::SUB * (u + 1) <= steps, wave, lane);
+  };
+  auto rows = [&](const StreamTile<F>& t, int at, int k) {
+    t.ld.issue_rows(rslot(at), k, steps, t.end - t.begin, wave, lane);
+  };
+  StreamAcc<F> acc;
+  StreamTile<F> cur, nxt;
+  locate(0, cur);
+  setup(cur);
+  rows(cur, 0, 0);
+  unit(cur, 0, 0);
+  rows(cur, 1, 1);
+  unit(cur, 1, 1);
+  acc.clear();
+  int g = 0, gu = 0;  // slot steps and units before this one
+  for (int j = 0; j < tr.count; ++j) {
+    const bool more = j + 1 < tr.count;
+    for (int k = 0; k < n; ++k, ++g) {
+      const int sub = F::GRAN == 2 ? k & 1 : 0, u = F::GRAN == 2 ? k >> 1 : k;
+      // units issued after this step's rows: the next (a unit's first step) or the one after it
+      const bool kept = more || u + 1 + sub < units;
+      if (kept)
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(F::UNIT_LOADS + F::ROW_LOADS) : "memory");
+      else
+        ring_wait_all();
+      if (k == 0 && more) locate(j + 1, nxt);
+      if (sub == 0 && more && u + 2 == units) setup(nxt);
+      if (k + 2 < n) rows(cur, g + 2, k + 2);
+      else if (more) rows(nxt, g + 2, k + 2 - n);
+      if (sub == 0) {
+        if (u + 2 < units) unit(cur, gu + 2, u + 2);
+        else if (more) unit(nxt, gu + 2, u + 2 - units);
+      }
+#pragma unroll
+      for (int h = 0; h < F::BSUB; ++h) {
+        const int ks = F::BSUB * k + h;
+        if (ks >= steps) break;  // uniform
+        if constexpr (F::BM == 16) {
+          stream_step16<F>(wslot(gu), rslot(g), h, wave, lane, acc.q);
+        } else {
+          float f0 = 1.0f, f1 = 1.0f;
+          if constexpr (F::BLOCK_F32) f0 = cur.s0[ks], f1 = cur.s1[ks];
+          stream_step<F>(wslot(gu), rslot(g), sub, cur.end - cur.begin, wave, lane, f0, f1, acc.v);
+        }
+      }
+      if (sub == F::GRAN - 1) ++gu;
+    }
+    epilogue(cur, acc);
+    acc.clear();
+    cur = nxt;
+  }
+}
+
+// act rows of TW / 2 intermediate columns; wave w owns 16 of them: result lane (r, g) register i < 8
+// is the gate and i + 8 the up product of column 8 (i / 4) + 4 g + i % 4 for row r of a row
+// tile. Waves 2 p and 2 p + 1 share a 32-value block of the act row.
+template <typename F, typename Table>
+__device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
+                                               const int32_t* __restrict__ row_token, const Lists& L, const Table& routed,
+                                               const Table& shared, int before, uint8_t* __restrict__ a8,
+                                               uint8_t* __restrict__ a8s) {
+  float(*block_max)[F::BM] = reinterpret_cast<float(*)[F::BM]>(lds + F::RINGS);
+  constexpr int TG = F::TW / 2;
+  const int H = routed.hidden, I = routed.inter;
+  const int n_tiles = I / TG;  // I is a multiple of 128
+  const TileRange tr = tile_range_after(active_row_tiles<F::BM>(L) * n_tiles, before, F::HOT_COST);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  auto locate = [&](int j, StreamTile<F>& t) { stream_locate<F>(L, tr.at(j), n_tiles, t); };
+  auto setup = [&](StreamTile<F>& t) {
+    const TileWeights tw = tile_weights_s(routed, shared, t.expert);
+    t.limit = tw.limit;
+    const int gate0 = (tw.up_first ? I : 0) + t.nt * TG, up0 = (tw.up_first ? 0 : I) + t.nt * TG;
+    t.ld.weights(tw.w13, tw.w13s, 2 * I, H, table_tiled(routed), wave, lane,
+                 [=](int j) { return (j % 32 < 16 ? gate0 : up0) + j / 32 * 16 + j % 16; });
+    if constexpr (F::BLOCK_F32) {
+      t.s0 = uniform_ptr(reinterpret_cast<const float*>(tw.w13s) + (int64_t)(gate0 / 128) * (H / 128));
+      t.s1 = uniform_ptr(reinterpret_cast<const float*>(tw.w13s) + (int64_t)(up0 / 128) * (H / 128));
+    }
+    const int begin = t.begin, end = t.end;
+    t.ld.rows(x8, x8s, H, wave, lane, [&](int r) { return scalar_i32(row_token, begin + r < end ? begin + r : begin); });
+  };
+  auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
+    // Lane (r, g) holds row r of row tile ni, values [q][i] of the wave's columns 4 g + 8 q + i.
+    constexpr int ROWS = F::BM == 16 ? 16 : 32, NI = F::BM / ROWS, Q = F::BM == 16 ? 1 : 2;
+    const int r = lane % ROWS, g = lane / ROWS;
+    const int rows = t.end - t.begin;
+    float v[NI][Q][4], amax[NI];
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      amax[ni] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4 * Q; ++i) {
+        float gv, uv;
+        if constexpr (F::BM == 16) gv = acc.q[0][i], uv = acc.q[1][i];
+        else gv = acc.v[ni][i], uv = acc.v[ni][i + 8];
+        if (t.limit > 0.0f) {
+          gv = fminf(gv, t.limit);
+          uv = fminf(fmaxf(uv, -t.limit), t.limit);
+        }
+        v[ni][i / 4][i % 4] = silu(gv) * uv;
+        amax[ni] = fmaxf(amax[ni], fabsf(v[ni][i / 4][i % 4]));
+      }
+      if (F::BM == 16) amax[ni] = fmaxf(amax[ni], __shfl_xor(amax[ni], 16, 64));
+      amax[ni] = fmaxf(amax[ni], __shfl_xor(amax[ni], 32, 64));
+      if (g == 0) block_max[wave][ROWS * ni + r] = amax[ni];
+    }
+    stage_barrier();
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni) {
+      const int row = ROWS * ni + r;
+      if (row >= rows) continue;
+      const int s = fp8_term_exponent(fmaxf(amax[ni], block_max[wave ^ 1][row]));
+      const int n = t.nt * TG + 16 * wave;  // the wave's first column
+      const int64_t at = (int64_t)(t.begin + row) * (I / 128);
+      uint8_t* dst = a8 + (at + n / 128) * XSTEP8 + n % 128 + 4 * g;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        uint32_t hi, lo;
+        fp8_terms4(v[ni][q], pow2_biased(254 - s), hi, lo);
+        *reinterpret_cast<uint32_t*>(dst + 8 * q) = hi;
+        *reinterpret_cast<uint32_t*>(dst + 128 + 8 * q) = lo;
+      }
+      if (wave % 2 == 0 && g == 0) a8s[at * 4 + n / 32] = (uint8_t)s;
+    }
+  };
+  stream_tiles<F>(tr, H / 128, lds, wave, lane, locate, setup, epilogue);
+}
+
+// Output rows (bf16, permuted order) of TW columns; wave w owns columns 32 w .. + 31.
+template <typename F, typename Table>
+__device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
+                                            const Lists& L, const Table& routed, const Table& shared, int before,
+                                            uint16_t* __restrict__ out) {
+  const int H = routed.hidden, I = routed.inter;
+  const int n_tiles = (H + F::TW - 1) / F::TW;
+  const TileRange tr = tile_range_after(active_row_tiles<F::BM>(L) * n_tiles, before, F::HOT_COST);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+  auto locate = [&](int j, StreamTile<F>& t) { stream_locate<F>(L, tr.at(j), n_tiles, t); };
+  auto setup = [&](StreamTile<F>& t) {
+    const TileWeights tw = tile_weights_s(routed, shared, t.expert);
+    // a multiple of 128; the rows past a narrow last tile's columns read its first ones
+    const int col0 = t.nt * F::TW, valid = min(F::TW, H - col0);
+    t.ld.weights(tw.w2, tw.w2s, H, I, table_tiled(routed), wave, lane, [=](int j) { return col0 + j % valid; });
+    if constexpr (F::BLOCK_F32)
+      t.s0 = t.s1 = uniform_ptr(reinterpret_cast<const float*>(tw.w2s) +
+                                (int64_t)((col0 + 32 * wave % valid) / 128) * (I / 128));
+    const int begin = t.begin, end = t.end;
+    t.ld.rows(a8, a8s, I, wave, lane, [&](int r) { return begin + r < end ? begin + r : begin; });
+  };
+  auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
+    const int col = t.nt * F::TW + 32 * wave;
+    if (col >= H) return;
+    if constexpr (F::BM == 16) {
+      const int row = t.begin + lane % 16;
+      if (row >= t.end) return;
+      uint16_t* dst = out + (int64_t)row * H + col + lane / 16 * 4;
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        *reinterpret_cast<uint2*>(dst + 16 * q) =
+            make_uint2(pack_bf16x2(acc.q[q][0], acc.q[q][1]), pack_bf16x2(acc.q[q][2], acc.q[q][3]));
+    } else {
+      const int r = lane % 32, g = lane / 32;
+#pragma unroll
+      for (int ni = 0; ni < F::NI; ++ni) {
+        const int row = t.begin + 32 * ni + r;
+        if (row >= t.end) continue;
+        const v16f& a = acc.v[ni];
+        uint16_t* dst = out + (int64_t)row * H + col + 4 * g;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *reinterpret_cast<uint2*>(dst + 8 * q) =
+              make_uint2(pack_bf16x2(a[4 * q], a[4 * q + 1]), pack_bf16x2(a[4 * q + 2], a[4 * q + 3]));
+      }
+    }
+  };
+  stream_tiles<F>(tr, I / 128, lds, wave, lane, locate, setup, epilogue);
+}
+
+// 16-row tiles alone.
+template <typename F, typename Table>
+__global__ void __launch_bounds__(64 * F::WAVES, 2) stream_gate_up_kernel(const uint8_t* __restrict__ x8,
+                                                                          const uint8_t* __restrict__ x8s,
+                                                                          const int32_t* __restrict__ row_token, Lists L,
+                                                                          Table routed, Table shared,
+                                                                          uint8_t* __restrict__ a8,
+                                                                          uint8_t* __restrict__ a8s) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[F::BYTES];
+  stream_gate_up<F>(lds, x8, x8s, row_token, L, routed, shared, 0, a8, a8s);
+}
+template <typename F, typename Table>
+__global__ void __launch_bounds__(64 * F::WAVES, 2) stream_down_kernel(const uint8_t* __restrict__ a8,
+                                                                       const uint8_t* __restrict__ a8s, Lists L,
+                                                                       Table routed, Table shared,
+                                                                       uint16_t* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[F::BYTES];
+  stream_down<F>(lds, a8, a8s, L, routed, shared, 0, out);
+}
+
+// 128-row tiles of the experts with more than 64 rows (`hot`), then 64-row tiles of the others
+// (`cold`, one tile an expert, so its weights are read once). One launch, so that the workgroups
+// with a 128-row tile less take more of the others (tile_range_after: with routing as skewed as
+// natural text's, 2048 tokens over 128 MXFP4 experts of 2048/768, 303 us without and 249 with).
+template <typename F>
+using StreamOf = StreamF<F::FP8, F::A_SCALED, 64, 8>;
+template <typename F>
+constexpr int MIXED_LDS = RingMx<F, F::DA, F::DB>::BYTES > StreamOf<F>::BYTES ? RingMx<F, F::DA, F::DB>::BYTES
+                                                                              : StreamOf<F>::BYTES;
+
+template <typename F, typename Table>
+__global__ void __launch_bounds__(512, 2) mixed_gate_up_kernel(const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
+                                                               const int32_t* __restrict__ row_token, Lists hot,
+                                                               Lists cold, Table routed, Table shared,
+                                                               uint8_t* __restrict__ a8, uint32_t* __restrict__ a8s) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[MIXED_LDS<F>];
+  gate_up_mx<F, F::DA, F::DB>(lds, x8, x8s, row_token, hot, routed, shared, a8, a8s);
+  ring_wait_all();  // no load into the rings and no LDS access of the first part is left
+  stream_gate_up<StreamOf<F>>(lds, x8, x8s, row_token, cold, routed, shared,
+                              active_row_tiles(hot) * ((routed.inter + F::TW / 2 - 1) / (F::TW / 2)), a8, (uint8_t*)a8s);
+}
+template <typename F, typename Table>
+__global__ void __launch_bounds__(512, 2) mixed_down_kernel(const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
+                                                            Lists hot, Lists cold, Table routed, Table shared,
+                                                            uint16_t* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[MIXED_LDS<F>];
+  down_mx<F, F::DA, F::DB>(lds, a8, a8s, hot, routed, shared, out);
+  ring_wait_all();
+  stream_down<StreamOf<F>>(lds, a8, a8s, cold, routed, shared, active_row_tiles(hot) * ((routed.hidden + F::TW - 1) / F::TW),
+                           out);
+}
+
+}  // namespace mf
+}  // namespace wm

@@ -14,7 +14,7 @@
 //             rank among earlier same-expert pairs: stable.
 //
 // Invalid expert ids (< 0 or >= E) are left out of every list; their inverse is -1.
-#include "wm_common.h"
+#include "moe_internal.h"
 
 namespace wm {
 
@@ -105,19 +105,32 @@ __device__ __forceinline__ int32_t block_inclusive_scan(int32_t v, int32_t* wave
 
 // One workgroup of 1024 threads, thread e = expert e: offsets[e] (exclusive scan of the
 // totals), offsets[E], the tile count, and expert e's tiles (expert, first row) at its
-// place in the list.
+// place in the list. With cold_rows, the experts of up to that many rows go to cold_tiles
+// instead, one tile each, counted in tile_count[1].
 __global__ void __launch_bounds__(1024) permute_offsets_kernel(const int32_t* __restrict__ totals, int experts,
-                                                              int tile_rows, int32_t* __restrict__ offsets,
+                                                              int tile_rows, int cold_rows,
+                                                              int32_t* __restrict__ offsets,
                                                               int32_t* __restrict__ tiles,
+                                                              int32_t* __restrict__ cold_tiles,
                                                               int32_t* __restrict__ tile_count) {
   __shared__ int32_t wave_total[16];
   __shared__ int32_t tile_start[PERMUTE_MAX_EXPERTS + 1];
   __shared__ int32_t row_start[PERMUTE_MAX_EXPERTS];
   const int e = threadIdx.x;
   const int32_t mine = e < experts ? totals[e] : 0;
-  const int32_t my_tiles = (mine + tile_rows - 1) / tile_rows;
+  const bool cold = mine <= cold_rows;
+  const int32_t my_tiles = cold ? 0 : (mine + tile_rows - 1) / tile_rows;
   const int32_t rows_incl = block_inclusive_scan(mine, wave_total);
   const int32_t tiles_incl = block_inclusive_scan(my_tiles, wave_total);
+  if (cold_rows > 0) {  // one tile each, in their own list
+    const int32_t mine_cold = cold && mine > 0 ? 1 : 0;
+    const int32_t cold_incl = block_inclusive_scan(mine_cold, wave_total);
+    if (mine_cold) {
+      cold_tiles[2 * (cold_incl - 1)] = e;
+      cold_tiles[2 * (cold_incl - 1) + 1] = rows_incl - mine;
+    }
+    if (e == experts - 1) tile_count[1] = cold_incl;
+  }
   if (e < experts) {
     const int32_t row0 = rows_incl - mine, tile0 = tiles_incl - my_tiles;
     offsets[e] = row0;
@@ -181,6 +194,30 @@ __global__ void __launch_bounds__(64) permute_scatter_kernel(const int32_t* __re
   }
 }
 
+// See moe_internal.h.
+void permute_tiles(const int32_t* indices, int64_t pairs, int experts, int tile_rows, int cold_rows, int32_t* order,
+                   int32_t* inverse, int32_t* offsets, int32_t* tiles, int32_t* cold_tiles, int32_t* tile_count,
+                   void* workspace, hipStream_t s) {
+  const int64_t chunks = (pairs + PERMUTE_CHUNK - 1) / PERMUTE_CHUNK;
+  int32_t* counts = (int32_t*)workspace;
+  int32_t* totals = counts + (size_t)(chunks > 0 ? chunks : 1) * experts;
+  if (chunks > 0) {
+    hipLaunchKernelGGL(permute_count_kernel, dim3((unsigned)chunks), dim3(64), 0, s, indices, pairs, experts, counts);
+    check_launch("permute_count");
+  }
+  hipLaunchKernelGGL(permute_colscan_kernel, dim3((unsigned)((experts + SCAN_EXPERTS - 1) / SCAN_EXPERTS)),
+                     dim3(64 * SCAN_SEGS), 0, s, counts, chunks, experts, totals);
+  check_launch("permute_colscan");
+  hipLaunchKernelGGL(permute_offsets_kernel, dim3(1), dim3(1024), 0, s, totals, experts, tile_rows, cold_rows, offsets, tiles,
+                     cold_tiles, tile_count);
+  check_launch("permute_offsets");
+  if (chunks > 0) {
+    hipLaunchKernelGGL(permute_scatter_kernel, dim3((unsigned)chunks), dim3(64), 0, s, indices, pairs, experts, counts,
+                       offsets, order, inverse);
+    check_launch("permute_scatter");
+  }
+}
+
 }  // namespace wm
 
 using namespace wm;
@@ -203,25 +240,8 @@ WM_EXPORT int wm_permute(const int32_t* indices, int64_t pairs, int32_t experts,
     if (workspace_bytes < wm_permute_workspace_size(pairs, experts)) fail("wm_permute: workspace too small");
     if (!offsets || !tile_count || !workspace || (pairs > 0 && (!indices || !order || !inverse || !tiles)))
       fail("wm_permute: null pointer");
-    int64_t chunks = (pairs + PERMUTE_CHUNK - 1) / PERMUTE_CHUNK;
-    int32_t* counts = (int32_t*)workspace;
-    int32_t* totals = counts + (size_t)(chunks > 0 ? chunks : 1) * experts;
-    hipStream_t s = as_stream(stream);
-    if (chunks > 0) {
-      hipLaunchKernelGGL(permute_count_kernel, dim3((unsigned)chunks), dim3(64), 0, s, indices, pairs, experts, counts);
-      check_launch("permute_count");
-    }
-    hipLaunchKernelGGL(permute_colscan_kernel, dim3((unsigned)((experts + SCAN_EXPERTS - 1) / SCAN_EXPERTS)),
-                       dim3(64 * SCAN_SEGS), 0, s, counts, chunks, experts, totals);
-    check_launch("permute_colscan");
-    hipLaunchKernelGGL(permute_offsets_kernel, dim3(1), dim3(1024), 0, s, totals, experts, tile_rows, offsets, tiles,
-                       tile_count);
-    check_launch("permute_offsets");
-    if (chunks > 0) {
-      hipLaunchKernelGGL(permute_scatter_kernel, dim3((unsigned)chunks), dim3(64), 0, s, indices, pairs, experts, counts,
-                         offsets, order, inverse);
-      check_launch("permute_scatter");
-    }
+    permute_tiles(indices, pairs, experts, tile_rows, 0, order, inverse, offsets, tiles, nullptr, tile_count, workspace,
+                  as_stream(stream));
   });
 }
 
