@@ -1,0 +1,85 @@
+"""MXFP4 calls of a few tokens (T k <= 256 pairs of experts large enough, T k H I >= 1.2e8): grouped 8-row tiles whose activations enter as four
+E4M3 terms and whose rows stay fp32, against the oracle's fp32 experts and a float64 combine.
+
+Bounds: y is rounded to bf16 once, at most 2^-9 of each value, so 2^-9 of the result's norm; the
+fp32 sums and the terms (below 2^-17 of a block's maximum) get 2^-13 more. Rows or act kept in
+16 bits would not pass: they add 2^-9 each.
+"""
+import numpy as np
+import pytest
+import torch
+
+import whallm_amd as wa
+from oracle import moe as M
+from whallm_amd import synthetic as S
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 2.0 ** -9 + 2.0 ** -13
+
+
+def oracle_experts(a):
+    return [M.MXFP4Expert(a["gate_up"][e], a["gate_up_scales"][e], a["down"][e], a["down_scales"][e])
+            for e in range(len(a["gate_up"]))]
+
+
+# one row an expert and none, 8 and 9 rows of one expert, up to 32 of each, as many pairs as the path
+# takes; K of the fewest, odd and many steps, last column tiles of half width
+@pytest.mark.parametrize("T,k,E,H,I", [(32, 8, 512, 1024, 512), (25, 10, 64, 1152, 640), (32, 8, 9, 384, 1280),
+                                       (16, 16, 16, 1280, 384), (9, 2, 2, 4096, 2048), (8, 1, 1, 7168, 2432),
+                                       (3, 4, 4, 5120, 2304)])
+def test_few_tokens_match_oracle(device, T, k, E, H, I):
+    rng = np.random.default_rng(T + k + E + H + I)
+    arrays, shared_arrays = S.mxfp4_experts_np(rng, E, H, I), S.mxfp4_experts_np(rng, 1, H, I)
+    x_bits, g_bits = S.bf16_normal_np(rng, (T, H)), S.bf16_normal_np(rng, (H,), 0.02)
+    x_bits[:, :32] = 0                       # a block of zeros
+    x_bits[T - 1, 64:96] = (x_bits[T - 1, 64:96] & 0x807f) | np.uint16(2 << 7)  # tiny values
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    w = rng.random((T, k)).astype(np.float32) + 0.1
+    routed, shared = S.experts_to_device(arrays, device), S.experts_to_device(shared_arrays, device)
+    x, gate = S.bf16_bits_to_tensor(x_bits, device), S.bf16_bits_to_tensor(g_bits, device)
+    i_d, w_d = torch.from_numpy(ids).to(device), torch.from_numpy(w).to(device)
+    xf = S.bf16_bits_to_f32(x_bits)
+    rows = M.routed_outputs(xf, ids, oracle_experts(arrays))
+    want = M.combine(rows, w, M.expert_ffn(xf, oracle_experts(shared_arrays)[0]),
+                     xf.astype(np.float64) @ S.bf16_bits_to_f32(g_bits).astype(np.float64))
+
+    def close(got, ref):
+        ref = np.asarray(ref, dtype=np.float64)
+        assert np.linalg.norm(got.double().cpu().numpy() - ref) <= BOUND * np.linalg.norm(ref)
+
+    close(wa.moe_mxfp4(x, i_d, w_d, routed, shared, gate), want)
+    close(wa.experts_mxfp4(x, i_d, routed), rows)
+
+
+def test_few_tokens_slots_masks_and_replays(device):
+    """Non-resident and out-of-range experts add nothing (zero rows per pair), a masked pair's row is left
+    as it is, and a captured call gives the same bits on every replay."""
+    rng = np.random.default_rng(7)
+    T, k, E, H, I = 6, 4, 12, 2560, 2048
+    slots = np.arange(E, dtype=np.int32)
+    slots[2], slots[5] = 5, -1
+    tab = S.experts_to_device(S.mxfp4_experts_np(rng, E, H, I), device, slots=torch.from_numpy(slots).to(device), experts=E)
+    x = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (T, H)), device)
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    ids[0, 0], ids[1, 1] = 5, E
+    live = (ids != 5) & (ids != E)
+    i_d, w_d = torch.from_numpy(ids).to(device), torch.rand(T, k, device=device) + 0.1
+    per_pair = wa.experts_mxfp4(x, i_d, tab).double()
+    assert bool((per_pair[torch.from_numpy(~live).to(device)] == 0).all())
+    want = (per_pair * w_d.double()[..., None]).sum(1)
+    got = wa.moe_mxfp4(x, i_d, w_d, tab)
+    assert (got.double() - want).norm() <= 2 * BOUND * want.norm()  # the pairs' rows are rounded too
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        wa.moe_mxfp4(x, i_d, w_d, tab)
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph):
+        captured = wa.moe_mxfp4(x, i_d, w_d, tab)
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, got)
+        assert torch.equal(wa.moe_mxfp4(x, i_d, w_d, tab), got)

@@ -320,6 +320,27 @@ __device__ __forceinline__ void fp8_terms4(const float (&v)[4], float f, uint32_
   lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[2], l[3], (int)u01, true);
 }
 
+// Four terms, for fp32 values: each the E4M3 rounding of 16 times what the one before it leaves, under
+// the scales s, s - 4, s - 8, s - 12. What is left is below 2^-17 of the block's maximum.
+__device__ __forceinline__ int fp8_term_exponent_wide(float amax) {
+  const int s = fp8_term_exponent(amax);
+  return s > 13 ? s : 13;  // the fourth term's scale stays a normal power of two
+}
+__device__ __forceinline__ void fp8_terms4_wide(const float (&v)[4], float f, uint32_t (&t)[4]) {
+  float h[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = v[j] * f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[0], h[1], 0, false);
+    t[e] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[2], h[3], (int)w01, true);
+    h[0] = (h[0] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 0)) * 16.0f;
+    h[1] = (h[1] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 1)) * 16.0f;
+    h[2] = (h[2] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 2)) * 16.0f;
+    h[3] = (h[3] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 3)) * 16.0f;
+  }
+}
+
 // The hi and lo E4M3 terms of one 32-value block (v in K order) as 8 words each (byte i of
 // the 32 = value i), and the hi scale byte.
 __device__ __forceinline__ void fp8_terms32(const float (&v)[32], uint32_t (&hi)[8], uint32_t (&lo)[8], int& s_hi) {
@@ -1387,8 +1408,9 @@ __device__ __forceinline__ bool pair_resident(const int32_t* __restrict__ indice
 // non-resident expert contribute nothing; so does a non-resident shared expert.
 // per-pair (combine = 0): out[p, c] = rows[inverse[p], c], a zero row for an unknown or
 // non-resident expert, and no write at all for a masked pair (negative index).
-// 8 columns per thread.
-__global__ void __launch_bounds__(256) combine_rows_kernel(const uint16_t* __restrict__ rows,
+// 8 columns per thread. Row: bf16 or fp32 rows.
+template <typename Row>
+__global__ void __launch_bounds__(256) combine_rows_kernel(const Row* __restrict__ rows,
                                                            const int32_t* __restrict__ inverse,
                                                            const float* __restrict__ weights,
                                                            const float* __restrict__ gate, int tokens, int k,
@@ -1405,18 +1427,38 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(const uint16_t* __res
     if (indices[t] < 0) return;
     const int row = inverse[t];
     const bool live = row >= 0 && pair_resident(indices, slots, t);
-    const uint4 v = live ? reinterpret_cast<const uint4*>(rows + (int64_t)row * hidden)[c8] : make_uint4(0, 0, 0, 0);
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if constexpr (sizeof(Row) == 2) {
+      if (live) v = reinterpret_cast<const uint4*>(rows + (int64_t)row * hidden)[c8];
+    } else if (live) {
+      const float4* src = reinterpret_cast<const float4*>(rows + (int64_t)row * hidden) + 2 * c8;
+      const float4 a = src[0], b = src[1];
+      v = make_uint4(pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w));
+    }
     reinterpret_cast<uint4*>(out + (int64_t)t * hidden)[c8] = v;
     return;
   }
   const bool shared_live = has_shared && (!shared_slots || shared_slots[0] >= 0);
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  auto add = [&](const uint4 v, float s) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  struct Eight {
+    uint4 v[sizeof(Row) / 2];
+  };
+  auto add = [&](const Eight& r, float s) {
+    if constexpr (sizeof(Row) == 2) {
+      const uint32_t w[4] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      acc[2 * q] = fmaf(s, bf16_bits_to_f32(w[q] & 0xffffu), acc[2 * q]);
-      acc[2 * q + 1] = fmaf(s, bf16_bits_to_f32(w[q] >> 16), acc[2 * q + 1]);
+      for (int q = 0; q < 4; ++q) {
+        acc[2 * q] = fmaf(s, bf16_bits_to_f32(w[q] & 0xffffu), acc[2 * q]);
+        acc[2 * q + 1] = fmaf(s, bf16_bits_to_f32(w[q] >> 16), acc[2 * q + 1]);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        acc[4 * q] = fmaf(s, __uint_as_float(r.v[q].x), acc[4 * q]);
+        acc[4 * q + 1] = fmaf(s, __uint_as_float(r.v[q].y), acc[4 * q + 1]);
+        acc[4 * q + 2] = fmaf(s, __uint_as_float(r.v[q].z), acc[4 * q + 2]);
+        acc[4 * q + 3] = fmaf(s, __uint_as_float(r.v[q].w), acc[4 * q + 3]);
+      }
     }
   };
   // the rows of the token's pairs and its shared row are loaded before any is summed (sums
@@ -1426,8 +1468,12 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(const uint16_t* __res
   const int n = k + (has_shared ? 1 : 0);
   auto load_row = [&](int r) {
     const __amdgpu_buffer_rsrc_t rr =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(rows + (int64_t)r * hidden), 0, hidden * 2, 0x00020000);
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rr, c8 * 16, 0, 2));
+        __builtin_amdgcn_make_buffer_rsrc((void*)(rows + (int64_t)r * hidden), 0, hidden * (int)sizeof(Row), 0x00020000);
+    Eight e;
+#pragma unroll
+    for (int q = 0; q < (int)sizeof(Row) / 2; ++q)
+      e.v[q] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rr, c8 * 8 * (int)sizeof(Row) + 16 * q, 0, 2));
+    return e;
   };
   auto row_of = [&](int j) {
     int r = j < k ? inverse[t * k + j] : (j < n && shared_live ? pairs + t : -1);
@@ -1437,7 +1483,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(const uint16_t* __res
   constexpr int ONE_PASS = 17;  // up to 16 pairs + the shared row in one unrolled pass
   if (n <= ONE_PASS) {
     int row[ONE_PASS];
-    uint4 v[ONE_PASS];
+    Eight v[ONE_PASS];
 #pragma unroll
     for (int j = 0; j < ONE_PASS; ++j) row[j] = j < n ? row_of(j) : -1;
 #pragma unroll
@@ -1450,7 +1496,7 @@ __global__ void __launch_bounds__(256) combine_rows_kernel(const uint16_t* __res
   constexpr int BATCH = 16;
   for (int j0 = 0; n > ONE_PASS && j0 < n; j0 += BATCH) {
     int row[BATCH];
-    uint4 v[BATCH];
+    Eight v[BATCH];
 #pragma unroll
     for (int q = 0; q < BATCH; ++q) row[q] = j0 + q < n ? row_of(j0 + q) : -1;
 #pragma unroll
@@ -1667,10 +1713,10 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
     if (how == ROWS_16) {
       using S = StreamF<false, true, 16, 4>;
       hipLaunchKernelGGL((stream_gate_up_kernel<S, Table>), grid_for(I / (S::TW / 2)), dim3(64 * S::WAVES), 0, s, x6, x6s,
-                         row_token, L, routed, sh, a6, (uint8_t*)a6s);
+                         row_token, L, routed, sh, 0, 0, a6, (uint8_t*)a6s);
       mid();
       hipLaunchKernelGGL((stream_down_kernel<S, Table>), grid_for((H + S::TW - 1) / S::TW), dim3(64 * S::WAVES), 0, s, a6,
-                         (const uint8_t*)a6s, L, routed, sh, out_rows);
+                         (const uint8_t*)a6s, L, routed, sh, 0, out_rows);
     }
   }
   if constexpr (F::Terms::E4) {
@@ -1694,16 +1740,238 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
   if (te) check_hip(hipEventRecord(te->ev[2], s), "hipEventRecord");
   const int32_t* shared_slots = has_shared ? shared->slots : nullptr;
   if (combine)
-    hipLaunchKernelGGL(combine_rows_kernel, dim3(tokens, (H / 8 + 255) / 256), dim3(256), 0, s, out_rows, inverse,
+    hipLaunchKernelGGL((combine_rows_kernel<uint16_t>), dim3(tokens, (H / 8 + 255) / 256), dim3(256), 0, s, out_rows, inverse,
                        weights, L.shared_gate, tokens, k, H, has_shared ? 1 : 0, 1, indices, routed.slots,
                        shared_slots, y);
   else
-    hipLaunchKernelGGL(combine_rows_kernel, dim3((unsigned)pairs, (H / 8 + 255) / 256), dim3(256), 0, s, out_rows,
+    hipLaunchKernelGGL((combine_rows_kernel<uint16_t>), dim3((unsigned)pairs, (H / 8 + 255) / 256), dim3(256), 0, s, out_rows,
                        inverse, weights, L.shared_gate, tokens, k, H, 0, 0, indices, routed.slots, nullptr, y);
   check_launch("combine_rows");
 }
 
+// ---------------------------------------------------------------------------------
+// A few tokens (T k <= 256 pairs) of MXFP4 row-layout experts: the 16-row streaming tiles with the
+// decode GEMV's precision. The GEMV passes an expert's weights once per pair that chose it (the shared
+// expert's once per token) and is bound by its converts and by act reads past the first token:
+// 1.7 TB/s in down. Here a weight row is read once per 8 rows, at the streaming tiles' rate; four E4M3
+// terms carry x exactly and the fp32 act to 2^-17 of its block (the matrix instructions
+// have 16 columns and an expert few rows, so the second pair of terms takes the columns
+// 8..15), and the rows stay fp32 up to the combine. One launch does what the prefill's
+// permute, row map, split and gate launches do.
+constexpr int FEW_PAIRS = 256;
+
+// Block 0: the pair lists (thread p: pair p). Blocks 1 .. split: the terms of x, a lane per 32-value
+// block, the third and fourth as rows tokens .. 2 tokens - 1. The others: the shared gate, a wave
+// per token.
+__global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restrict__ x, int tokens, int hidden,
+                                                       const int32_t* __restrict__ indices, int k, int experts,
+                                                       const uint16_t* __restrict__ g, int split_blocks,
+                                                       int32_t* __restrict__ inverse, int32_t* __restrict__ offsets,
+                                                       int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count,
+                                                       int32_t* __restrict__ row_token, float* __restrict__ gate,
+                                                       uint8_t* __restrict__ x8, uint32_t* __restrict__ x8s) {
+  const int pairs = tokens * k;
+  if (blockIdx.x == 0) {
+    __shared__ __attribute__((aligned(16))) int32_t id[FEW_PAIRS], head[FEW_PAIRS];
+    const int p = threadIdx.x;
+    const int32_t raw = p < pairs ? indices[p] : -1;
+    const bool valid = raw >= 0 && raw < experts;
+    const int32_t e = valid ? raw : 0x7fffffff;  // after every expert
+    id[p] = e;
+    __syncthreads();
+    int before = 0, rank = 0, count = 0;  // pairs of lower experts, earlier ones of this, all of this
+#pragma unroll 4
+    for (int j = 0; j < pairs; j += 4) {  // the words past the last pair hold no expert
+      const int4 o = *reinterpret_cast<const int4*>(&id[j]);
+      const int32_t q[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        before += q[c] < e;
+        rank += q[c] == e && j + c < p;
+        count += q[c] == e;
+      }
+    }
+    const bool first = valid && rank % 8 == 0;  // a tile's first row
+    head[p] = first ? before + rank : 0x7fffffff;
+    __syncthreads();
+    const int row = before + rank;
+    int tile = 0, total = 0;
+#pragma unroll 4
+    for (int j = 0; j < pairs; j += 4) {
+      const int4 o = *reinterpret_cast<const int4*>(&head[j]);
+      tile += (o.x < row) + (o.y < row) + (o.z < row) + (o.w < row);
+      total += (o.x != 0x7fffffff) + (o.y != 0x7fffffff) + (o.z != 0x7fffffff) + (o.w != 0x7fffffff);
+    }
+    if (first) {
+      tiles[2 * tile] = e;
+      tiles[2 * tile + 1] = row;
+      if (rank == 0) {  // read for experts with tiles only
+        offsets[e] = before;
+        offsets[e + 1] = before + count;
+      }
+    }
+    if (p < pairs) inverse[p] = valid ? row : -1;
+    if (valid) row_token[row] = p / k;
+    for (int t = p; t < tokens; t += 256) row_token[pairs + t] = t;  // the shared rows
+    if (p == 0) tile_count[0] = total;
+    return;
+  }
+  if ((int)blockIdx.x > split_blocks) {
+    const int t = ((int)blockIdx.x - 1 - split_blocks) * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (t >= tokens) return;
+    float v = 1.0f;
+    if (g) {
+      const uint32_t* xr = reinterpret_cast<const uint32_t*>(x) + (int64_t)t * (hidden / 2);
+      const uint32_t* gr = reinterpret_cast<const uint32_t*>(g);
+      float a = 0.0f;
+      for (int q = lane; q < hidden / 2; q += 64) a = dot2_bf16(bits_to_bf16x2(xr[q]), bits_to_bf16x2(gr[q]), a);
+      a = segment_sum<64>(a);
+      v = 1.0f / (1.0f + __expf(-a));
+    }
+    if (lane == 0) gate[t] = v;
+    return;
+  }
+  const int blocks = hidden / 32;
+  const int job = ((int)blockIdx.x - 1) * 256 + threadIdx.x;  // (token, block)
+  if (job >= tokens * blocks) return;
+  const int row = job / blocks, blk = job % blocks;
+  const uint4* src = reinterpret_cast<const uint4*>(x + (int64_t)row * hidden + blk * 32);
+  float v[8][4];
+  float amax = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint4 u = src[q];
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = bf16_bits_to_f32(w[j] & 0xffffu), b = bf16_bits_to_f32(w[j] >> 16);
+      v[2 * q + j / 2][2 * (j % 2)] = a;
+      v[2 * q + j / 2][2 * (j % 2) + 1] = b;
+      amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
+    }
+  }
+  const int s = fp8_term_exponent_wide(amax);
+  uint32_t t[4][8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    uint32_t four[4];
+    fp8_terms4_wide(v[q], pow2_biased(254 - s), four);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e][q] = four[e];
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t at = ((int64_t)(row + h * tokens) * (hidden / 128) + blk / 4);
+    uint8_t* step = x8 + at * XSTEP8 + (blk % 4) * 32;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint32_t* w = t[2 * h + e];
+      uint4* dst = reinterpret_cast<uint4*>(step + 128 * e);
+      dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+      dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+    reinterpret_cast<uint8_t*>(x8s + at)[blk % 4] = (uint8_t)(s - 8 * h);
+  }
+}
+
+struct FewLayout {
+  size_t inverse, offsets, tiles, tile_count, gate, row_token, x8, x8s, a8, a8s, rows, total;
+};
+static FewLayout few_layout(int tokens, int k, int experts, int hidden, int inter) {
+  const size_t pairs = (size_t)tokens * k, rows = pairs + tokens;
+  FewLayout p{};
+  size_t at = 0;
+  auto take = [&](size_t& where, size_t bytes) {
+    where = at;
+    at += align256(bytes);
+  };
+  take(p.inverse, 4 * pairs);
+  take(p.offsets, 4 * (size_t)(experts + 1));
+  take(p.tiles, 8 * pairs);
+  take(p.tile_count, 4);
+  take(p.gate, 4 * (size_t)tokens);
+  take(p.row_token, 4 * rows);
+  take(p.x8, 2 * (size_t)tokens * (hidden / 128) * XSTEP8);
+  take(p.x8s, 2 * (size_t)tokens * (hidden / 128) * 4);
+  take(p.a8, 2 * rows * (inter / 128) * XSTEP8);
+  take(p.a8s, 2 * rows * (inter / 128) * 4);
+  take(p.rows, 4 * rows * hidden);
+  p.total = at;
+  return p;
+}
+
+static void run_few(const uint16_t* x, int tokens, const int32_t* indices, const float* weights, int k,
+                    const wm_mxfp4_experts& routed, const wm_mxfp4_experts* shared, const uint16_t* shared_gate,
+                    uint16_t* y, bool combine, void* ws, hipStream_t s) {
+  const int H = routed.hidden, I = routed.inter;
+  const bool has_shared = combine && shared != nullptr;
+  const FewLayout p = few_layout(tokens, k, routed.experts, H, I);
+  const int pairs = tokens * k, rows = pairs + tokens;
+  uint8_t* base = (uint8_t*)ws;
+  Lists L{};
+  L.offsets = (int32_t*)(base + p.offsets);
+  L.tiles = (int32_t*)(base + p.tiles);
+  L.tile_count = (int32_t*)(base + p.tile_count);
+  L.shared_gate = (float*)(base + p.gate);
+  L.pairs = pairs;
+  L.tokens = tokens;
+  L.k = k;
+  L.has_shared = has_shared ? 1 : 0;
+  int32_t* inverse = (int32_t*)(base + p.inverse);
+  int32_t* row_token = (int32_t*)(base + p.row_token);
+  uint8_t *x8 = base + p.x8, *x8s = base + p.x8s, *a8 = base + p.a8, *a8s = base + p.a8s;
+  float* out_rows = (float*)(base + p.rows);
+  const int split_blocks = (tokens * (H / 32) + 255) / 256, gate_blocks = has_shared ? (tokens + 3) / 4 : 0;
+  hipLaunchKernelGGL(few_prep_kernel, dim3(1 + split_blocks + gate_blocks), dim3(256), 0, s, x, tokens, H, indices, k,
+                     routed.experts, shared_gate, split_blocks, inverse, (int32_t*)L.offsets, (int32_t*)L.tiles,
+                     (int32_t*)L.tile_count, row_token, (float*)L.shared_gate, x8, (uint32_t*)x8s);
+  check_launch("few_prep");
+  const wm_mxfp4_experts sh = shared ? *shared : routed;
+  using S = StreamF<false, true, 16, 4, true>;
+  const int row_tiles = pairs + (has_shared ? (tokens + S::ROWS - 1) / S::ROWS : 0);  // at most
+  auto grid_for = [&](int n_tiles) {
+    const int per_xcd = std::min((row_tiles * n_tiles + XCDS - 1) / XCDS, std::max(compute_units() / XCDS, 1) * 2);
+    return dim3((unsigned)(per_xcd * XCDS));
+  };
+  hipLaunchKernelGGL((stream_gate_up_kernel<S, wm_mxfp4_experts>), grid_for(I / (S::TW / 2)), dim3(64 * S::WAVES), 0, s, x8,
+                     x8s, row_token, L, routed, sh, tokens, rows, a8, a8s);
+  check_launch("few gate_up");
+  hipLaunchKernelGGL((stream_down_kernel<S, wm_mxfp4_experts>), grid_for((H + S::TW - 1) / S::TW), dim3(64 * S::WAVES), 0, s,
+                     a8, a8s, L, routed, sh, rows, (void*)out_rows);
+  check_launch("few down");
+  const dim3 cgrid(combine ? tokens : pairs, (H / 8 + 63) / 64);
+  hipLaunchKernelGGL((combine_rows_kernel<float>), cgrid, dim3(64), 0, s, out_rows, inverse, weights, L.shared_gate, tokens, k,
+                     H, has_shared ? 1 : 0, combine ? 1 : 0, indices, routed.slots, has_shared ? shared->slots : nullptr, y);
+  check_launch("combine_rows");
+}
+
 }  // namespace mf
+
+// The line to the GEMV is the bytes of weights that it would pass, T k times an expert's 1.5 H I: below
+// about 180 MB its two launches are the faster (us of a whole call, GEMV / here): 2048/512 top 10,
+// 8 tokens (126 MB) 45/55, 12 (189 MB) 62.5/62.8, 25 116/88; 2560/640 top 10, 6 (147 MB) 60/62, 8 (197 MB)
+// 78/67, 25 199/131; 4096/2048 top 8, 1 (101 MB) 53/59, 2 94/77, 8 326/146, 32 1205/296; 5120/2304 top 6,
+// 1 (106 MB) 51/56, 2 83/76, 8 288/187, 32 1098/550.
+constexpr int64_t FEW_WEIGHTS = 120000000;  // T k H I
+
+bool few_mxfp4_takes(int tokens, int k, const wm_mxfp4_experts& e) {
+  if (e.tiled || e.hidden % 128 || e.inter % 128 || e.hidden < 384 || e.inter < 384) return false;
+  if (!decode_mxfp4_supports(e.hidden, e.inter)) return false;
+  const int64_t pairs = (int64_t)tokens * k;
+  return pairs <= mf::FEW_PAIRS && pairs * e.hidden * e.inter >= FEW_WEIGHTS;
+}
+bool few_mxfp4_aligned(const wm_mxfp4_experts* e) {  // a row's 4 scale bytes are read as one dword
+  auto dword = [](const void* p, int64_t stride) { return (uintptr_t)p % 4 == 0 && stride % 4 == 0; };
+  return !e || (dword(e->gate_up_scales, e->gate_up_scales_stride) && dword(e->down_scales, e->down_scales_stride));
+}
+size_t few_mxfp4_workspace_size(int tokens, int k, const wm_mxfp4_experts& e) {
+  return mf::few_layout(tokens, k, e.experts, e.hidden, e.inter).total;
+}
+void few_mxfp4(const uint16_t* x, int tokens, const int32_t* indices, const float* weights, int k,
+               const wm_mxfp4_experts& routed, const wm_mxfp4_experts* shared, const uint16_t* shared_gate, uint16_t* y,
+               bool combine, void* ws, hipStream_t s) {
+  mf::run_few(x, tokens, indices, weights, k, routed, shared, shared_gate, y, combine, ws, s);
+}
 
 size_t prefill_workspace_size(int tokens, int k, const wm_mxfp4_experts& e, bool has_shared) {
   return mf::layout(tokens, k, e.experts, e.hidden, e.inter, has_shared).total;

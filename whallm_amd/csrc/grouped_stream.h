@@ -17,7 +17,8 @@
 // Both go to LDS rings of three slots by direct loads, two units (steps) ahead, across tiles.
 // Two shapes: 64 rows x 256 weight rows (8 waves, 154 KB), one row tile an expert; and, for MXFP4, 16
 // rows x 128 (4 waves, 77 KB), two workgroups on a CU, one's epilogue and tile set-up under the
-// other's loads. row_tiles() says which call takes which, with times. At 2 rows an expert of
+// other's loads. row_tiles() says which call takes which, with times. WIDE: the 16-row shape for calls
+// of a few tokens, 8 rows a tile with activations of four terms (see run_few). At 2 rows an expert of
 // 7168/2048 FP8 weights (11.3 GB): 1486 us a call against 2791 with 128-row tiles, 7.6 TB/s.
 #pragma once
 
@@ -26,8 +27,11 @@ namespace mf {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <bool FP8_, bool A_SCALED_, int BM_, int WAVES_>
+template <bool FP8_, bool A_SCALED_, int BM_, int WAVES_, bool WIDE_ = false>
 struct StreamF {
+  // WIDE: tile row r >= 8 holds the third and fourth term of row r - 8
+  static constexpr bool WIDE = WIDE_;
+  static constexpr int ROWS = WIDE_ ? 8 : BM_;  // rows of a tile
   static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
   static constexpr int BM = BM_, WAVES = WAVES_, NI = 2, TW = 32 * WAVES_;  // NI: 32-row row tiles of 64 rows
   static constexpr int SUB = FP8_ ? 1 : 2;                 // K steps of a weight unit
@@ -44,6 +48,7 @@ struct StreamF {
   // loads of a wave: a unit's, and at least a split-row slot's (see issue_rows)
   static constexpr int UNIT_LOADS = NQA + (A_SCALED_ ? 1 : 0), ROW_LOADS = BM_ == 16 ? BSUB + 1 : 2;
   static_assert(BM_ == 16 ? NQB == 1 && !FP8_ : BM_ == 64 && NQB == 2, "the loader's split-row loads");
+  static_assert(!WIDE_ || BM_ == 16, "four terms: 16-row tiles");
 };
 
 // Loads of one tile. Weight load i of wave w fills rows 8 (w + WAVES i) .. + 7 of the tile: lane l
@@ -156,8 +161,8 @@ template <typename F>
 __device__ __forceinline__ void stream_locate(const Lists& L, int logical, int n_tiles, StreamTile<F>& t) {
   int mt = logical / n_tiles;
   t.nt = logical - mt * n_tiles;
-  if constexpr (F::BM == 16) order_tile<F::BM>(L, logical, n_tiles, mt, t.nt);
-  resolve_tile_s<F::BM>(L, mt, t.expert, t.begin, t.end);
+  if constexpr (F::BM == 16) order_tile<F::ROWS>(L, logical, n_tiles, mt, t.nt);
+  resolve_tile_s<F::ROWS>(L, mt, t.expert, t.begin, t.end);
 }
 
 // A wave's results: 32-row weight tile x two 32-row row tiles (v_mfma_scale_f32_32x32x64), or with 16 rows
@@ -336,13 +341,13 @@ __device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uin
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
                                                const int32_t* __restrict__ row_token, const Lists& L, const Table& routed,
-                                               const Table& shared, int before, uint8_t* __restrict__ a8,
-                                               uint8_t* __restrict__ a8s) {
+                                               const Table& shared, int before, int x_rows, int a_rows,
+                                               uint8_t* __restrict__ a8, uint8_t* __restrict__ a8s) {
   float(*block_max)[F::BM] = reinterpret_cast<float(*)[F::BM]>(lds + F::RINGS);
   constexpr int TG = F::TW / 2;
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = I / TG;  // I is a multiple of 128
-  const TileRange tr = tile_range_after(active_row_tiles<F::BM>(L) * n_tiles, before, F::HOT_COST);
+  const TileRange tr = tile_range_after(active_row_tiles<F::ROWS>(L) * n_tiles, before, F::HOT_COST);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   auto locate = [&](int j, StreamTile<F>& t) { stream_locate<F>(L, tr.at(j), n_tiles, t); };
   auto setup = [&](StreamTile<F>& t) {
@@ -356,7 +361,10 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
       t.s1 = uniform_ptr(reinterpret_cast<const float*>(tw.w13s) + (int64_t)(up0 / 128) * (H / 128));
     }
     const int begin = t.begin, end = t.end;
-    t.ld.rows(x8, x8s, H, wave, lane, [&](int r) { return scalar_i32(row_token, begin + r < end ? begin + r : begin); });
+    t.ld.rows(x8, x8s, H, wave, lane, [&](int r) {
+      const int q = begin + r % F::ROWS;
+      return scalar_i32(row_token, q < end ? q : begin) + (r < F::ROWS ? 0 : x_rows);
+    });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
     // Lane (r, g) holds row r of row tile ni, values [q][i] of the wave's columns 4 g + 8 q + i.
@@ -372,6 +380,10 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
         float gv, uv;
         if constexpr (F::BM == 16) gv = acc.q[0][i], uv = acc.q[1][i];
         else gv = acc.v[ni][i], uv = acc.v[ni][i + 8];
+        if constexpr (F::WIDE) {  // the upper terms' products, in the lane of row r +- 8
+          gv += __shfl_xor(gv, 8, 64);
+          uv += __shfl_xor(uv, 8, 64);
+        }
         if (t.limit > 0.0f) {
           gv = fminf(gv, t.limit);
           uv = fminf(fmaxf(uv, -t.limit), t.limit);
@@ -388,18 +400,30 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
     for (int ni = 0; ni < NI; ++ni) {
       const int row = ROWS * ni + r;
       if (row >= rows) continue;
-      const int s = fp8_term_exponent(fmaxf(amax[ni], block_max[wave ^ 1][row]));
+      const float block = fmaxf(amax[ni], block_max[wave ^ 1][row]);
+      const int s = F::WIDE ? fp8_term_exponent_wide(block) : fp8_term_exponent(block);
       const int n = t.nt * TG + 16 * wave;  // the wave's first column
       const int64_t at = (int64_t)(t.begin + row) * (I / 128);
       uint8_t* dst = a8 + (at + n / 128) * XSTEP8 + n % 128 + 4 * g;
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        uint32_t hi, lo;
-        fp8_terms4(v[ni][q], pow2_biased(254 - s), hi, lo);
-        *reinterpret_cast<uint32_t*>(dst + 8 * q) = hi;
-        *reinterpret_cast<uint32_t*>(dst + 128 + 8 * q) = lo;
+        if constexpr (F::WIDE) {
+          uint32_t t[4];
+          fp8_terms4_wide(v[ni][q], pow2_biased(254 - s), t);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint32_t*>(dst + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128 + 8 * q) = t[e];
+        } else {
+          uint32_t hi, lo;
+          fp8_terms4(v[ni][q], pow2_biased(254 - s), hi, lo);
+          *reinterpret_cast<uint32_t*>(dst + 8 * q) = hi;
+          *reinterpret_cast<uint32_t*>(dst + 128 + 8 * q) = lo;
+        }
       }
-      if (wave % 2 == 0 && g == 0) a8s[at * 4 + n / 32] = (uint8_t)s;
+      if (wave % 2 == 0 && g == 0) {
+        a8s[at * 4 + n / 32] = (uint8_t)s;
+        if (F::WIDE) a8s[(at + (int64_t)a_rows * (I / 128)) * 4 + n / 32] = (uint8_t)(s - 8);
+      }
     }
   };
   stream_tiles<F>(tr, H / 128, lds, wave, lane, locate, setup, epilogue);
@@ -409,10 +433,11 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
                                             const Lists& L, const Table& routed, const Table& shared, int before,
-                                            uint16_t* __restrict__ out) {
+                                            int a_rows, void* __restrict__ out_rows) {
+  uint16_t* __restrict__ out = (uint16_t*)out_rows;
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = (H + F::TW - 1) / F::TW;
-  const TileRange tr = tile_range_after(active_row_tiles<F::BM>(L) * n_tiles, before, F::HOT_COST);
+  const TileRange tr = tile_range_after(active_row_tiles<F::ROWS>(L) * n_tiles, before, F::HOT_COST);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   auto locate = [&](int j, StreamTile<F>& t) { stream_locate<F>(L, tr.at(j), n_tiles, t); };
   auto setup = [&](StreamTile<F>& t) {
@@ -424,12 +449,25 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
       t.s0 = t.s1 = uniform_ptr(reinterpret_cast<const float*>(tw.w2s) +
                                 (int64_t)((col0 + 32 * wave % valid) / 128) * (I / 128));
     const int begin = t.begin, end = t.end;
-    t.ld.rows(a8, a8s, I, wave, lane, [&](int r) { return begin + r < end ? begin + r : begin; });
+    t.ld.rows(a8, a8s, I, wave, lane, [&](int r) {
+      const int q = begin + r % F::ROWS;
+      return (q < end ? q : begin) + (r < F::ROWS ? 0 : a_rows);
+    });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
     const int col = t.nt * F::TW + 32 * wave;
     if (col >= H) return;
-    if constexpr (F::BM == 16) {
+    if constexpr (F::WIDE) {  // fp32 rows
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc.q[q][i] += __shfl_xor(acc.q[q][i], 8, 64);
+      const int row = t.begin + lane % 16;
+      if (lane % 16 >= F::ROWS || row >= t.end) return;
+      float* dst = (float*)out_rows + (int64_t)row * H + col + lane / 16 * 4;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) *reinterpret_cast<v4f*>(dst + 16 * q) = acc.q[q];
+    } else if constexpr (F::BM == 16) {
       const int row = t.begin + lane % 16;
       if (row >= t.end) return;
       uint16_t* dst = out + (int64_t)row * H + col + lane / 16 * 4;
@@ -460,19 +498,19 @@ template <typename F, typename Table>
 __global__ void __launch_bounds__(64 * F::WAVES, 2) stream_gate_up_kernel(const uint8_t* __restrict__ x8,
                                                                           const uint8_t* __restrict__ x8s,
                                                                           const int32_t* __restrict__ row_token, Lists L,
-                                                                          Table routed, Table shared,
-                                                                          uint8_t* __restrict__ a8,
+                                                                          Table routed, Table shared, int x_rows,
+                                                                          int a_rows, uint8_t* __restrict__ a8,
                                                                           uint8_t* __restrict__ a8s) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[F::BYTES];
-  stream_gate_up<F>(lds, x8, x8s, row_token, L, routed, shared, 0, a8, a8s);
+  stream_gate_up<F>(lds, x8, x8s, row_token, L, routed, shared, 0, x_rows, a_rows, a8, a8s);
 }
 template <typename F, typename Table>
 __global__ void __launch_bounds__(64 * F::WAVES, 2) stream_down_kernel(const uint8_t* __restrict__ a8,
                                                                        const uint8_t* __restrict__ a8s, Lists L,
-                                                                       Table routed, Table shared,
-                                                                       uint16_t* __restrict__ out) {
+                                                                       Table routed, Table shared, int a_rows,
+                                                                       void* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[F::BYTES];
-  stream_down<F>(lds, a8, a8s, L, routed, shared, 0, out);
+  stream_down<F>(lds, a8, a8s, L, routed, shared, 0, a_rows, out);
 }
 
 // 128-row tiles of the experts with more than 64 rows (`hot`), then 64-row tiles of the others
@@ -494,7 +532,7 @@ __global__ void __launch_bounds__(512, 2) mixed_gate_up_kernel(const uint8_t* __
   gate_up_mx<F, F::DA, F::DB>(lds, x8, x8s, row_token, hot, routed, shared, a8, a8s);
   ring_wait_all();  // no load into the rings and no LDS access of the first part is left
   stream_gate_up<StreamOf<F>>(lds, x8, x8s, row_token, cold, routed, shared,
-                              active_row_tiles(hot) * ((routed.inter + F::TW / 2 - 1) / (F::TW / 2)), a8, (uint8_t*)a8s);
+                              active_row_tiles(hot) * ((routed.inter + F::TW / 2 - 1) / (F::TW / 2)), 0, 0, a8, (uint8_t*)a8s);
 }
 template <typename F, typename Table>
 __global__ void __launch_bounds__(512, 2) mixed_down_kernel(const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
@@ -504,7 +542,7 @@ __global__ void __launch_bounds__(512, 2) mixed_down_kernel(const uint8_t* __res
   down_mx<F, F::DA, F::DB>(lds, a8, a8s, hot, routed, shared, out);
   ring_wait_all();
   stream_down<StreamOf<F>>(lds, a8, a8s, cold, routed, shared, active_row_tiles(hot) * ((routed.hidden + F::TW - 1) / F::TW),
-                           out);
+                           0, out);
 }
 
 }  // namespace mf

@@ -1,5 +1,7 @@
 // C-ABI entry points of the MXFP4 MoE layer: argument checks, path choice
-// (fused dequant-GEMV for decode, MFMA grouped GEMM for prefill) and workspace sizing.
+// (fused dequant-GEMV for decode, its few-token grouped form once pairs pass enough weights, MFMA
+// grouped GEMM for prefill) and workspace sizing.
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -45,6 +47,13 @@ static bool use_decode(int tokens, int k) { return (int64_t)tokens * k <= DECODE
 // kernels do not take (above 16384).
 static bool use_decode(int tokens, int k, const wm_mxfp4_experts& e) {
   return !e.tiled && use_decode(tokens, k) && decode_mxfp4_supports(e.hidden, e.inter);
+}
+
+// Calls of the decode path that the few-token path takes over (the workspace of either fits both).
+static bool use_few(int tokens, int k, const wm_mxfp4_experts& e, const wm_mxfp4_experts* shared, const void* x,
+                    const void* y, const void* workspace) {
+  return few_mxfp4_takes(tokens, k, e) && few_mxfp4_aligned(&e) && few_mxfp4_aligned(shared) && (uintptr_t)x % 16 == 0 &&
+         (uintptr_t)y % 16 == 0 && (uintptr_t)workspace % 16 == 0;
 }
 
 static void validate_fp8(const wm_fp8_experts* e, const char* what, bool shared) {
@@ -122,8 +131,11 @@ extern "C" {
 
 WM_EXPORT size_t wm_moe_mxfp4_workspace_size(int32_t tokens, int32_t k, const wm_mxfp4_experts* experts) {
   if (!experts || tokens < 0 || k < 1) return 0;
-  if (use_decode(tokens, k, *experts)) return decode_workspace(tokens, k, *experts) + 256;
-  return prefill_workspace_size(tokens, k, *experts, true) + 256;
+  // no less than any smaller call's, so that a workspace made for the largest call serves all
+  const int few = std::min(tokens, DECODE_MAX_PAIRS / k);
+  const size_t least = few_mxfp4_takes(few, k, *experts) ? few_mxfp4_workspace_size(few, k, *experts) : 0;
+  if (use_decode(tokens, k, *experts)) return std::max(least, decode_workspace(tokens, k, *experts)) + 256;
+  return std::max(least, prefill_workspace_size(tokens, k, *experts, true)) + 256;
 }
 
 WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices, const float* weights, int32_t k,
@@ -138,7 +150,10 @@ WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices
     if (workspace_bytes < wm_moe_mxfp4_workspace_size(tokens, k, experts) - 256 || !workspace)
       fail("wm_moe_mxfp4: workspace too small");
     hipStream_t s = as_stream(stream);
-    if (use_decode(tokens, k, *experts))
+    if (use_few(tokens, k, *experts, shared, x, y, workspace))
+      few_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
+                (uint16_t*)y, true, workspace, s);
+    else if (use_decode(tokens, k, *experts))
       decode_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
                     (uint16_t*)y, true, (float*)workspace, s);
     else
@@ -165,6 +180,10 @@ WM_EXPORT int wm_moe_mxfp4_noalloc(const void* x, int32_t tokens, const int32_t*
       fail("wm_moe_mxfp4_noalloc: the call needs " + std::to_string(need) + " bytes of scratch, more than the " +
            std::to_string(kNoAllocScratchBytes) + " it has");
     void* ws = scratch_for_current_device();
+    // the few-token path where its buffers fit, as in wm_moe_mxfp4
+    if (use_few(tokens, k, *experts, shared, x, y, ws) && few_mxfp4_workspace_size(tokens, k, *experts) <= kNoAllocScratchBytes)
+      return few_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
+                       (uint16_t*)y, true, ws, as_stream(stream));
     decode_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
                  (uint16_t*)y, true, (float*)ws, as_stream(stream));
   });
@@ -182,7 +201,10 @@ WM_EXPORT int wm_experts_mxfp4(const void* x, int32_t tokens, const int32_t* ind
     if (workspace_bytes < wm_moe_mxfp4_workspace_size(tokens, k, experts) - 256 || !workspace)
       fail("wm_experts_mxfp4: workspace too small");
     hipStream_t s = as_stream(stream);
-    if (use_decode(tokens, k, *experts))
+    if (use_few(tokens, k, *experts, nullptr, x, out, workspace))
+      few_mxfp4((const uint16_t*)x, tokens, indices, nullptr, k, *experts, nullptr, nullptr, (uint16_t*)out, false,
+                workspace, s);
+    else if (use_decode(tokens, k, *experts))
       decode_mxfp4((const uint16_t*)x, tokens, indices, nullptr, k, *experts, nullptr, nullptr, (uint16_t*)out, false,
                    (float*)workspace, s);
     else

@@ -67,6 +67,15 @@ void prefill_mxfp4(const uint16_t* x, int tokens, const int32_t* indices, const 
                    const wm_mxfp4_experts& routed, const wm_mxfp4_experts* shared, const uint16_t* shared_gate,
                    uint16_t* y, bool combine, void* ws, size_t ws_bytes, hipStream_t s);
 
+// Few-token path: grouped tiles with the decode path's precision. takes: by sizes and layout (row
+// tables, T * K <= 256); aligned: whether a table's scales may be read as dwords.
+bool few_mxfp4_takes(int tokens, int k, const wm_mxfp4_experts& e);
+bool few_mxfp4_aligned(const wm_mxfp4_experts* e);
+size_t few_mxfp4_workspace_size(int tokens, int k, const wm_mxfp4_experts& e);
+void few_mxfp4(const uint16_t* x, int tokens, const int32_t* indices, const float* weights, int k,
+               const wm_mxfp4_experts& routed, const wm_mxfp4_experts* shared, const uint16_t* shared_gate, uint16_t* y,
+               bool combine, void* ws, hipStream_t s);
+
 // FP8 expert FFN (hidden and intermediate multiples of 128; up to 8192 for decode).
 void decode_fp8(const uint16_t* x, int tokens, const int32_t* indices, const float* weights, int k,
                 const wm_fp8_experts& routed, const wm_fp8_experts* shared, const uint16_t* shared_gate,
