@@ -6,9 +6,14 @@
 // a memory round trip each K step, and, in the row layout, half a 128-byte line of every
 // MXFP4 row a step. Here:
 //
-//   tile    : BM rows of one expert x TW = 32 WAVES weight rows; wave w owns the 32-row weight tile
-//             w: for gate_up 16 gate rows and the same 16 up rows, so that a lane holds both
-//             results of a column.
+//   tile    : BM rows of one expert x TW = 32 WAVES weight rows in 32-row weight tiles, for gate_up
+//             16 gate rows and the same 16 up rows, so that a lane holds both results of a column.
+//             With 16 rows wave w owns weight tile w; with 64, wave (wm, wn) = (w / 4, w % 4) owns the
+//             weight tiles 2 wn and 2 wn + 1 and the row tile of 32 rows wm, so that a step reads
+//             96 KB of LDS (MXFP4) where 32 weight rows x 64 rows a wave read 144, as many
+//             LDS cycles as MFMA ones (2048 tokens over 512 experts of 2560/640: gate_up 320 ->
+//             301 us, down 194 -> 186; 219 and 136 without the compute, 217 and 139 without the
+//             loads, so what is left is how far the two overlap).
 //   weights : a unit is 128 bytes of every row (two 128-wide K steps of MXFP4, one of FP8), eight
 //             whole lines of 8 rows a load, in either layout, with the non-temporal hint (a
 //             plain read of HBM: 7.0 against 5.9 TB/s).
@@ -33,14 +38,14 @@ struct StreamF {
   static constexpr bool WIDE = WIDE_;
   static constexpr int ROWS = WIDE_ ? 8 : BM_;  // rows of a tile
   static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
-  static constexpr int BM = BM_, WAVES = WAVES_, NI = 2, TW = 32 * WAVES_;  // NI: 32-row row tiles of 64 rows
+  static constexpr int BM = BM_, WAVES = WAVES_, MI = 2, TW = 32 * WAVES_;  // MI: a wave's weight tiles with 64 rows
   static constexpr int SUB = FP8_ ? 1 : 2;                 // K steps of a weight unit
   static constexpr int BSUB = BM_ == 16 ? SUB : 1;         // K steps of a split-row slot
   static constexpr int GRAN = SUB / BSUB;                  // split-row slots of a unit
   static constexpr int A_FMT = FP8_ ? FMT_FP8 : FMT_FP4;
   static constexpr int A_SLOT = TW * 128 + (A_SCALED_ ? TW * 4 * SUB : 0);
   static constexpr int B_TERMS = BM_ * XSTEP8 * BSUB, B_SLOT = B_TERMS + BM_ * 4 * BSUB;
-  static constexpr int RINGS = 3 * (A_SLOT + B_SLOT), BYTES = RINGS + WAVES_ * BM_ * 4;  // and block maxima
+  static constexpr int RINGS = 3 * (A_SLOT + B_SLOT), BYTES = RINGS + (BM_ == 16 ? WAVES_ * BM_ * 4 : 0);  // and block maxima
   static constexpr int NQA = 4, NQB = BM_ / 4 / WAVES_;    // 1 KB loads of a wave: a unit's, a K step's rows
   // about how many of its tiles take as long as one 128-row tile (twice the weight rows for MXFP4, and
   // bound by its MFMAs)
@@ -165,20 +170,20 @@ __device__ __forceinline__ void stream_locate(const Lists& L, int logical, int n
   resolve_tile_s<F::ROWS>(L, mt, t.expert, t.begin, t.end);
 }
 
-// A wave's results: 32-row weight tile x two 32-row row tiles (v_mfma_scale_f32_32x32x64), or with 16 rows
+// A wave's results: two 32-row weight tiles x a 32-row row tile (v_mfma_scale_f32_32x32x64), or with 16 rows
 // its two 16-row weight tiles (gate_up: the gate and the up rows) x 16 rows (16x16x128).
 template <typename F>
 struct StreamAcc {
-  v16f v[F::NI];
+  v16f v[F::MI];
   v4f q[2];
   __device__ __forceinline__ void clear() {
     if constexpr (F::BM == 16) {
       q[0] = q[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     } else {
 #pragma unroll
-      for (int ni = 0; ni < F::NI; ++ni)
+      for (int mi = 0; mi < F::MI; ++mi)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[ni][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) v[mi][i] = 0.0f;
     }
   }
 };
@@ -208,59 +213,69 @@ __device__ __forceinline__ void stream_step16(const uint8_t* wa, const uint8_t* 
   }
 }
 
-// acc += K step `sub` of a weight unit x a step of split rows.
+// acc += K step `sub` of a weight unit x a step of split rows; f0, f1: the fp32 block scales of result
+// registers 0..7 and 8..15. A half's fragment reads run under the other half's MFMAs.
 template <typename F>
-__device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb, int sub, int rows, int wave, int lane,
-                                            float f0, float f1, v16f (&acc)[F::NI]) {
+__device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb, int sub, int wm, int wn, int lane,
+                                            float f0, float f1, v16f (&acc)[F::MI]) {
   const int r = lane % 32, g = lane / 32;
-  const uint8_t* arow = wa + (32 * wave + r) * 128;
-  uint32_t sa = 127;
-  if constexpr (F::A_SCALED)
-    sa = *reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + (32 * wave + r) * 4 * F::SUB + 4 * sub);
-  v8i a[2];
+  const int row = 32 * wm + r;
+  const uint8_t* arow = wa + (64 * wn + r) * 128;
+  uint32_t sa[F::MI];
+#pragma unroll
+  for (int mi = 0; mi < F::MI; ++mi)
+    sa[mi] = F::A_SCALED ? *reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + (64 * wn + 32 * mi + r) * 4 * F::SUB + 4 * sub)
+                         : 127;
+  // where the loader put the row's scale dword
+  const uint32_t sw = *reinterpret_cast<const uint32_t*>(
+      rb + F::B_TERMS + 4 * (8 * (row / 4 % F::WAVES) + 4 * (row / (4 * F::WAVES)) + row % 4));
+  v8i a[2][F::MI], t[2][2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    auto piece = [&](int p) { return *reinterpret_cast<const uint4*>(arow + 16 * (p ^ (r % 8))); };
-    if constexpr (F::FP8) {
-      const uint4 u = piece(4 * h + g), v = piece(4 * h + 2 + g);
-      a[h] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
-    } else {
-      const uint4 u = piece(4 * sub + 2 * h + g);
-      a[h] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, 0, 0, 0, 0};
+#pragma unroll
+    for (int mi = 0; mi < F::MI; ++mi) {
+      auto piece = [&](int p) { return *reinterpret_cast<const uint4*>(arow + 4096 * mi + 16 * (p ^ (r % 8))); };
+      if constexpr (F::FP8) {
+        const uint4 u = piece(4 * h + g), v = piece(4 * h + 2 + g);
+        a[h][mi] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
+      } else {
+        const uint4 u = piece(4 * sub + 2 * h + g);
+        a[h][mi] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, 0, 0, 0, 0};
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const uint4 u = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + g));
+      const uint4 v = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + 2 + g));
+      t[h][e] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
     }
   }
+  v16f blk[F::BLOCK_F32 ? F::MI : 1];
+  if constexpr (F::BLOCK_F32) {
 #pragma unroll
-  for (int ni = 0; ni < F::NI; ++ni) {
-    if (32 * ni >= rows) break;  // no rows in this row tile (uniform)
-    const int row = 32 * ni + r;
-    // where the loader put the row's scale dword
-    const uint32_t sw = *reinterpret_cast<const uint32_t*>(
-        rb + F::B_TERMS + 4 * (8 * (row / 4 % F::WAVES) + 4 * (row / (4 * F::WAVES)) + row % 4));
-    v16f blk;
-    if constexpr (F::BLOCK_F32) {
+    for (int mi = 0; mi < F::MI; ++mi)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) blk[i] = 0.0f;
-    }
-    v16f& sum = F::BLOCK_F32 ? blk : acc[ni];
+      for (int i = 0; i < 16; ++i) blk[mi][i] = 0.0f;
+  }
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int sh = 8 * g + 16 * h;
-      v8i t[2];
+  for (int h = 0; h < 2; ++h) {
+    const int sh = 8 * g + 16 * h;
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const uint4 u = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + g));
-        const uint4 v = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + 2 + g));
-        t[e] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int mi = 0; mi < F::MI; ++mi) {
+        v16f& sum = F::BLOCK_F32 ? blk[F::BLOCK_F32 ? mi : 0] : acc[mi];
+        // lo scales: hi - 4 (every hi scale byte is >= 5)
+        sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[h][mi], t[h][e], sum, F::A_FMT, FMT_FP8, 0,
+                                                              F::A_SCALED ? (int)(sa[mi] >> sh) : 127, 0,
+                                                              (int)((sw - (e ? 0x04040404u : 0u)) >> sh));
       }
-      const int ws = F::A_SCALED ? (int)(sa >> sh) : 127;
-      sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[h], t[0], sum, F::A_FMT, FMT_FP8, 0, ws, 0, (int)(sw >> sh));
-      sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[h], t[1], sum, F::A_FMT, FMT_FP8, 0, ws, 0,
-                                                            (int)((sw - 0x04040404u) >> sh));
-    }
-    if constexpr (F::BLOCK_F32) {  // the fp32 block scale cannot ride on the MFMA's E8M0 scales
+  }
+  if constexpr (F::BLOCK_F32) {  // the fp32 block scale cannot ride on the MFMA's E8M0 scales
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[ni][i] = fmaf(i < 8 ? f0 : f1, blk[i], acc[ni][i]);
-    }
+    for (int mi = 0; mi < F::MI; ++mi)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mi][i] = fmaf(i < 8 ? f0 : f1, blk[mi][i], acc[mi][i]);
   }
 }
 
@@ -322,9 +337,11 @@ __device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uin
         if constexpr (F::BM == 16) {
           stream_step16<F>(wslot(gu), rslot(g), h, wave, lane, acc.q);
         } else {
+          const int wm = wave / 4, wn = wave % 4;
+          if (32 * wm >= cur.end - cur.begin) continue;  // no rows in this row tile (uniform)
           float f0 = 1.0f, f1 = 1.0f;
           if constexpr (F::BLOCK_F32) f0 = cur.s0[ks], f1 = cur.s1[ks];
-          stream_step<F>(wslot(gu), rslot(g), sub, cur.end - cur.begin, wave, lane, f0, f1, acc.v);
+          stream_step<F>(wslot(gu), rslot(g), sub, wm, wn, lane, f0, f1, acc.v);
         }
       }
       if (sub == F::GRAN - 1) ++gu;
@@ -335,15 +352,16 @@ __device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uin
   }
 }
 
-// act rows of TW / 2 intermediate columns; wave w owns 16 of them: result lane (r, g) register i < 8
-// is the gate and i + 8 the up product of column 8 (i / 4) + 4 g + i % 4 for row r of a row
-// tile. Waves 2 p and 2 p + 1 share a 32-value block of the act row.
+// act rows of TW / 2 intermediate columns, 16 a weight tile: result lane (r, g) register i < 8 is the
+// gate and i + 8 the up product of column 8 (i / 4) + 4 g + i % 4 for row r of the row tile.
+// Weight tiles 2 p and 2 p + 1 share a 32-value block of the act row: a wave's own two, or with 16 rows
+// those of two waves.
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
                                                const int32_t* __restrict__ row_token, const Lists& L, const Table& routed,
                                                const Table& shared, int before, int x_rows, int a_rows,
                                                uint8_t* __restrict__ a8, uint8_t* __restrict__ a8s) {
-  float(*block_max)[F::BM] = reinterpret_cast<float(*)[F::BM]>(lds + F::RINGS);
+  float(*block_max)[F::BM] = reinterpret_cast<float(*)[F::BM]>(lds + F::RINGS);  // 16 rows
   constexpr int TG = F::TW / 2;
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = I / TG;  // I is a multiple of 128
@@ -367,69 +385,92 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
-    // Lane (r, g) holds row r of row tile ni, values [q][i] of the wave's columns 4 g + 8 q + i.
-    constexpr int ROWS = F::BM == 16 ? 16 : 32, NI = F::BM / ROWS, Q = F::BM == 16 ? 1 : 2;
-    const int r = lane % ROWS, g = lane / ROWS;
     const int rows = t.end - t.begin;
-    float v[NI][Q][4], amax[NI];
+    auto act = [&](float gv, float uv) {
+      if (t.limit > 0.0f) {
+        gv = fminf(gv, t.limit);
+        uv = fminf(fmaxf(uv, -t.limit), t.limit);
+      }
+      return silu(gv) * uv;
+    };
+    if constexpr (F::BM == 16) {
+      const int row = lane % 16, g = lane / 16;
+      float v[4], amax = 0.0f;
 #pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      amax[ni] = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4 * Q; ++i) {
-        float gv, uv;
-        if constexpr (F::BM == 16) gv = acc.q[0][i], uv = acc.q[1][i];
-        else gv = acc.v[ni][i], uv = acc.v[ni][i + 8];
+      for (int i = 0; i < 4; ++i) {
+        float gv = acc.q[0][i], uv = acc.q[1][i];
         if constexpr (F::WIDE) {  // the upper terms' products, in the lane of row r +- 8
           gv += __shfl_xor(gv, 8, 64);
           uv += __shfl_xor(uv, 8, 64);
         }
-        if (t.limit > 0.0f) {
-          gv = fminf(gv, t.limit);
-          uv = fminf(fmaxf(uv, -t.limit), t.limit);
-        }
-        v[ni][i / 4][i % 4] = silu(gv) * uv;
-        amax[ni] = fmaxf(amax[ni], fabsf(v[ni][i / 4][i % 4]));
+        v[i] = act(gv, uv);
+        amax = fmaxf(amax, fabsf(v[i]));
       }
-      if (F::BM == 16) amax[ni] = fmaxf(amax[ni], __shfl_xor(amax[ni], 16, 64));
-      amax[ni] = fmaxf(amax[ni], __shfl_xor(amax[ni], 32, 64));
-      if (g == 0) block_max[wave][ROWS * ni + r] = amax[ni];
-    }
-    stage_barrier();
-#pragma unroll
-    for (int ni = 0; ni < NI; ++ni) {
-      const int row = ROWS * ni + r;
-      if (row >= rows) continue;
-      const float block = fmaxf(amax[ni], block_max[wave ^ 1][row]);
+      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      if (g == 0) block_max[wave][row] = amax;
+      stage_barrier();
+      if (row >= rows) return;
+      const float block = fmaxf(amax, block_max[wave ^ 1][row]);
       const int s = F::WIDE ? fp8_term_exponent_wide(block) : fp8_term_exponent(block);
       const int n = t.nt * TG + 16 * wave;  // the wave's first column
       const int64_t at = (int64_t)(t.begin + row) * (I / 128);
       uint8_t* dst = a8 + (at + n / 128) * XSTEP8 + n % 128 + 4 * g;
+      if constexpr (F::WIDE) {
+        uint32_t w[4];
+        fp8_terms4_wide(v, pow2_biased(254 - s), w);
 #pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        if constexpr (F::WIDE) {
-          uint32_t t[4];
-          fp8_terms4_wide(v[ni][q], pow2_biased(254 - s), t);
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            *reinterpret_cast<uint32_t*>(dst + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128 + 8 * q) = t[e];
-        } else {
-          uint32_t hi, lo;
-          fp8_terms4(v[ni][q], pow2_biased(254 - s), hi, lo);
-          *reinterpret_cast<uint32_t*>(dst + 8 * q) = hi;
-          *reinterpret_cast<uint32_t*>(dst + 128 + 8 * q) = lo;
-        }
+        for (int e = 0; e < 4; ++e)
+          *reinterpret_cast<uint32_t*>(dst + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128) = w[e];
+      } else {
+        uint32_t hi, lo;
+        fp8_terms4(v, pow2_biased(254 - s), hi, lo);
+        *reinterpret_cast<uint32_t*>(dst) = hi;
+        *reinterpret_cast<uint32_t*>(dst + 128) = lo;
       }
       if (wave % 2 == 0 && g == 0) {
         a8s[at * 4 + n / 32] = (uint8_t)s;
         if (F::WIDE) a8s[(at + (int64_t)a_rows * (I / 128)) * 4 + n / 32] = (uint8_t)(s - 8);
       }
+    } else {
+      const int wm = wave / 4, wn = wave % 4, g = lane / 32, row = 32 * wm + lane % 32;
+      if (32 * wm >= rows) return;  // uniform
+      float v[F::MI][2][4], amax = 0.0f;
+#pragma unroll
+      for (int mi = 0; mi < F::MI; ++mi)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          v[mi][i / 4][i % 4] = act(acc.v[mi][i], acc.v[mi][i + 8]);
+          amax = fmaxf(amax, fabsf(v[mi][i / 4][i % 4]));
+        }
+      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      const int s = fp8_term_exponent(amax);
+      // words [term][8-column group 2 mi + q] of columns 4 g .. + 3 of the group; two swaps between the lane
+      // halves (groups of a tile, then tiles) leave each lane the 16 columns of weight tile g
+      uint32_t w[2][4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) fp8_terms4(v[c / 2][c % 2], pow2_biased(254 - s), w[0][c], w[1][c]);
+      const int n = t.nt * TG + 32 * wn;  // the wave's first column
+      const int64_t at = (int64_t)(t.begin + row) * (I / 128);
+      uint8_t* dst = a8 + (at + n / 128) * XSTEP8 + n % 128 + 16 * g;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        uint32_t o[4];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {  // group q of tile 0 and of tile 1
+          const auto pr = __builtin_amdgcn_permlane32_swap(w[e][q], w[e][2 + q], false, false);
+          o[2 * q] = pr[0];
+          o[2 * q + 1] = pr[1];
+        }
+        if (row < rows) *reinterpret_cast<uint4*>(dst + 128 * e) = make_uint4(o[0], o[1], o[2], o[3]);
+      }
+      if (row < rows && g == 0) a8s[at * 4 + n / 32] = (uint8_t)s;
     }
   };
   stream_tiles<F>(tr, H / 128, lds, wave, lane, locate, setup, epilogue);
 }
 
-// Output rows (bf16, permuted order) of TW columns; wave w owns columns 32 w .. + 31.
+// Output rows (bf16, permuted order) of TW columns, 32 a weight tile.
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
                                             const Lists& L, const Table& routed, const Table& shared, int before,
@@ -447,7 +488,7 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
     t.ld.weights(tw.w2, tw.w2s, H, I, table_tiled(routed), wave, lane, [=](int j) { return col0 + j % valid; });
     if constexpr (F::BLOCK_F32)
       t.s0 = t.s1 = uniform_ptr(reinterpret_cast<const float*>(tw.w2s) +
-                                (int64_t)((col0 + 32 * wave % valid) / 128) * (I / 128));
+                                (int64_t)((col0 + 64 * (wave % 4) % valid) / 128) * (I / 128));
     const int begin = t.begin, end = t.end;
     t.ld.rows(a8, a8s, I, wave, lane, [&](int r) {
       const int q = begin + r % F::ROWS;
@@ -455,7 +496,7 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
-    const int col = t.nt * F::TW + 32 * wave;
+    const int col = t.nt * F::TW + (F::BM == 16 ? 32 * wave : 64 * (wave % 4));
     if (col >= H) return;
     if constexpr (F::WIDE) {  // fp32 rows
 #pragma unroll
@@ -476,18 +517,26 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
         *reinterpret_cast<uint2*>(dst + 16 * q) =
             make_uint2(pack_bf16x2(acc.q[q][0], acc.q[q][1]), pack_bf16x2(acc.q[q][2], acc.q[q][3]));
     } else {
-      const int r = lane % 32, g = lane / 32;
+      const int g = lane / 32, row = t.begin + 32 * (wave / 4) + lane % 32;
+      if (t.begin + 32 * (wave / 4) >= t.end) return;  // uniform
+      // a swap between the lane halves gives each lane 8 columns in a row: stores of 16 bytes
 #pragma unroll
-      for (int ni = 0; ni < F::NI; ++ni) {
-        const int row = t.begin + 32 * ni + r;
-        if (row >= t.end) continue;
-        const v16f& a = acc.v[ni];
-        uint16_t* dst = out + (int64_t)row * H + col + 4 * g;
+      for (int mi = 0; mi < F::MI; ++mi)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<uint2*>(dst + 8 * q) =
-              make_uint2(pack_bf16x2(a[4 * q], a[4 * q + 1]), pack_bf16x2(a[4 * q + 2], a[4 * q + 3]));
-      }
+        for (int p = 0; p < 2; ++p) {
+          const v16f& a = acc.v[mi];
+          uint32_t o[4];
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const auto pr = __builtin_amdgcn_permlane32_swap(pack_bf16x2(a[8 * p + 2 * q], a[8 * p + 2 * q + 1]),
+                                                             pack_bf16x2(a[8 * p + 4 + 2 * q], a[8 * p + 4 + 2 * q + 1]),
+                                                             false, false);
+            o[q] = pr[0];
+            o[2 + q] = pr[1];
+          }
+          if (row < t.end)
+            *reinterpret_cast<uint4*>(out + (int64_t)row * H + col + 32 * mi + 16 * p + 8 * g) = make_uint4(o[0], o[1], o[2], o[3]);
+        }
     }
   };
   stream_tiles<F>(tr, I / 128, lds, wave, lane, locate, setup, epilogue);
