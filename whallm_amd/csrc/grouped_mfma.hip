@@ -31,6 +31,7 @@
 
 #include "lds_dma.h"
 #include "moe_internal.h"
+#include "permute_device.h"
 
 namespace wm {
 namespace mf {
@@ -44,7 +45,6 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 struct Lists {
-  const int32_t* order;       // [P] pair of each permuted row
   const int32_t* offsets;     // [E + 1]
   const int32_t* tiles;       // [n][2] (expert, first row)
   const int32_t* tile_count;  // [1]
@@ -219,11 +219,11 @@ __device__ __forceinline__ void fp6_terms32(const float (&v)[32], v6u_t& hi, v6u
 // With g (bf16 [H]) the kernel also writes gate[row] = sigmoid(x[row] . g), the shared
 // expert's gate: a row's H/32 lanes are contiguous and aligned (H/32 a power of two <= 64),
 // so their partial dots meet in a butterfly inside the group.
-__global__ void __launch_bounds__(256) split6_rows_kernel(const uint16_t* __restrict__ x, int rows, int hidden,
-                                                          uint8_t* __restrict__ x6, const uint16_t* __restrict__ g,
-                                                          float* __restrict__ gate) {
+__device__ __forceinline__ void split6_rows(int64_t block, const uint16_t* __restrict__ x, int rows, int hidden,
+                                            uint8_t* __restrict__ x6, const uint16_t* __restrict__ g,
+                                            float* __restrict__ gate) {
   const int blocks = hidden / 32;
-  const int64_t job = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (row, block)
+  const int64_t job = block * 256 + threadIdx.x;  // (row, block)
   if (job >= (int64_t)rows * blocks) return;
   const int64_t row = job / blocks;
   const int blk = (int)(job % blocks);
@@ -358,12 +358,12 @@ __device__ __forceinline__ void fp8_terms32(const float (&v)[32], uint32_t (&hi)
 
 // x [rows, H] bf16 -> E4M3 split rows: terms [rows][H/128][256 bytes], scales
 // [rows][H/128] dwords. One lane per 32-value block. With g (bf16 [H]) also gate[row] =
-// sigmoid(x[row] . g) as in split6_rows_kernel.
-__global__ void __launch_bounds__(256) split8_rows_kernel(const uint16_t* __restrict__ x, int rows, int hidden,
-                                                          uint8_t* __restrict__ x8, uint32_t* __restrict__ x8s,
-                                                          const uint16_t* __restrict__ g, float* __restrict__ gate) {
+// sigmoid(x[row] . g) as in split6_rows.
+__device__ __forceinline__ void split8_rows(int64_t block, const uint16_t* __restrict__ x, int rows, int hidden,
+                                            uint8_t* __restrict__ x8, uint32_t* __restrict__ x8s,
+                                            const uint16_t* __restrict__ g, float* __restrict__ gate) {
   const int blocks = hidden / 32;
-  const int64_t job = (int64_t)blockIdx.x * 256 + threadIdx.x;  // (row, block)
+  const int64_t job = block * 256 + threadIdx.x;  // (row, block)
   if (job >= (int64_t)rows * blocks) return;
   const int64_t row = job / blocks;
   const int blk = (int)(job % blocks);
@@ -1371,18 +1371,20 @@ __global__ void __launch_bounds__(64 * F::WAVES, F::WAVES / 4)
 namespace wm {
 namespace mf {
 
-// Token of every permuted row: order[p] / K for routed rows, p - P for the shared rows.
-__global__ void __launch_bounds__(256) row_tokens_kernel(const int32_t* __restrict__ order, int pairs, int k,
-                                                         int rows, int32_t* __restrict__ row_token) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p < rows) row_token[p] = p < pairs ? order[p] / k : p - pairs;
+__global__ void __launch_bounds__(256) split6_rows_kernel(const uint16_t* __restrict__ x, int rows, int hidden,
+                                                          uint8_t* __restrict__ x6) {
+  split6_rows(blockIdx.x, x, rows, hidden, x6, nullptr, nullptr);
+}
+__global__ void __launch_bounds__(256) split8_rows_kernel(const uint16_t* __restrict__ x, int rows, int hidden,
+                                                          uint8_t* __restrict__ x8, uint32_t* __restrict__ x8s) {
+  split8_rows(blockIdx.x, x, rows, hidden, x8, x8s, nullptr, nullptr);
 }
 
 // ---------------------------------------------------------------------------------
-// gate[t] = sigmoid(x[t] . g) (1 when g is null); one wave per token.
-__global__ void __launch_bounds__(64) shared_gate_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ g,
-                                                         int tokens, int hidden, float* __restrict__ gate) {
-  const int t = blockIdx.x, lane = threadIdx.x;
+// gate[t] = sigmoid(x[t] . g) (1 when g is null); one wave per token, four a block.
+__device__ __forceinline__ void shared_gates(int block, const uint16_t* __restrict__ x, const uint16_t* __restrict__ g,
+                                             int tokens, int hidden, float* __restrict__ gate) {
+  const int t = block * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
   if (t >= tokens) return;
   float v = 1.0f;
   if (g) {
@@ -1394,6 +1396,40 @@ __global__ void __launch_bounds__(64) shared_gate_kernel(const uint16_t* __restr
     v = 1.0f / (1.0f + __expf(-a));
   }
   if (lane == 0) gate[t] = v;
+}
+
+// What a prefill call does before its lists are scanned, in one launch: the permute's counts, the
+// split of x (with the gate where a row's blocks fit a wave, else in blocks of its own) and
+// the shared rows' tokens. With the scan and the scatter a call has 3 small launches where it had 6 or 7
+// (301 tokens over 512 experts: the whole block 225.3 -> 220.6 us; 2048 tokens 527.5 -> 522.1).
+struct PrepArgs {
+  const int32_t* indices;
+  int64_t pairs;
+  int experts, tokens, hidden;
+  int64_t count_blocks, split_blocks;
+  int32_t *counts, *done;
+  const uint16_t *x, *split_gate, *block_gate;  // the shared gate's vector, by the split or by the gate blocks
+  uint8_t* terms;
+  uint32_t* scales;
+  float* gate;
+  int32_t* shared_rows;  // null without a shared expert
+};
+template <bool E4>
+__global__ void __launch_bounds__(256) prefill_prep_kernel(PrepArgs a) {
+  int64_t b = blockIdx.x;
+  if (b < a.count_blocks) {
+    permute_count_block(a.indices, a.pairs, a.experts, b, a.counts, a.done);
+    return;
+  }
+  b -= a.count_blocks;
+  if (b < a.split_blocks) {
+    const int64_t t = b * 256 + threadIdx.x;
+    if (a.shared_rows && t < a.tokens) a.shared_rows[t] = (int32_t)t;  // tokens <= split lanes
+    if constexpr (E4) split8_rows(b, a.x, a.tokens, a.hidden, a.terms, a.scales, a.split_gate, a.gate);
+    else split6_rows(b, a.x, a.tokens, a.hidden, a.terms, a.split_gate, a.gate);
+    return;
+  }
+  shared_gates((int)(b - a.split_blocks), a.x, a.block_gate, a.tokens, a.hidden, a.gate);
 }
 
 // Whether pair p's expert is resident: its slot map entry (when the table has one) is
@@ -1555,7 +1591,7 @@ static int compute_units() {
 }
 
 struct Layout {
-  size_t permute_ws, order, inverse, offsets, tiles, tile_count, gate, row_token, x6, x6s, a6, a6s, rows, total;
+  size_t permute_ws, inverse, offsets, tiles, tile_count, gate, row_token, x6, x6s, a6, a6s, rows, total;
   int64_t max_tiles;
 };
 
@@ -1569,7 +1605,6 @@ static Layout layout(int tokens, int k, int experts, int hidden, int inter, bool
   Layout p{};
   size_t at = 0;
   p.permute_ws = at; at += align256(wm_permute_workspace_size(pairs, experts));
-  p.order = at;      at += align256(sizeof(int32_t) * (size_t)(pairs > 0 ? pairs : 1));
   p.inverse = at;    at += align256(sizeof(int32_t) * (size_t)(pairs > 0 ? pairs : 1));
   p.offsets = at;    at += align256(sizeof(int32_t) * (size_t)(experts + 1));
   p.tiles = at;      at += align256(sizeof(int32_t) * 2 * (size_t)(max_tiles + experts));
@@ -1641,7 +1676,6 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
     fail("prefill: split operands of 4 GiB or more (split the call into smaller token batches)");
   uint8_t* base = (uint8_t*)ws;
   Lists L;
-  L.order = (int32_t*)(base + p.order);
   L.offsets = (int32_t*)(base + p.offsets);
   L.tiles = (int32_t*)(base + p.tiles);
   L.tile_count = (int32_t*)(base + p.tile_count);
@@ -1662,32 +1696,36 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
     L.has_shared = has_shared && tokens > COLD_ROWS;
     cold.has_shared = has_shared && tokens <= COLD_ROWS;
   }
-  permute_tiles(indices, pairs, routed.experts, bm, how == ROWS_MIXED ? COLD_ROWS : 0, (int32_t*)L.order, inverse,
-                (int32_t*)L.offsets, (int32_t*)L.tiles, (int32_t*)cold.tiles, (int32_t*)L.tile_count, base + p.permute_ws, s);
-  // the split kernel computes the shared gate when a row's blocks fit one wave in a
-  // power-of-two group; otherwise a kernel of its own does
+  // the split computes the shared gate when a row's blocks fit one wave in a power-of-two
+  // group; otherwise blocks of their own do
   const bool fused_gate = has_shared && shared_gate && (H / 32) <= 64 && ((H / 32) & (H / 32 - 1)) == 0;
-  if (has_shared && !fused_gate) {
-    hipLaunchKernelGGL(shared_gate_kernel, dim3(tokens), dim3(64), 0, s, x, shared_gate, tokens, H,
-                       (float*)L.shared_gate);
-    check_launch("shared_gate");
-  }
   uint8_t* x6 = base + p.x6;
-  int32_t* row_token = (int32_t*)(base + p.row_token);
-  if (rows > 0) {
-    hipLaunchKernelGGL(row_tokens_kernel, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, s, L.order, (int)pairs,
-                       k, (int)rows, row_token);
-    check_launch("row_tokens");
-  }
   uint8_t* x6s = base + p.x6s;
-  const int64_t split_jobs = (int64_t)tokens * (H / 32);
-  if constexpr (F::Terms::E4)
-    hipLaunchKernelGGL(split8_rows_kernel, dim3((unsigned)((split_jobs + 255) / 256)), dim3(256), 0, s, x, tokens, H,
-                       x6, (uint32_t*)x6s, fused_gate ? shared_gate : nullptr, (float*)L.shared_gate);
-  else
-    hipLaunchKernelGGL(split6_rows_kernel, dim3((unsigned)((split_jobs + 255) / 256)), dim3(256), 0, s, x, tokens, H,
-                       x6, fused_gate ? shared_gate : nullptr, (float*)L.shared_gate);
-  check_launch("split_rows");
+  int32_t* row_token = (int32_t*)(base + p.row_token);
+  const PermuteWorkspace pw = permute_workspace(base + p.permute_ws, pairs, routed.experts);
+  PrepArgs pa{};
+  pa.indices = indices;
+  pa.pairs = pairs;
+  pa.experts = routed.experts;
+  pa.tokens = tokens;
+  pa.hidden = H;
+  pa.count_blocks = permute_count_blocks(pairs);
+  pa.split_blocks = ((int64_t)tokens * (H / 32) + 255) / 256;
+  pa.counts = pw.counts;
+  pa.done = pw.done;
+  pa.x = x;
+  pa.split_gate = fused_gate ? shared_gate : nullptr;
+  pa.block_gate = shared_gate;
+  pa.terms = x6;
+  pa.scales = (uint32_t*)x6s;
+  pa.gate = (float*)L.shared_gate;
+  pa.shared_rows = has_shared ? row_token + pairs : nullptr;
+  const int64_t gate_blocks = has_shared && !fused_gate ? (tokens + 3) / 4 : 0;
+  hipLaunchKernelGGL((prefill_prep_kernel<F::Terms::E4>), dim3((unsigned)(pa.count_blocks + pa.split_blocks + gate_blocks)),
+                     dim3(256), 0, s, pa);
+  check_launch("prefill_prep");
+  permute_lists(indices, pairs, routed.experts, bm, how == ROWS_MIXED ? COLD_ROWS : 0, nullptr, inverse, row_token, k,
+                (int32_t*)L.offsets, (int32_t*)L.tiles, (int32_t*)cold.tiles, (int32_t*)L.tile_count, pw, s);
   const Table sh = shared ? *shared : routed;
   const int64_t max_row_tiles = (pairs + bm - 1) / bm + routed.experts + (has_shared ? (tokens + bm - 1) / bm : 0);
   // Persistent launches: as many workgroups per CU as the LDS rings allow, a multiple of the 8
@@ -1817,18 +1855,7 @@ __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restric
     return;
   }
   if ((int)blockIdx.x > split_blocks) {
-    const int t = ((int)blockIdx.x - 1 - split_blocks) * 4 + threadIdx.x / 64, lane = threadIdx.x % 64;
-    if (t >= tokens) return;
-    float v = 1.0f;
-    if (g) {
-      const uint32_t* xr = reinterpret_cast<const uint32_t*>(x) + (int64_t)t * (hidden / 2);
-      const uint32_t* gr = reinterpret_cast<const uint32_t*>(g);
-      float a = 0.0f;
-      for (int q = lane; q < hidden / 2; q += 64) a = dot2_bf16(bits_to_bf16x2(xr[q]), bits_to_bf16x2(gr[q]), a);
-      a = segment_sum<64>(a);
-      v = 1.0f / (1.0f + __expf(-a));
-    }
-    if (lane == 0) gate[t] = v;
+    shared_gates((int)blockIdx.x - 1 - split_blocks, x, g, tokens, hidden, gate);
     return;
   }
   const int blocks = hidden / 32;
@@ -2088,8 +2115,7 @@ WM_EXPORT int wm_split_rows_e2m3(const void* x, int32_t rows, int32_t hidden, vo
     if ((uintptr_t)x % 16 || (uintptr_t)out % 16) wm::fail("wm_split_rows_e2m3: x and out must be 16-byte aligned");
     const int64_t jobs = (int64_t)rows * (hidden / 32);
     hipLaunchKernelGGL(wm::mf::split6_rows_kernel, dim3((unsigned)((jobs + 255) / 256)), dim3(256), 0,
-                       wm::as_stream(stream), (const uint16_t*)x, (int)rows, (int)hidden, (uint8_t*)out, nullptr,
-                       nullptr);
+                       wm::as_stream(stream), (const uint16_t*)x, (int)rows, (int)hidden, (uint8_t*)out);
     wm::check_launch("split_rows_e2m3");
   });
 }
@@ -2104,7 +2130,7 @@ WM_EXPORT int wm_split_rows_e4m3(const void* x, int32_t rows, int32_t hidden, vo
     const int64_t jobs = (int64_t)rows * (hidden / 32);
     hipLaunchKernelGGL(wm::mf::split8_rows_kernel, dim3((unsigned)((jobs + 255) / 256)), dim3(256), 0,
                        wm::as_stream(stream), (const uint16_t*)x, (int)rows, (int)hidden, (uint8_t*)terms,
-                       (uint32_t*)scales, nullptr, nullptr);
+                       (uint32_t*)scales);
     wm::check_launch("split_rows_e4m3");
   });
 }

@@ -88,12 +88,17 @@ void prefill_fp8(const uint16_t* x, int tokens, const int32_t* indices, const fl
 // The one-launch decode layer (decode_layer.hip): shapes with a fused instantiation.
 bool moe_layer_fused_supports(int hidden, int inter, int k);
 
-// wm_permute on checked arguments. With cold_rows > 0 the experts of up to that many rows (and more
-// than none) are left out of `tiles` and get one tile each in cold_tiles [experts][2], counted in
-// tile_count[1].
-void permute_tiles(const int32_t* indices, int64_t pairs, int experts, int tile_rows, int cold_rows, int32_t* order,
-                   int32_t* inverse, int32_t* offsets, int32_t* tiles, int32_t* cold_tiles, int32_t* tile_count,
-                   void* workspace, hipStream_t s);
+// wm_permute on checked arguments, after permute_count_block's launch (permute_device.h). With
+// cold_rows > 0 the experts of up to that many rows (and more than none) are left out of `tiles` and get
+// one tile each in cold_tiles [experts][2], counted in tile_count[1]. order may be null; row_token (or
+// null): pair / k of every permuted row.
+struct PermuteWorkspace {
+  int32_t *counts, *totals, *done;
+};
+PermuteWorkspace permute_workspace(void* workspace, int64_t pairs, int experts);
+void permute_lists(const int32_t* indices, int64_t pairs, int experts, int tile_rows, int cold_rows, int32_t* order,
+                   int32_t* inverse, int32_t* row_token, int k, int32_t* offsets, int32_t* tiles, int32_t* cold_tiles,
+                   int32_t* tile_count, const PermuteWorkspace& ws, hipStream_t s);
 
 // Pairs at or below this count take the decode path.
 constexpr int DECODE_MAX_PAIRS = 256;
