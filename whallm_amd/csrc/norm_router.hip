@@ -267,13 +267,16 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const float* __restr
   ss = segment_sum<64>(ss);
   if (lane == 0) part[0][wave] = ss;
   __syncthreads();
-  const float inv = rsqrtf(((part[0][0] + part[0][1]) + (part[0][2] + part[0][3])) / (float)hidden + eps);
+  // In 64 bits up to x's rounding: memory bounds the kernel, and a row's values share the error of `inv`, which
+  // moves them over bf16 rounding boundaries together: 4 x 4000 rows of 2560, 93 values off by a bf16 step, 334 in 32 bits.
+  const double inv =
+      1.0 / sqrt((((double)part[0][0] + part[0][1]) + ((double)part[0][2] + part[0][3])) / hidden + (double)eps);
   float dot = 0.0f;
 #pragma unroll
   for (int j = 0; j < Q; ++j) {
     const int q = threadIdx.x + 256 * j;
     if (q >= quads) continue;
-    float f[4] = {v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv};
+    double f[4] = {v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv};
     if (nw) {
       const uint2 n = ((const uint2*)nw)[q];
       f[0] *= bf16_bits_to_f32(n.x & 0xffffu);
@@ -281,8 +284,9 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const float* __restr
       f[2] *= bf16_bits_to_f32(n.y & 0xffffu);
       f[3] *= bf16_bits_to_f32(n.y >> 16);
     }
-    const uint2 xv = make_uint2((uint32_t)f32_to_bf16_bits(f[0]) | ((uint32_t)f32_to_bf16_bits(f[1]) << 16),
-                                (uint32_t)f32_to_bf16_bits(f[2]) | ((uint32_t)f32_to_bf16_bits(f[3]) << 16));
+    const uint2 xv =
+        make_uint2((uint32_t)f32_to_bf16_bits((float)f[0]) | ((uint32_t)f32_to_bf16_bits((float)f[1]) << 16),
+                   (uint32_t)f32_to_bf16_bits((float)f[2]) | ((uint32_t)f32_to_bf16_bits((float)f[3]) << 16));
     ((uint2*)(x_out + row))[q] = xv;
     if (r_out) ((float4*)(r_out + row))[q] = v[j];
     if (gate) {
