@@ -38,7 +38,8 @@ struct StreamF {
   static constexpr bool WIDE = WIDE_;
   static constexpr int ROWS = WIDE_ ? 8 : BM_;  // rows of a tile
   static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
-  static constexpr int BM = BM_, WAVES = WAVES_, MI = 2, TW = 32 * WAVES_;  // MI: a wave's weight tiles with 64 rows
+  static constexpr int BM = BM_, WAVES = WAVES_, TW = 32 * WAVES_;
+  static constexpr int MI = BM_ == 16 ? 1 : 2;             // a wave's weight tiles
   static constexpr int SUB = FP8_ ? 1 : 2;                 // K steps of a weight unit
   static constexpr int BSUB = BM_ == 16 ? SUB : 1;         // K steps of a split-row slot
   static constexpr int GRAN = SUB / BSUB;                  // split-row slots of a unit
@@ -170,25 +171,25 @@ __device__ __forceinline__ void stream_locate(const Lists& L, int logical, int n
   resolve_tile_s<F::ROWS>(L, mt, t.expert, t.begin, t.end);
 }
 
-// A wave's results: two 32-row weight tiles x a 32-row row tile (v_mfma_scale_f32_32x32x64), or with 16 rows
-// its two 16-row weight tiles (gate_up: the gate and the up rows) x 16 rows (16x16x128).
+// A wave's results: MI weight tiles of 32 rows x a row tile of 32 columns (v_mfma_scale_f32_32x32x64 in the
+// order of the 128-row tiles, so that a row's results do not depend on the tile that held it: with 16
+// rows half the columns go unused, 2.5% of a call of 64 tokens of 5120/2304 over 16x16x128, whose sums of
+// 128 products round otherwise). WIDE: its two 16-row weight tiles (gate_up: the gate and the up rows) x 16
+// columns (16x16x128).
 template <typename F>
 struct StreamAcc {
   v16f v[F::MI];
   v4f q[2];
   __device__ __forceinline__ void clear() {
-    if constexpr (F::BM == 16) {
-      q[0] = q[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    } else {
+    q[0] = q[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int mi = 0; mi < F::MI; ++mi)
+    for (int mi = 0; mi < F::MI; ++mi)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[mi][i] = 0.0f;
-    }
+      for (int i = 0; i < 16; ++i) v[mi][i] = 0.0f;
   }
 };
 
-// acc += K step `sub` of an MXFP4 weight unit and of a split-row slot of 16 rows. Lane (c, q) holds row
+// WIDE: acc += K step `sub` of an MXFP4 weight unit and of a split-row slot. Lane (c, q) holds row
 // c's E2M1 K [32 q, +32), or E4M3 K [16 q, +16) and [64 + 16 q, +16); scale lane (c, q) covers K block q.
 template <typename F>
 __device__ __forceinline__ void stream_step16(const uint8_t* wa, const uint8_t* rb, int sub, int wave, int lane,
@@ -213,22 +214,26 @@ __device__ __forceinline__ void stream_step16(const uint8_t* wa, const uint8_t* 
   }
 }
 
-// acc += K step `sub` of a weight unit x a step of split rows; f0, f1: the fp32 block scales of result
-// registers 0..7 and 8..15. A half's fragment reads run under the other half's MFMAs.
+// acc += K step `sub` of a weight unit x a step of split rows, for the weight rows w0 .. and the tile's rows
+// row0 ..; f0, f1: the fp32 block scales of result registers 0..7 and 8..15. A half's fragment reads run
+// under the other half's MFMAs. With 16 rows the slot holds BSUB steps and columns 16..31 repeat the
+// rows of 0..15.
 template <typename F>
-__device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb, int sub, int wm, int wn, int lane,
+__device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb, int sub, int w0, int row0, int lane,
                                             float f0, float f1, v16f (&acc)[F::MI]) {
   const int r = lane % 32, g = lane / 32;
-  const int row = 32 * wm + r;
-  const uint8_t* arow = wa + (64 * wn + r) * 128;
+  const int row = row0 + r % F::BM;
+  const uint8_t* arow = wa + (w0 + r) * 128;
   uint32_t sa[F::MI];
 #pragma unroll
   for (int mi = 0; mi < F::MI; ++mi)
-    sa[mi] = F::A_SCALED ? *reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + (64 * wn + 32 * mi + r) * 4 * F::SUB + 4 * sub)
+    sa[mi] = F::A_SCALED ? *reinterpret_cast<const uint32_t*>(wa + F::TW * 128 + (w0 + 32 * mi + r) * 4 * F::SUB + 4 * sub)
                          : 127;
   // where the loader put the row's scale dword
   const uint32_t sw = *reinterpret_cast<const uint32_t*>(
-      rb + F::B_TERMS + 4 * (8 * (row / 4 % F::WAVES) + 4 * (row / (4 * F::WAVES)) + row % 4));
+      rb + F::B_TERMS + (F::BM == 16 ? 16 * (F::BSUB * (row / 4) + sub) + 4 * (row % 4)
+                                     : 4 * (8 * (row / 4 % F::WAVES) + 4 * (row / (4 * F::WAVES)) + row % 4)));
+  const uint8_t* terms = rb + (F::BM == 16 ? sub * 16 * XSTEP8 : 0);
   v8i a[2][F::MI], t[2][2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -245,8 +250,8 @@ __device__ __forceinline__ void stream_step(const uint8_t* wa, const uint8_t* rb
     }
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
-      const uint4 u = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + g));
-      const uint4 v = *reinterpret_cast<const uint4*>(rb + e4_piece(row, 8 * e + 4 * h + 2 + g));
+      const uint4 u = *reinterpret_cast<const uint4*>(terms + e4_piece(row, 8 * e + 4 * h + g));
+      const uint4 v = *reinterpret_cast<const uint4*>(terms + e4_piece(row, 8 * e + 4 * h + 2 + g));
       t[h][e] = v8i{(int)u.x, (int)u.y, (int)u.z, (int)u.w, (int)v.x, (int)v.y, (int)v.z, (int)v.w};
     }
   }
@@ -335,13 +340,14 @@ __device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uin
         const int ks = F::BSUB * k + h;
         if (ks >= steps) break;  // uniform
         if constexpr (F::BM == 16) {
-          stream_step16<F>(wslot(gu), rslot(g), h, wave, lane, acc.q);
+          if constexpr (F::WIDE) stream_step16<F>(wslot(gu), rslot(g), h, wave, lane, acc.q);
+          else stream_step<F>(wslot(gu), rslot(g), h, 32 * wave, 0, lane, 1.0f, 1.0f, acc.v);
         } else {
           const int wm = wave / 4, wn = wave % 4;
           if (32 * wm >= cur.end - cur.begin) continue;  // no rows in this row tile (uniform)
           float f0 = 1.0f, f1 = 1.0f;
           if constexpr (F::BLOCK_F32) f0 = cur.s0[ks], f1 = cur.s1[ks];
-          stream_step<F>(wslot(gu), rslot(g), sub, wm, wn, lane, f0, f1, acc.v);
+          stream_step<F>(wslot(gu), rslot(g), sub, 64 * wn, 32 * wm, lane, f0, f1, acc.v);
         }
       }
       if (sub == F::GRAN - 1) ++gu;
@@ -394,21 +400,22 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
       return silu(gv) * uv;
     };
     if constexpr (F::BM == 16) {
-      const int row = lane % 16, g = lane / 16;
-      float v[4], amax = 0.0f;
+      constexpr int COLS = F::WIDE ? 16 : 32, GROUPS = F::WIDE ? 1 : 2;  // result columns; a lane's groups of 4 values
+      const int row = lane % COLS, g = lane / COLS;
+      float v[GROUPS][4], amax = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float gv = acc.q[0][i], uv = acc.q[1][i];
+      for (int i = 0; i < 4 * GROUPS; ++i) {
+        float gv = F::WIDE ? acc.q[0][i % 4] : acc.v[0][i], uv = F::WIDE ? acc.q[1][i % 4] : acc.v[0][i + 8];
         if constexpr (F::WIDE) {  // the upper terms' products, in the lane of row r +- 8
           gv += __shfl_xor(gv, 8, 64);
           uv += __shfl_xor(uv, 8, 64);
         }
-        v[i] = act(gv, uv);
-        amax = fmaxf(amax, fabsf(v[i]));
+        v[i / 4][i % 4] = act(gv, uv);
+        amax = fmaxf(amax, fabsf(v[i / 4][i % 4]));
       }
-      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+      if constexpr (F::WIDE) amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
       amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-      if (g == 0) block_max[wave][row] = amax;
+      if (lane < F::BM) block_max[wave][lane] = amax;
       stage_barrier();
       if (row >= rows) return;
       const float block = fmaxf(amax, block_max[wave ^ 1][row]);
@@ -416,17 +423,20 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
       const int n = t.nt * TG + 16 * wave;  // the wave's first column
       const int64_t at = (int64_t)(t.begin + row) * (I / 128);
       uint8_t* dst = a8 + (at + n / 128) * XSTEP8 + n % 128 + 4 * g;
-      if constexpr (F::WIDE) {
-        uint32_t w[4];
-        fp8_terms4_wide(v, pow2_biased(254 - s), w);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          *reinterpret_cast<uint32_t*>(dst + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128) = w[e];
-      } else {
-        uint32_t hi, lo;
-        fp8_terms4(v, pow2_biased(254 - s), hi, lo);
-        *reinterpret_cast<uint32_t*>(dst) = hi;
-        *reinterpret_cast<uint32_t*>(dst + 128) = lo;
+      for (int q = 0; q < GROUPS; ++q) {  // columns 8 q + 4 g .. + 3
+        if constexpr (F::WIDE) {
+          uint32_t w[4];
+          fp8_terms4_wide(v[q], pow2_biased(254 - s), w);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            *reinterpret_cast<uint32_t*>(dst + 8 * q + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128) = w[e];
+        } else {
+          uint32_t hi, lo;
+          fp8_terms4(v[q], pow2_biased(254 - s), hi, lo);
+          *reinterpret_cast<uint32_t*>(dst + 8 * q) = hi;
+          *reinterpret_cast<uint32_t*>(dst + 8 * q + 128) = lo;
+        }
       }
       if (wave % 2 == 0 && g == 0) {
         a8s[at * 4 + n / 32] = (uint8_t)s;
@@ -508,17 +518,9 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
       float* dst = (float*)out_rows + (int64_t)row * H + col + lane / 16 * 4;
 #pragma unroll
       for (int q = 0; q < 2; ++q) *reinterpret_cast<v4f*>(dst + 16 * q) = acc.q[q];
-    } else if constexpr (F::BM == 16) {
-      const int row = t.begin + lane % 16;
-      if (row >= t.end) return;
-      uint16_t* dst = out + (int64_t)row * H + col + lane / 16 * 4;
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        *reinterpret_cast<uint2*>(dst + 16 * q) =
-            make_uint2(pack_bf16x2(acc.q[q][0], acc.q[q][1]), pack_bf16x2(acc.q[q][2], acc.q[q][3]));
     } else {
-      const int g = lane / 32, row = t.begin + 32 * (wave / 4) + lane % 32;
-      if (t.begin + 32 * (wave / 4) >= t.end) return;  // uniform
+      const int row0 = t.begin + (F::BM == 16 ? 0 : 32 * (wave / 4)), row = row0 + lane % 32, g = lane / 32;
+      if (row0 >= t.end) return;  // uniform
       // a swap between the lane halves gives each lane 8 columns in a row: stores of 16 bytes
 #pragma unroll
       for (int mi = 0; mi < F::MI; ++mi)
