@@ -1,8 +1,8 @@
-"""MXFP4 calls of a few tokens (T k <= 256 pairs of experts large enough, T k H I >= 1.2e8): grouped 8-row tiles whose activations enter as four
+"""MXFP4 calls of a few tokens (T k <= 256 pairs of experts large enough, T k H I >= 1.2e8): grouped 5-row tiles whose activations enter as six
 E4M3 terms and whose rows stay fp32, against the oracle's fp32 experts and a float64 combine.
 
 Bounds: y is rounded to bf16 once, at most 2^-9 of each value, so 2^-9 of the result's norm; the
-fp32 sums and the terms (below 2^-17 of a block's maximum) get 2^-13 more. Rows or act kept in
+fp32 sums and the terms (24 bits of a value down to 2^-13 of its block's maximum) get 2^-13 more. Rows or act kept in
 16 bits would not pass: they add 2^-9 each.
 """
 import numpy as np
@@ -23,10 +23,10 @@ def oracle_experts(a):
             for e in range(len(a["gate_up"]))]
 
 
-# one row an expert and none, 8 and 9 rows of one expert, up to 32 of each, as many pairs as the path
+# one row an expert and none, 5, 8 and 9 rows of one expert, up to 32 of each, as many pairs as the path
 # takes; K of the fewest, odd and many steps, last column tiles of half width
 @pytest.mark.parametrize("T,k,E,H,I", [(32, 8, 512, 1024, 512), (25, 10, 64, 1152, 640), (32, 8, 9, 384, 1280),
-                                       (16, 16, 16, 1280, 384), (9, 2, 2, 4096, 2048), (8, 1, 1, 7168, 2432),
+                                       (16, 16, 16, 1280, 384), (9, 2, 2, 4096, 2048), (8, 1, 1, 7168, 2432), (5, 4, 4, 4096, 2048),
                                        (3, 4, 4, 5120, 2304)])
 def test_few_tokens_match_oracle(device, T, k, E, H, I):
     rng = np.random.default_rng(T + k + E + H + I)
@@ -83,3 +83,22 @@ def test_few_tokens_slots_masks_and_replays(device):
         torch.cuda.synchronize()
         assert torch.equal(captured, got)
         assert torch.equal(wa.moe_mxfp4(x, i_d, w_d, tab), got)
+
+
+def test_few_tokens_hold_act_in_32_bits(device):
+    """Act enters the down product as fp32 holds it, also beside a value 2^24 times as large in its 32-value block:
+    columns 32 n of gate_up carry 2^12 times the weights (gate and up) and none in down, so y is made
+    of the others. Six terms leave at most 2^-37 of the block's maximum, 2^-13 of those."""
+    rng = np.random.default_rng(24)
+    T, k, E, H, I = 6, 4, 8, 2560, 2048
+    a = S.mxfp4_experts_np(rng, E, H, I)
+    for base in (0, I):
+        a["gate_up_scales"][:, base:base + I:32] += 12
+    a["down"][..., ::4] &= ~a["down"].dtype.type(15)
+    tab = S.experts_to_device(a, device)
+    x_bits = S.bf16_normal_np(rng, (T, H))
+    ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
+    got = wa.experts_mxfp4(S.bf16_bits_to_tensor(x_bits, device), torch.from_numpy(ids).to(device), tab)
+    want = np.asarray(M.routed_outputs(S.bf16_bits_to_f32(x_bits), ids, oracle_experts(a)), dtype=np.float64)
+    err = np.linalg.norm(got.double().cpu().numpy() - want, axis=-1) / np.linalg.norm(want, axis=-1)
+    assert err.max() <= BOUND + 2.0 ** -13

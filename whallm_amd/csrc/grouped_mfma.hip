@@ -320,18 +320,21 @@ __device__ __forceinline__ void fp8_terms4(const float (&v)[4], float f, uint32_
   lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[2], l[3], (int)u01, true);
 }
 
-// Four terms, for fp32 values: each the E4M3 rounding of 16 times what the one before it leaves, under
-// the scales s, s - 4, s - 8, s - 12. What is left is below 2^-17 of the block's maximum.
+// Six terms, for fp32 values: each the E4M3 rounding of 16 times what the one before it leaves, under the
+// scales s, s - 4, .., s - 20. A term takes 4 bits off a value, so six hold all 24 of one down to 2^-13 of its
+// block's maximum; the last term's smallest step bounds what a smaller one loses, 2^-37 of the maximum (a
+// bf16 value is exact down to 2^-29), or 2^-136 where the maximum is below 2^-99 and the scale stops.
+constexpr int WIDE_TERMS = 6;
 __device__ __forceinline__ int fp8_term_exponent_wide(float amax) {
   const int s = fp8_term_exponent(amax);
-  return s > 13 ? s : 13;  // the fourth term's scale stays a normal power of two
+  return s > 21 ? s : 21;  // the last term's scale stays a normal power of two
 }
-__device__ __forceinline__ void fp8_terms4_wide(const float (&v)[4], float f, uint32_t (&t)[4]) {
+__device__ __forceinline__ void fp8_terms4_wide(const float (&v)[4], float f, uint32_t (&t)[WIDE_TERMS]) {
   float h[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) h[j] = v[j] * f;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  for (int e = 0; e < WIDE_TERMS; ++e) {
     const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[0], h[1], 0, false);
     t[e] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[2], h[3], (int)w01, true);
     h[0] = (h[0] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 0)) * 16.0f;
@@ -1791,15 +1794,16 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
 // A few tokens (T k <= 256 pairs) of MXFP4 row-layout experts: the 16-row streaming tiles with the
 // decode GEMV's precision. The GEMV passes an expert's weights once per pair that chose it (the shared
 // expert's once per token) and is bound by its converts and by act reads past the first token:
-// 1.7 TB/s in down. Here a weight row is read once per 8 rows, at the streaming tiles' rate; four E4M3
-// terms carry x exactly and the fp32 act to 2^-17 of its block (the matrix instructions
-// have 16 columns and an expert few rows, so the second pair of terms takes the columns
-// 8..15), and the rows stay fp32 up to the combine. One launch does what the prefill's
-// permute, row map, split and gate launches do.
+// 1.7 TB/s in down. Here a weight row is read once per 5 rows, at the streaming tiles' rate; six E4M3
+// terms carry x and the fp32 act (fp8_terms4_wide; the matrix instructions have 16 columns and an expert
+// few rows, so the second and third pair of terms take columns of their own), and the rows
+// stay fp32 up to the combine. One launch does what the prefill's permute, row map, split and
+// gate launches do.
 constexpr int FEW_PAIRS = 256;
+using FewF = StreamF<false, true, 16, 4, true>;
 
 // Block 0: the pair lists (thread p: pair p). Blocks 1 .. split: the terms of x, a lane per 32-value
-// block, the third and fourth as rows tokens .. 2 tokens - 1. The others: the shared gate, a wave
+// block, set h of them as rows h tokens .. (h + 1) tokens - 1. The others: the shared gate, a wave
 // per token.
 __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restrict__ x, int tokens, int hidden,
                                                        const int32_t* __restrict__ indices, int k, int experts,
@@ -1829,7 +1833,7 @@ __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restric
         count += q[c] == e;
       }
     }
-    const bool first = valid && rank % 8 == 0;  // a tile's first row
+    const bool first = valid && rank % FewF::ROWS == 0;  // a tile's first row
     head[p] = first ? before + rank : 0x7fffffff;
     __syncthreads();
     const int row = before + rank;
@@ -1878,16 +1882,16 @@ __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restric
     }
   }
   const int s = fp8_term_exponent_wide(amax);
-  uint32_t t[4][8];
+  uint32_t t[WIDE_TERMS][8];
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
-    uint32_t four[4];
-    fp8_terms4_wide(v[q], pow2_biased(254 - s), four);
+    uint32_t w[WIDE_TERMS];
+    fp8_terms4_wide(v[q], pow2_biased(254 - s), w);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) t[e][q] = four[e];
+    for (int e = 0; e < WIDE_TERMS; ++e) t[e][q] = w[e];
   }
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < FewF::SETS; ++h) {
     const int64_t at = ((int64_t)(row + h * tokens) * (hidden / 128) + blk / 4);
     uint8_t* step = x8 + at * XSTEP8 + (blk % 4) * 32;
 #pragma unroll
@@ -1918,10 +1922,10 @@ static FewLayout few_layout(int tokens, int k, int experts, int hidden, int inte
   take(p.tile_count, 4);
   take(p.gate, 4 * (size_t)tokens);
   take(p.row_token, 4 * rows);
-  take(p.x8, 2 * (size_t)tokens * (hidden / 128) * XSTEP8);
-  take(p.x8s, 2 * (size_t)tokens * (hidden / 128) * 4);
-  take(p.a8, 2 * rows * (inter / 128) * XSTEP8);
-  take(p.a8s, 2 * rows * (inter / 128) * 4);
+  take(p.x8, FewF::SETS * (size_t)tokens * (hidden / 128) * XSTEP8);
+  take(p.x8s, FewF::SETS * (size_t)tokens * (hidden / 128) * 4);
+  take(p.a8, FewF::SETS * rows * (inter / 128) * XSTEP8);
+  take(p.a8s, FewF::SETS * rows * (inter / 128) * 4);
   take(p.rows, 4 * rows * hidden);
   p.total = at;
   return p;
@@ -1954,7 +1958,7 @@ static void run_few(const uint16_t* x, int tokens, const int32_t* indices, const
                      (int32_t*)L.tile_count, row_token, (float*)L.shared_gate, x8, (uint32_t*)x8s);
   check_launch("few_prep");
   const wm_mxfp4_experts sh = shared ? *shared : routed;
-  using S = StreamF<false, true, 16, 4, true>;
+  using S = FewF;
   const int row_tiles = pairs + (has_shared ? (tokens + S::ROWS - 1) / S::ROWS : 0);  // at most
   auto grid_for = [&](int n_tiles) {
     const int per_xcd = std::min((row_tiles * n_tiles + XCDS - 1) / XCDS, std::max(compute_units() / XCDS, 1) * 2);

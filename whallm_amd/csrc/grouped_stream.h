@@ -23,7 +23,7 @@
 // Two shapes: 64 rows x 256 weight rows (8 waves, 154 KB), one row tile an expert; and, for MXFP4, 16
 // rows x 128 (4 waves, 77 KB), two workgroups on a CU, one's epilogue and tile set-up under the
 // other's loads. row_tiles() says which call takes which, with times. WIDE: the 16-row shape for calls
-// of a few tokens, 8 rows a tile with activations of four terms (see run_few). At 2 rows an expert of
+// of a few tokens, 5 rows a tile with activations of six terms (see run_few). At 2 rows an expert of
 // 7168/2048 FP8 weights (11.3 GB): 1486 us a call against 2791 with 128-row tiles, 7.6 TB/s.
 #pragma once
 
@@ -34,9 +34,10 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <bool FP8_, bool A_SCALED_, int BM_, int WAVES_, bool WIDE_ = false>
 struct StreamF {
-  // WIDE: tile row r >= 8 holds the third and fourth term of row r - 8
+  // WIDE: six terms, two in each of SETS operand rows; operand row r holds set r / ROWS of tile row r % ROWS
+  // (the one past the last repeats the last set and goes unused)
   static constexpr bool WIDE = WIDE_;
-  static constexpr int ROWS = WIDE_ ? 8 : BM_;  // rows of a tile
+  static constexpr int SETS = WIDE_ ? 3 : 1, ROWS = BM_ / SETS;  // rows of a tile
   static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
   static constexpr int BM = BM_, WAVES = WAVES_, TW = 32 * WAVES_;
   static constexpr int MI = BM_ == 16 ? 1 : 2;             // a wave's weight tiles
@@ -54,7 +55,7 @@ struct StreamF {
   // loads of a wave: a unit's, and at least a split-row slot's (see issue_rows)
   static constexpr int UNIT_LOADS = NQA + (A_SCALED_ ? 1 : 0), ROW_LOADS = BM_ == 16 ? BSUB + 1 : 2;
   static_assert(BM_ == 16 ? NQB == 1 && !FP8_ : BM_ == 64 && NQB == 2, "the loader's split-row loads");
-  static_assert(!WIDE_ || BM_ == 16, "four terms: 16-row tiles");
+  static_assert(!WIDE_ || BM_ == 16, "six terms: 16-row tiles");
 };
 
 // Loads of one tile. Weight load i of wave w fills rows 8 (w + WAVES i) .. + 7 of the tile: lane l
@@ -358,6 +359,15 @@ __device__ __forceinline__ void stream_tiles(const TileRange& tr, int steps, uin
   }
 }
 
+// WIDE: in the lanes of the first set, its product plus those of the others, the smallest first.
+template <typename F>
+__device__ __forceinline__ float sum_sets(float v, int lane) {
+  float low = __shfl(v, lane + (F::SETS - 1) * F::ROWS, 64);
+#pragma unroll
+  for (int h = F::SETS - 2; h > 0; --h) low += __shfl(v, lane + h * F::ROWS, 64);
+  return v + low;
+}
+
 // act rows of TW / 2 intermediate columns, 16 a weight tile: result lane (r, g) register i < 8 is the
 // gate and i + 8 the up product of column 8 (i / 4) + 4 g + i % 4 for row r of the row tile.
 // Weight tiles 2 p and 2 p + 1 share a 32-value block of the act row: a wave's own two, or with 16 rows
@@ -387,7 +397,7 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
     const int begin = t.begin, end = t.end;
     t.ld.rows(x8, x8s, H, wave, lane, [&](int r) {
       const int q = begin + r % F::ROWS;
-      return scalar_i32(row_token, q < end ? q : begin) + (r < F::ROWS ? 0 : x_rows);
+      return scalar_i32(row_token, q < end ? q : begin) + min(r / F::ROWS, F::SETS - 1) * x_rows;
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
@@ -406,10 +416,7 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
 #pragma unroll
       for (int i = 0; i < 4 * GROUPS; ++i) {
         float gv = F::WIDE ? acc.q[0][i % 4] : acc.v[0][i], uv = F::WIDE ? acc.q[1][i % 4] : acc.v[0][i + 8];
-        if constexpr (F::WIDE) {  // the upper terms' products, in the lane of row r +- 8
-          gv += __shfl_xor(gv, 8, 64);
-          uv += __shfl_xor(uv, 8, 64);
-        }
+        if constexpr (F::WIDE) gv = sum_sets<F>(gv, lane), uv = sum_sets<F>(uv, lane);
         v[i / 4][i % 4] = act(gv, uv);
         amax = fmaxf(amax, fabsf(v[i / 4][i % 4]));
       }
@@ -426,10 +433,10 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
 #pragma unroll
       for (int q = 0; q < GROUPS; ++q) {  // columns 8 q + 4 g .. + 3
         if constexpr (F::WIDE) {
-          uint32_t w[4];
+          uint32_t w[WIDE_TERMS];
           fp8_terms4_wide(v[q], pow2_biased(254 - s), w);
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
+          for (int e = 0; e < WIDE_TERMS; ++e)
             *reinterpret_cast<uint32_t*>(dst + 8 * q + (int64_t)(e / 2) * a_rows * (I / 128) * XSTEP8 + e % 2 * 128) = w[e];
         } else {
           uint32_t hi, lo;
@@ -439,8 +446,8 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
         }
       }
       if (wave % 2 == 0 && g == 0) {
-        a8s[at * 4 + n / 32] = (uint8_t)s;
-        if (F::WIDE) a8s[(at + (int64_t)a_rows * (I / 128)) * 4 + n / 32] = (uint8_t)(s - 8);
+#pragma unroll
+        for (int h = 0; h < F::SETS; ++h) a8s[(at + (int64_t)h * a_rows * (I / 128)) * 4 + n / 32] = (uint8_t)(s - 8 * h);
       }
     } else {
       const int wm = wave / 4, wn = wave % 4, g = lane / 32, row = 32 * wm + lane % 32;
@@ -502,7 +509,7 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
     const int begin = t.begin, end = t.end;
     t.ld.rows(a8, a8s, I, wave, lane, [&](int r) {
       const int q = begin + r % F::ROWS;
-      return (q < end ? q : begin) + (r < F::ROWS ? 0 : a_rows);
+      return (q < end ? q : begin) + min(r / F::ROWS, F::SETS - 1) * a_rows;
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
@@ -512,7 +519,7 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
 #pragma unroll
       for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc.q[q][i] += __shfl_xor(acc.q[q][i], 8, 64);
+        for (int i = 0; i < 4; ++i) acc.q[q][i] = sum_sets<F>(acc.q[q][i], lane);
       const int row = t.begin + lane % 16;
       if (lane % 16 >= F::ROWS || row >= t.end) return;
       float* dst = (float*)out_rows + (int64_t)row * H + col + lane / 16 * 4;
