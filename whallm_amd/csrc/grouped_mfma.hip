@@ -320,14 +320,18 @@ __device__ __forceinline__ void fp8_terms4(const float (&v)[4], float f, uint32_
   lo = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(l[2], l[3], (int)u01, true);
 }
 
-// Six terms, for fp32 values: each the E4M3 rounding of 16 times what the one before it leaves, under the
-// scales s, s - 4, .., s - 20. A term takes 4 bits off a value, so six hold all 24 of one down to 2^-13 of its
-// block's maximum; the last term's smallest step bounds what a smaller one loses, 2^-37 of the maximum (a
-// bf16 value is exact down to 2^-29), or 2^-136 where the maximum is below 2^-99 and the scale stops.
-constexpr int WIDE_TERMS = 6;
+// Eight terms, for fp32 values and fp32 sums: the digits of v 2^(127 - s) in base 16 (the first up to 16, the
+// others up to 8 in size; whole numbers that E4M3 holds exactly) under the scales s, s - 4, .., s - 28. A
+// value is off by at most 2^-32 of its block's maximum, exact down to 2^-8 of it (a bf16 value down
+// to 2^-24); below a maximum of 2^-95 the scale stops and it is 2^-127. Digits and not roundings of what is left, as
+// in the two terms: the matrix instruction adds the products of 8 neighbours in about 14 bits (beside
+// 256 it drops 2^-6 and keeps 2^-5), so terms of unlike size lose bits of the sum, whole numbers up to 16 times
+// E2M1 values none (8 tokens of 2560/640: 1.4% of the results rounded to another bf16 value
+// than the 64-bit ones' with floating terms, GEMV 0.03%).
+constexpr int WIDE_TERMS = 8;
 __device__ __forceinline__ int fp8_term_exponent_wide(float amax) {
-  const int s = fp8_term_exponent(amax);
-  return s > 21 ? s : 21;  // the last term's scale stays a normal power of two
+  const int s = fp8_term_exponent(amax) + 4;  // the maximum in [8, 16)
+  return s > 29 ? s : 29;  // the last term's scale stays a normal power of two
 }
 __device__ __forceinline__ void fp8_terms4_wide(const float (&v)[4], float f, uint32_t (&t)[WIDE_TERMS]) {
   float h[4];
@@ -335,12 +339,14 @@ __device__ __forceinline__ void fp8_terms4_wide(const float (&v)[4], float f, ui
   for (int j = 0; j < 4; ++j) h[j] = v[j] * f;
 #pragma unroll
   for (int e = 0; e < WIDE_TERMS; ++e) {
-    const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[0], h[1], 0, false);
-    t[e] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(h[2], h[3], (int)w01, true);
-    h[0] = (h[0] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 0)) * 16.0f;
-    h[1] = (h[1] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 1)) * 16.0f;
-    h[2] = (h[2] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 2)) * 16.0f;
-    h[3] = (h[3] - __builtin_amdgcn_cvt_f32_fp8((int)t[e], 3)) * 16.0f;
+    float d[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      d[j] = rintf(h[j]);
+      h[j] = (h[j] - d[j]) * 16.0f;
+    }
+    const uint32_t w01 = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(d[0], d[1], 0, false);
+    t[e] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(d[2], d[3], (int)w01, true);
   }
 }
 
@@ -1794,9 +1800,9 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
 // A few tokens (T k <= 256 pairs) of MXFP4 row-layout experts: the 16-row streaming tiles with the
 // decode GEMV's precision. The GEMV passes an expert's weights once per pair that chose it (the shared
 // expert's once per token) and is bound by its converts and by act reads past the first token:
-// 1.7 TB/s in down. Here a weight row is read once per 5 rows, at the streaming tiles' rate; six E4M3
+// 1.7 TB/s in down. Here a weight row is read once per 4 rows, at the streaming tiles' rate; eight E4M3
 // terms carry x and the fp32 act (fp8_terms4_wide; the matrix instructions have 16 columns and an expert
-// few rows, so the second and third pair of terms take columns of their own), and the rows
+// few rows, so each further pair of terms takes columns of its own), and the rows
 // stay fp32 up to the combine. One launch does what the prefill's permute, row map, split and
 // gate launches do.
 constexpr int FEW_PAIRS = 256;

@@ -23,7 +23,7 @@
 // Two shapes: 64 rows x 256 weight rows (8 waves, 154 KB), one row tile an expert; and, for MXFP4, 16
 // rows x 128 (4 waves, 77 KB), two workgroups on a CU, one's epilogue and tile set-up under the
 // other's loads. row_tiles() says which call takes which, with times. WIDE: the 16-row shape for calls
-// of a few tokens, 5 rows a tile with activations of six terms (see run_few). At 2 rows an expert of
+// of a few tokens, 4 rows a tile with activations of eight terms (see run_few). At 2 rows an expert of
 // 7168/2048 FP8 weights (11.3 GB): 1486 us a call against 2791 with 128-row tiles, 7.6 TB/s.
 #pragma once
 
@@ -34,10 +34,9 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 template <bool FP8_, bool A_SCALED_, int BM_, int WAVES_, bool WIDE_ = false>
 struct StreamF {
-  // WIDE: six terms, two in each of SETS operand rows; operand row r holds set r / ROWS of tile row r % ROWS
-  // (the one past the last repeats the last set and goes unused)
+  // WIDE: eight terms, two in each of SETS operand rows; operand row r holds set r / ROWS of tile row r % ROWS
   static constexpr bool WIDE = WIDE_;
-  static constexpr int SETS = WIDE_ ? 3 : 1, ROWS = BM_ / SETS;  // rows of a tile
+  static constexpr int SETS = WIDE_ ? 4 : 1, ROWS = BM_ / SETS;  // rows of a tile
   static constexpr bool FP8 = FP8_, A_SCALED = A_SCALED_, BLOCK_F32 = FP8_ && !A_SCALED_;
   static constexpr int BM = BM_, WAVES = WAVES_, TW = 32 * WAVES_;
   static constexpr int MI = BM_ == 16 ? 1 : 2;             // a wave's weight tiles
@@ -55,7 +54,7 @@ struct StreamF {
   // loads of a wave: a unit's, and at least a split-row slot's (see issue_rows)
   static constexpr int UNIT_LOADS = NQA + (A_SCALED_ ? 1 : 0), ROW_LOADS = BM_ == 16 ? BSUB + 1 : 2;
   static_assert(BM_ == 16 ? NQB == 1 && !FP8_ : BM_ == 64 && NQB == 2, "the loader's split-row loads");
-  static_assert(!WIDE_ || BM_ == 16, "six terms: 16-row tiles");
+  static_assert(!WIDE_ || BM_ == 16, "eight terms: 16-row tiles");
 };
 
 // Loads of one tile. Weight load i of wave w fills rows 8 (w + WAVES i) .. + 7 of the tile: lane l
@@ -397,7 +396,7 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
     const int begin = t.begin, end = t.end;
     t.ld.rows(x8, x8s, H, wave, lane, [&](int r) {
       const int q = begin + r % F::ROWS;
-      return scalar_i32(row_token, q < end ? q : begin) + min(r / F::ROWS, F::SETS - 1) * x_rows;
+      return scalar_i32(row_token, q < end ? q : begin) + r / F::ROWS * x_rows;
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
@@ -509,7 +508,7 @@ __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restr
     const int begin = t.begin, end = t.end;
     t.ld.rows(a8, a8s, I, wave, lane, [&](int r) {
       const int q = begin + r % F::ROWS;
-      return (q < end ? q : begin) + min(r / F::ROWS, F::SETS - 1) * a_rows;
+      return (q < end ? q : begin) + r / F::ROWS * a_rows;
     });
   };
   auto epilogue = [&](const StreamTile<F>& t, StreamAcc<F>& acc) {
