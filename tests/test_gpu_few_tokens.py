@@ -5,13 +5,17 @@ Bounds: y is rounded to bf16 once, at most 2^-9 of each value, so 2^-9 of the re
 fp32 sums and the terms (2^-32 of a block's maximum) get 2^-13 more. Rows or act kept in
 16 bits would not pass: they add 2^-9 each.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import whallm_amd as wa
 from oracle import moe as M
+from whallm_amd import _lib
 from whallm_amd import synthetic as S
+from whallm_amd.ops import _ptr, _stream
 
 pytestmark = pytest.mark.gpu
 
@@ -134,3 +138,25 @@ def test_few_tokens_sum_in_32_bits(device, T, k, E, H, I):
         off += int((got[t, j].cpu() != rounded).sum())
         n += rounded.numel()
     assert off <= 1e-3 * n, off / n
+
+
+def test_few_tokens_read_nothing_for_what_is_not_resident(device):
+    """With no expert resident, routed or shared, the call adds nothing and computes nothing: its act and output
+    rows in the workspace stay untouched (every byte of the rows, 4 H T (k + 1), and more)."""
+    rng = np.random.default_rng(3)
+    T, k, E, H, I = 6, 4, 12, 2560, 2048
+    gone = torch.full((E,), -1, dtype=torch.int32, device=device)
+    tab = S.experts_to_device(S.mxfp4_experts_np(rng, E, H, I), device, slots=gone, experts=E)
+    shared = S.experts_to_device(S.mxfp4_experts_np(rng, 1, H, I), device, slots=gone[:1], experts=1)
+    x = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (T, H)), device)
+    ids = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)).to(device)
+    w = torch.rand(T, k, device=device) + 0.1
+    c, sc = tab.c_struct(), shared.c_struct()
+    nbytes = _lib.load().wm_moe_mxfp4_workspace_size(T, k, ctypes.byref(c))
+    ws = torch.full((nbytes,), 0x5a, dtype=torch.uint8, device=device)
+    y = torch.full_like(x, 3.0)
+    _lib.call("wm_moe_mxfp4", _ptr(x), T, _ptr(ids), _ptr(w), k, ctypes.byref(c), ctypes.byref(sc), None, _ptr(y),
+              _ptr(ws), nbytes, _stream(device))
+    torch.cuda.synchronize()
+    assert bool((y == 0).all())
+    assert int((ws == 0x5a).sum()) >= 4 * H * T * (k + 1) + 2 * I * T * (k + 1)

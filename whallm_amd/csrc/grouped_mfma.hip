@@ -1808,11 +1808,13 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
 constexpr int FEW_PAIRS = 256;
 using FewF = StreamF<false, true, 16, 4, true>;
 
-// Block 0: the pair lists (thread p: pair p). Blocks 1 .. split: the terms of x, a lane per 32-value
+// Block 0: the pair lists (thread p: pair p; pairs of experts that are not resident are left out, so that no
+// weights are read for them). Blocks 1 .. split: the terms of x, a lane per 32-value
 // block, set h of them as rows h tokens .. (h + 1) tokens - 1. The others: the shared gate, a wave
 // per token.
 __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restrict__ x, int tokens, int hidden,
                                                        const int32_t* __restrict__ indices, int k, int experts,
+                                                       const int32_t* __restrict__ slots,
                                                        const uint16_t* __restrict__ g, int split_blocks,
                                                        int32_t* __restrict__ inverse, int32_t* __restrict__ offsets,
                                                        int32_t* __restrict__ tiles, int32_t* __restrict__ tile_count,
@@ -1823,7 +1825,7 @@ __global__ void __launch_bounds__(256) few_prep_kernel(const uint16_t* __restric
     __shared__ __attribute__((aligned(16))) int32_t id[FEW_PAIRS], head[FEW_PAIRS];
     const int p = threadIdx.x;
     const int32_t raw = p < pairs ? indices[p] : -1;
-    const bool valid = raw >= 0 && raw < experts;
+    const bool valid = raw >= 0 && raw < experts && (!slots || slots[raw] >= 0);
     const int32_t e = valid ? raw : 0x7fffffff;  // after every expert
     id[p] = e;
     __syncthreads();
@@ -1960,7 +1962,7 @@ static void run_few(const uint16_t* x, int tokens, const int32_t* indices, const
   float* out_rows = (float*)(base + p.rows);
   const int split_blocks = (tokens * (H / 32) + 255) / 256, gate_blocks = has_shared ? (tokens + 3) / 4 : 0;
   hipLaunchKernelGGL(few_prep_kernel, dim3(1 + split_blocks + gate_blocks), dim3(256), 0, s, x, tokens, H, indices, k,
-                     routed.experts, shared_gate, split_blocks, inverse, (int32_t*)L.offsets, (int32_t*)L.tiles,
+                     routed.experts, routed.slots, shared_gate, split_blocks, inverse, (int32_t*)L.offsets, (int32_t*)L.tiles,
                      (int32_t*)L.tile_count, row_token, (float*)L.shared_gate, x8, (uint32_t*)x8s);
   check_launch("few_prep");
   const wm_mxfp4_experts sh = shared ? *shared : routed;

@@ -367,16 +367,27 @@ __device__ __forceinline__ float sum_sets(float v, int lane) {
   return v + low;
 }
 
+// The lists of a launch. WIDE: without the shared expert's rows where its table says that it is not resident, so
+// that no weights are read for it (the routed experts' rows are left out of the lists themselves).
+template <typename F, typename Table>
+__device__ __forceinline__ Lists resident_lists(const Lists& all, const Table& shared) {
+  Lists L = all;
+  if constexpr (F::WIDE)
+    if (L.has_shared && shared.slots && scalar_i32(shared.slots, 0) < 0) L.has_shared = 0;
+  return L;
+}
+
 // act rows of TW / 2 intermediate columns, 16 a weight tile: result lane (r, g) register i < 8 is the
 // gate and i + 8 the up product of column 8 (i / 4) + 4 g + i % 4 for row r of the row tile.
 // Weight tiles 2 p and 2 p + 1 share a 32-value block of the act row: a wave's own two, or with 16 rows
 // those of two waves.
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
-                                               const int32_t* __restrict__ row_token, const Lists& L, const Table& routed,
+                                               const int32_t* __restrict__ row_token, const Lists& all, const Table& routed,
                                                const Table& shared, int before, int x_rows, int a_rows,
                                                uint8_t* __restrict__ a8, uint8_t* __restrict__ a8s) {
   float(*block_max)[F::BM] = reinterpret_cast<float(*)[F::BM]>(lds + F::RINGS);  // 16 rows
+  const Lists L = resident_lists<F>(all, shared);
   constexpr int TG = F::TW / 2;
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = I / TG;  // I is a multiple of 128
@@ -489,9 +500,10 @@ __device__ __forceinline__ void stream_gate_up(uint8_t* lds, const uint8_t* __re
 // Output rows (bf16, permuted order) of TW columns, 32 a weight tile.
 template <typename F, typename Table>
 __device__ __forceinline__ void stream_down(uint8_t* lds, const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
-                                            const Lists& L, const Table& routed, const Table& shared, int before,
+                                            const Lists& all, const Table& routed, const Table& shared, int before,
                                             int a_rows, void* __restrict__ out_rows) {
   uint16_t* __restrict__ out = (uint16_t*)out_rows;
+  const Lists L = resident_lists<F>(all, shared);
   const int H = routed.hidden, I = routed.inter;
   const int n_tiles = (H + F::TW - 1) / F::TW;
   const TileRange tr = tile_range_after(active_row_tiles<F::ROWS>(L) * n_tiles, before, F::HOT_COST);
