@@ -153,7 +153,9 @@ WM_EXPORT int wm_permute(const int32_t* indices, int64_t pairs, int32_t experts,
  *   y[t] = sum_k weights[t,k] * FFN_{indices[t,k]}(x[t]) + sigmoid(x[t] . shared_gate) * FFN_shared(x[t])
  * x, y bf16 [T, H]; shared may be NULL (no shared term) and shared_gate NULL
  * (ungated shared expert, the DeepSeek form, model.py:540-541).
- * Decode path (fused dequant-GEMV) for T*K <= 256, MFMA grouped GEMM otherwise.
+ * T*K <= 256 in the row layout: the decode path (fused dequant-GEMV), or from T*K*H*I = 1.2e8
+ * (H and I multiples of 128 from 384, 4-byte aligned scales, 16-byte aligned x and y) grouped tiles
+ * at the GEMV's precision. Otherwise the MFMA grouped GEMM.
  * workspace: wm_moe_mxfp4_workspace_size bytes. */
 WM_EXPORT size_t wm_moe_mxfp4_workspace_size(int32_t tokens, int32_t k, const wm_mxfp4_experts* experts);
 WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices, const float* weights,
@@ -162,11 +164,11 @@ WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices
                            void* stream);
 /* wm_moe_mxfp4 without a workspace and without any allocation, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). No counterpart in the reference. Its scratch (the decode path's act rows) is
- * a file-scope device array of wm_moe_mxfp4_noalloc_max_bytes() = 4 MiB per GPU, held until
- * the process ends; its address is looked up on a device's first call. Only calls that take
- * the decode path (tokens * k <= 256, row layout) and need at most that much scratch
- * (4 * (tokens * (k + 1)) * inter bytes) are accepted; others fail with a message. Every
+ * hipMalloc). No counterpart in the reference. Its scratch is a file-scope device array of
+ * 16 MiB per GPU, held until the process ends; its address is looked up on a device's first
+ * call. Only calls of tokens * k <= 256 in the row layout whose act rows
+ * (4 * (tokens * (k + 1)) * inter bytes) are at most wm_moe_mxfp4_noalloc_max_bytes() = 4 MiB
+ * are accepted; others fail with a message. Every
  * call on one GPU shares its array, so calls that may overlap on one GPU (other streams,
  * other threads) race; calls ordered on one stream do not. Same results as wm_moe_mxfp4. */
 WM_EXPORT size_t wm_moe_mxfp4_noalloc_max_bytes(void);

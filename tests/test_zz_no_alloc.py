@@ -49,6 +49,18 @@ def test_noalloc_matches_the_workspace_entry_point(device):
         assert torch.equal(y, y_ref), (tokens, k)
 
 
+# the grouped tiles' buffers: 10.5 MB at once, and 43 MB in pieces of the call
+@pytest.mark.parametrize("tokens,k,E,H,I", [(32, 8, 16, 4096, 2048), (256, 1, 2, 8192, 2048)])
+def test_noalloc_takes_the_path_of_the_workspace_entry_point(device, tokens, k, E, H, I):
+    """Calls of the largest scratch still give wm_moe_mxfp4's bits."""
+    rng = np.random.default_rng(H)
+    table = S.experts_to_device(S.mxfp4_experts_np(rng, E, H, I), device)
+    shared = S.experts_to_device(S.mxfp4_experts_np(rng, 1, H, I), device)
+    gate = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (H,), 0.02), device)
+    y, y_ref = _call_pair(device, table, shared, gate, tokens, k, tokens + k)
+    assert torch.equal(y, y_ref)
+
+
 def test_noalloc_rejects_what_it_cannot_hold(device):
     # a real (small) table, so nothing would read outside it even if a check were missing
     rng = np.random.default_rng(5)

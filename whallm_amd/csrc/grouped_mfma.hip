@@ -1935,7 +1935,7 @@ static FewLayout few_layout(int tokens, int k, int experts, int hidden, int inte
   take(p.a8, FewF::SETS * rows * (inter / 128) * XSTEP8);
   take(p.a8s, FewF::SETS * rows * (inter / 128) * 4);
   take(p.rows, 4 * rows * hidden);
-  p.total = at;
+  p.total = at + 16;  // the buffers start at a multiple of 16 bytes
   return p;
 }
 
@@ -1946,7 +1946,7 @@ static void run_few(const uint16_t* x, int tokens, const int32_t* indices, const
   const bool has_shared = combine && shared != nullptr;
   const FewLayout p = few_layout(tokens, k, routed.experts, H, I);
   const int pairs = tokens * k, rows = pairs + tokens;
-  uint8_t* base = (uint8_t*)ws;
+  uint8_t* base = (uint8_t*)(((uintptr_t)ws + 15) & ~(uintptr_t)15);
   Lists L{};
   L.offsets = (int32_t*)(base + p.offsets);
   L.tiles = (int32_t*)(base + p.tiles);

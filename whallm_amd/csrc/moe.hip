@@ -51,9 +51,9 @@ static bool use_decode(int tokens, int k, const wm_mxfp4_experts& e) {
 
 // Calls of the decode path that the few-token path takes over (the workspace of either fits both).
 static bool use_few(int tokens, int k, const wm_mxfp4_experts& e, const wm_mxfp4_experts* shared, const void* x,
-                    const void* y, const void* workspace) {
+                    const void* y) {
   return few_mxfp4_takes(tokens, k, e) && few_mxfp4_aligned(&e) && few_mxfp4_aligned(shared) && (uintptr_t)x % 16 == 0 &&
-         (uintptr_t)y % 16 == 0 && (uintptr_t)workspace % 16 == 0;
+         (uintptr_t)y % 16 == 0;
 }
 
 static void validate_fp8(const wm_fp8_experts* e, const char* what, bool shared) {
@@ -99,12 +99,15 @@ static size_t decode_workspace(int tokens, int k, const wm_mxfp4_experts& e) {
   return sizeof(float) * (size_t)(tokens * k + tokens) * e.inter;
 }
 
-// Scratch of the allocation-free entry point: the decode path's act rows live in this
-// file-scope device array instead of a caller workspace. Each GPU holds its own copy for
+// Scratch of the allocation-free entry point: the workspace of its calls is this file-scope
+// device array instead of a caller's. A call is accepted by the GEMV's act rows (kNoAllocMaxBytes);
+// the few-token path of an accepted call needs more, for one token up to 11 MB (8 bytes for each of at
+// most 2^20 act values, 4 for each of 33 x 16384 row values, 8 for each of x) and for most calls of 256 pairs up to
+// 15 MB, and a call that needs more still runs some tokens at a time. Each GPU holds its own copy for
 // the life of the process. Host code never passes the array's name to a kernel (on the
 // host it is only a stand-in for the symbol): the device address is looked up once per
 // device with hipGetSymbolAddress, with that device current, and kept here.
-constexpr size_t kNoAllocScratchBytes = (size_t)4 << 20;
+constexpr size_t kNoAllocMaxBytes = (size_t)4 << 20, kNoAllocScratchBytes = (size_t)16 << 20;
 __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 static void* g_scratch_ptr[64];
 static std::mutex g_scratch_mu;
@@ -150,7 +153,7 @@ WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices
     if (workspace_bytes < wm_moe_mxfp4_workspace_size(tokens, k, experts) - 256 || !workspace)
       fail("wm_moe_mxfp4: workspace too small");
     hipStream_t s = as_stream(stream);
-    if (use_few(tokens, k, *experts, shared, x, y, workspace))
+    if (use_few(tokens, k, *experts, shared, x, y))
       few_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
                 (uint16_t*)y, true, workspace, s);
     else if (use_decode(tokens, k, *experts))
@@ -162,7 +165,7 @@ WM_EXPORT int wm_moe_mxfp4(const void* x, int32_t tokens, const int32_t* indices
   });
 }
 
-WM_EXPORT size_t wm_moe_mxfp4_noalloc_max_bytes(void) { return kNoAllocScratchBytes; }
+WM_EXPORT size_t wm_moe_mxfp4_noalloc_max_bytes(void) { return kNoAllocMaxBytes; }
 
 WM_EXPORT int wm_moe_mxfp4_noalloc(const void* x, int32_t tokens, const int32_t* indices, const float* weights,
                                    int32_t k, const wm_mxfp4_experts* experts, const wm_mxfp4_experts* shared,
@@ -176,14 +179,20 @@ WM_EXPORT int wm_moe_mxfp4_noalloc(const void* x, int32_t tokens, const int32_t*
     if (!use_decode(tokens, k, *experts))
       fail("wm_moe_mxfp4_noalloc: only calls that take the decode path (tokens * k <= 256, row layout)");
     const size_t need = decode_workspace(tokens, k, *experts);
-    if (need > kNoAllocScratchBytes)
+    if (need > kNoAllocMaxBytes)
       fail("wm_moe_mxfp4_noalloc: the call needs " + std::to_string(need) + " bytes of scratch, more than the " +
-           std::to_string(kNoAllocScratchBytes) + " it has");
+           std::to_string(kNoAllocMaxBytes) + " it has");
     void* ws = scratch_for_current_device();
-    // the few-token path where its buffers fit, as in wm_moe_mxfp4
-    if (use_few(tokens, k, *experts, shared, x, y, ws) && few_mxfp4_workspace_size(tokens, k, *experts) <= kNoAllocScratchBytes)
-      return few_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
-                       (uint16_t*)y, true, ws, as_stream(stream));
+    if (use_few(tokens, k, *experts, shared, x, y)) {
+      // as many tokens at a time as the scratch holds: a token's result does not depend on the others
+      int step = tokens;
+      while (step > 1 && few_mxfp4_workspace_size(step, k, *experts) > kNoAllocScratchBytes) step = (step + 1) / 2;
+      for (int t = 0; t < tokens; t += step)
+        few_mxfp4((const uint16_t*)x + (int64_t)t * experts->hidden, std::min(step, tokens - t), indices + (int64_t)t * k,
+                  weights + (int64_t)t * k, k, *experts, shared, (const uint16_t*)shared_gate,
+                  (uint16_t*)y + (int64_t)t * experts->hidden, true, ws, as_stream(stream));
+      return;
+    }
     decode_mxfp4((const uint16_t*)x, tokens, indices, weights, k, *experts, shared, (const uint16_t*)shared_gate,
                  (uint16_t*)y, true, (float*)ws, as_stream(stream));
   });
@@ -201,7 +210,7 @@ WM_EXPORT int wm_experts_mxfp4(const void* x, int32_t tokens, const int32_t* ind
     if (workspace_bytes < wm_moe_mxfp4_workspace_size(tokens, k, experts) - 256 || !workspace)
       fail("wm_experts_mxfp4: workspace too small");
     hipStream_t s = as_stream(stream);
-    if (use_few(tokens, k, *experts, nullptr, x, out, workspace))
+    if (use_few(tokens, k, *experts, nullptr, x, out))
       few_mxfp4((const uint16_t*)x, tokens, indices, nullptr, k, *experts, nullptr, nullptr, (uint16_t*)out, false,
                 workspace, s);
     else if (use_decode(tokens, k, *experts))
