@@ -344,7 +344,15 @@ WM_EXPORT int wm_linear_bf16(const void* x, const void* w, int32_t tokens, int32
       check_launch("linear_rows");
       return;
     }
-    if (gemm) {
+    // Outputs of few weights, from 17 tokens: a wave each. The GEMM gives them one or a few blocks, which
+    // take 4.4 us + 1.6 ns a K value however little they compute. Measured (waves / GEMM, us; x just written by
+    // another kernel, in brackets read before): 17 to 63 tokens of 1024 and 64 outputs 6.5 / 8.2 (3.2 / 6.0), of
+    // 2560 and 8 10.0 / 10.3 (4.2 / 8.0), of 7168 and 32 19 / 19 (7.9 / 16.4), 100 tokens of that 22.4 / 20.1; of more
+    // weights, 4096 and 128 13.6 / 12.1 (5.5 / 9.6), 2048 and 512 13.9 / 8.7 (5.8 / 6.1). Rows below 512 values
+    // cost as much as 512.
+    const int64_t weights = (int64_t)outputs * (hidden < 512 ? 512 : hidden);
+    const bool waves = tokens > 16 && weights <= 1 << 18 && tokens * weights <= 15000000;
+    if (gemm && !waves) {
       GemmArgs g{};
       g.x = (const uint16_t*)x;
       g.w = (const uint16_t*)w;
