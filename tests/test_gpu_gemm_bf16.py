@@ -60,7 +60,8 @@ def test_mlp_edges(T, H, I, gated):
 
 @pytest.mark.parametrize("T,H,E,gated", [(7, 2048, 64, True), (8, 2048, 65, True), (15, 4128, 33, False), (16, 4128, 33, True),
                                          (40, 1024, 512, True), (301, 1056, 130, True), (9, 40, 16, True),
-                                         (20, 10240, 32, True), (17, 10272, 16, True)])
+                                         (20, 10240, 32, True), (17, 10272, 16, True), (129, 9600, 64, True), (96, 9600, 64, True),
+                                         (33, 9600, 256, False)])
 def test_norm_router_edges(T, H, E, gated):
     g = torch.Generator(device="cuda")
     g.manual_seed(T + H + E)

@@ -304,10 +304,6 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const float* __restr
 }
 
 constexpr int NORM_MAX_HIDDEN = 10240;
-// Tokens from which the two launches are faster than the fused kernel below (hidden 2560, 512
-// experts: 4 tokens 10.9 us against 9.1, 8 tokens 11.6 against 15.8; hidden 7168, 256 experts, whose GEMM has half
-// the blocks: 8 tokens 18.8 against 18.0, 15 tokens 21.3 against 17.5).
-static int norm_gemm_min_tokens(int hidden) { return hidden <= 4096 ? 8 : 16; }
 
 static void residual_norm(const float* r, const uint16_t* y, const uint16_t* nw, int tokens, int hidden, float eps,
                           const uint16_t* gate, uint16_t* x, float* r_out, float* shared_logit, hipStream_t s) {
@@ -334,6 +330,19 @@ static int pick_token_block(int tokens, int hidden) {
   const int fit = (96 * 1024 - 64) / (hidden * 2);
   for (int tb : {16, 8, 4, 2}) if (tb <= fit && tokens >= tb) return tb;
   return 1;
+}
+
+// Whether the two launches are faster than the fused kernel (us, fused / two launches). Up to hidden 6144 from 8
+// tokens, where a fused block builds the rows of 8 or 16 tokens one after another: 2560, 512 experts: 4 tokens
+// 9.1 / 10.9, 8 tokens 15.8 / 11.6; 4160, 512 experts, 16 tokens 26.5 / 15.6; 5120, 384: 24.4 / 19.2. Wider rows, whose
+// fused blocks hold 4 tokens and whose GEMM takes as long as its K, once those blocks pass one round of
+// the chip (about 20 us a round): hidden 7168: 32 experts 96 tokens (240 blocks of 512) 20.2 / 24.2, 256 experts 24 tokens
+// (390) 22.2 / 24.0; 9600: 64 experts 96 tokens (408) 27.8 / 29.5, 128 tokens (544) 46 / 29.7.
+static bool norm_gemm_wins(int tokens, int hidden, int rows) {
+  if (hidden <= 6144) return tokens >= 8;
+  const int tb = pick_token_block(tokens, hidden);
+  const int64_t blocks = (int64_t)((rows + 3) / 4) * ((tokens + tb - 1) / tb);
+  return blocks > 256 * (160 * 1024 / (tb * hidden * 2 + 64));  // CUs, blocks a CU by their LDS
 }
 
 }  // namespace wm
@@ -393,7 +402,7 @@ WM_EXPORT int wm_norm_router(const float* residual, const void* y, const void* n
       if (p && ((uintptr_t)p % 16)) fail("wm_norm_router: tensors must be 16-byte aligned");
     hipStream_t s = as_stream(stream);
     const int rows = experts + (shared_gate ? 1 : 0);
-    if (tokens >= norm_gemm_min_tokens(hidden) && hidden <= NORM_MAX_HIDDEN && gemm_bf16_fits(x, router, hidden)) {
+    if (hidden <= NORM_MAX_HIDDEN && gemm_bf16_fits(x, router, hidden) && norm_gemm_wins(tokens, hidden, rows)) {
       residual_norm(residual, (const uint16_t*)y, (const uint16_t*)norm_weight, tokens, hidden, eps,
                     (const uint16_t*)shared_gate, (uint16_t*)x, residual_out, shared_logit, s);
       GemmArgs g{};
