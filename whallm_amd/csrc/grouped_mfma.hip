@@ -1638,9 +1638,17 @@ static Layout layout(int tokens, int k, int experts, int hidden, int inter, bool
 //   FP8 7168/2048, 256 experts top 8: 64 2490/1507, 2048 3190/2882, 4096 4722/4750; skewed 4642/4279
 // Where it loses its 3% (64 to 128 rows for every expert) the host, which knows the mean and not the
 // counts, cannot tell it from the skewed call that gains 9%.
-// ROWS_16, MXFP4 at up to 8 rows an expert: mixed / 16 rows, 2048/512: 1.2 rows 202/145, 5.9 268/202
-// (skewed 80/65, 121/120; at 11.7 skewed 152/181); 5120/2304: 1.0 934/846. Tokens are bounded since
-// the shared expert's rows take tiles of 16 too.
+// ROWS_16, MXFP4 at up to 8 rows an expert on average. It reads an expert's weights once per 16 rows, so
+// skewed routing ends its lead as the tokens grow, the sooner the larger the experts (128-row tiles / mixed
+// / 16 rows, even routing, then Zipf 1.1; row layout):
+//   5120/2304, 384 experts top 6: 64 tokens 1805/988/872, 407/263/233; 128 tokens 2372/1318/1166, 420/292/353;
+//     256 tokens 2768/1500/1433, 593/389/555; 512 tokens 2875/1602/1615, 787/564/910
+//   2560/640, 512 experts top 10: 128 tokens 556/337/280, 177/126/110; 409 tokens 637/381/347, 214/169/204
+//   2048/512: 512 experts top 10: 301 tokens 405/256/201, 112/112/116; 1024 experts top 8: 384 tokens
+//     653/427/337, 114/114/118; 512 tokens 664/432/355, 117/118/143
+// So up to 256 tokens of large experts and 416 of small ones, where skewed calls still beat the 128-row tiles or
+// are within 4% of them. Only calls of identical tokens (all in the same k experts) lose there: 5120/2304, 128 tokens
+// 191/199/207, 256 tokens 194/200/365.
 // The streaming kernels need two weight units a tile (FP8 256, MXFP4 384 wide); E2M3 terms have only
 // 128-row tiles.
 enum RowTiles {
@@ -1651,7 +1659,8 @@ enum RowTiles {
 static RowTiles row_tiles(bool e4m3, bool fp8, int tokens, int k, int experts, int hidden, int inter) {
   const int least = fp8 ? 256 : 384;
   if (!e4m3 || hidden < least || inter < least) return ROWS_128;
-  if (!fp8 && tokens <= 512 && (int64_t)tokens * k <= (int64_t)8 * experts) return ROWS_16;
+  const int most = (int64_t)hidden * inter <= 1 << 21 ? 416 : 256;
+  if (!fp8 && tokens <= most && (int64_t)tokens * k <= (int64_t)8 * experts) return ROWS_16;
   return ROWS_MIXED;
 }
 
