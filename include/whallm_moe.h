@@ -209,7 +209,7 @@ WM_EXPORT int wm_combine_pairs(const void* rows, const float* weights, int32_t t
  * MLP (qwen4_exp.py:763-771) with shared_expert_gate (:1002-1003, :1045); native
  * engine.mm:2075-2079. x [T, H], gate_w / up_w [I, H], down_w [H, I], gate_vec [H], add and y
  * [T, H], all bf16 and 16-byte aligned; add (nullable) may alias y. H and I multiples of
- * 32. Up to 4 tokens run two GEMV kernels, more the bf16 MFMA GEMM of wm_linear_bf16; at 64 or
+ * 32. Up to 5 tokens run two GEMV kernels, more the bf16 MFMA GEMM of wm_linear_bf16; at 64 or
  * more tokens H and I are at most 9568.
  * workspace: wm_mlp_bf16_workspace_size bytes. */
 WM_EXPORT size_t wm_mlp_bf16_workspace_size(int32_t tokens, int32_t hidden, int32_t inter);

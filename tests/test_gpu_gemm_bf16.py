@@ -40,7 +40,8 @@ def test_linear_edges(T, K, N):
     check_sums(wa.linear_bf16(x, w), x, w)
 
 
-@pytest.mark.parametrize("T,H,I", [(1, 32, 32), (2, 2592, 96), (4, 2048, 2080), (5, 32, 32), (33, 96, 160), (63, 2080, 640),
+@pytest.mark.parametrize("T,H,I", [(1, 32, 32), (2, 2592, 96), (4, 2048, 2080), (5, 32, 32), (5, 1056, 544),
+                                   (3, 544, 1056), (6, 544, 32), (33, 96, 160), (63, 2080, 640),
                                    (129, 288, 96), (700, 96, 544), (2049, 1056, 2080)])
 @pytest.mark.parametrize("gated", [True, False])
 def test_mlp_edges(T, H, I, gated):

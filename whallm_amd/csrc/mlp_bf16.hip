@@ -6,8 +6,10 @@
 // engine runs the same three linears with a mul_silu (Native/QwenNative/engine.mm:2075-2079).
 // Weights are bf16 [I, H] (gate, up) and [H, I] (down), y = x W^T as mlx nn.Linear.
 //
-// Up to 4 tokens (decode): two GEMV kernels, a wave per intermediate row (gate and up rows)
-// and a wave per output row, four 16-byte chunks of each row and of every token in flight.
+// Up to 5 tokens (decode): two GEMV kernels, a wave per intermediate row (gate and up rows)
+// and a wave per output row, up to four 16-byte chunks of each row and of every token in flight: as many as
+// the row has for a lane, since the ones past its end are loads too (96/32, 1 token: 6.0 us, 6.4 with four; 2560/640,
+// 4 tokens 10.4, 11.2).
 // More: the bf16 GEMM of gemm_bf16.hip twice, with the SwiGLU and the tokens' gate values in
 // the first launch and the gate and add in the second.
 // Measured (hidden 2560, intermediate 640): 8 tokens 24.3 us as GEMVs that looped over the
@@ -22,7 +24,9 @@ namespace wm {
 // The widths of the interface at 64 or more tokens.
 constexpr int MLP_MAX_WIDTH = 9568;
 
-constexpr int MLP_GEMV_MAX_TOKENS = 4;
+// Tokens of the GEMVs (5 tokens, GEMVs / GEMMs, us: 2048/512 9.3/13.2, 2560/640 11.8/15.3, 7168/2048 32.3/32.4,
+// 96/32 7.9/6.5).
+static int mlp_gemv_max_tokens(int hidden) { return hidden <= 512 ? 4 : 5; }
 
 // dot of 8 bf16 (one 16-byte chunk) against 8 bf16
 __device__ __forceinline__ float dot8_bf16(uint4 a, uint4 b, float acc) {
@@ -79,7 +83,7 @@ __device__ __forceinline__ void wave_dots(const uint4* const (&wr)[R], const uin
 
 // grid: ceil(I / 4) + 1; wave w of block b owns intermediate row i = 4 b + w; the last block
 // the tokens' gate values.
-template <int TMAX>
+template <int TMAX, int UNROLL>
 __global__ void __launch_bounds__(256) mlp_gate_up_gemv_kernel(const uint16_t* __restrict__ x, int tokens, int hidden,
                                                                int inter, const uint16_t* __restrict__ wg,
                                                                const uint16_t* __restrict__ wu,
@@ -88,9 +92,9 @@ __global__ void __launch_bounds__(256) mlp_gate_up_gemv_kernel(const uint16_t* _
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int i = blockIdx.x * 4 + wave;
   if (blockIdx.x == gridDim.x - 1) {
-    if (wave < tokens) {  // at most 4 tokens
-      const float g = wave_gate(x + (int64_t)wave * hidden, gate_vec, hidden, lane);
-      if (lane == 0) gate[wave] = g;
+    for (int t = wave; t < tokens; t += 4) {
+      const float g = wave_gate(x + (int64_t)t * hidden, gate_vec, hidden, lane);
+      if (lane == 0) gate[t] = g;
     }
     return;
   }
@@ -98,14 +102,14 @@ __global__ void __launch_bounds__(256) mlp_gate_up_gemv_kernel(const uint16_t* _
   const uint4* rows[2] = {reinterpret_cast<const uint4*>(wg + (int64_t)i * hidden),
                           reinterpret_cast<const uint4*>(wu + (int64_t)i * hidden)};
   float acc[2][TMAX];
-  wave_dots<TMAX, 2, 4>(rows, reinterpret_cast<const uint4*>(x), tokens, hidden / 8, lane, acc);
+  wave_dots<TMAX, 2, UNROLL>(rows, reinterpret_cast<const uint4*>(x), tokens, hidden / 8, lane, acc);
 #pragma unroll
   for (int t = 0; t < TMAX; ++t)
     if (t < tokens && lane == 0) act[(int64_t)t * inter + i] = f32_to_bf16_bits(silu(acc[0][t]) * acc[1][t]);
 }
 
 // grid: ceil(H / 4); wave w of block b owns output row o = 4 b + w.
-template <int TMAX>
+template <int TMAX, int UNROLL>
 __global__ void __launch_bounds__(256) mlp_down_gemv_kernel(const uint16_t* __restrict__ act, int tokens, int hidden,
                                                             int inter, const uint16_t* __restrict__ wd,
                                                             const float* __restrict__ gate, const uint16_t* add,
@@ -115,7 +119,7 @@ __global__ void __launch_bounds__(256) mlp_down_gemv_kernel(const uint16_t* __re
   if (o >= hidden) return;
   const uint4* rows[1] = {reinterpret_cast<const uint4*>(wd + (int64_t)o * inter)};
   float acc[1][TMAX];
-  wave_dots<TMAX, 1, 4>(rows, reinterpret_cast<const uint4*>(act), tokens, inter / 8, lane, acc);
+  wave_dots<TMAX, 1, UNROLL>(rows, reinterpret_cast<const uint4*>(act), tokens, inter / 8, lane, acc);
 #pragma unroll
   for (int t = 0; t < TMAX; ++t)
     if (t < tokens && lane == 0) {
@@ -172,20 +176,31 @@ WM_EXPORT int wm_mlp_bf16(const void* x, int32_t tokens, int32_t hidden, int32_t
     float* gate = (float*)(ws + p.gate);
     uint16_t* act = (uint16_t*)(ws + p.act);
     const uint16_t *xb = (const uint16_t*)x, *gv = (const uint16_t*)gate_vec, *ab = (const uint16_t*)add;
-    if (tokens <= MLP_GEMV_MAX_TOKENS) {
-#define WM_MLP(T)                                                                                                     \
-  do {                                                                                                                \
-    hipLaunchKernelGGL(mlp_gate_up_gemv_kernel<T>, dim3((inter + 3) / 4 + 1), dim3(256), 0, s, xb, tokens, hidden,    \
-                       inter, (const uint16_t*)gate_w, (const uint16_t*)up_w, gv, act, gate);                         \
-    check_launch("mlp_gate_up_gemv");                                                                                 \
-    hipLaunchKernelGGL(mlp_down_gemv_kernel<T>, dim3((hidden + 3) / 4), dim3(256), 0, s, act, tokens, hidden, inter,  \
-                       (const uint16_t*)down_w, gate, ab, (uint16_t*)y);                                              \
-    check_launch("mlp_down_gemv");                                                                                    \
+    if (tokens <= mlp_gemv_max_tokens(hidden)) {
+#define WM_GU(T, U)                                                                                                \
+  hipLaunchKernelGGL((mlp_gate_up_gemv_kernel<T, U>), dim3((inter + 3) / 4 + 1), dim3(256), 0, s, xb, tokens, hidden, inter, \
+                     (const uint16_t*)gate_w, (const uint16_t*)up_w, gv, act, gate)
+#define WM_DN(T, U)                                                                                                \
+  hipLaunchKernelGGL((mlp_down_gemv_kernel<T, U>), dim3((hidden + 3) / 4), dim3(256), 0, s, act, tokens, hidden, inter,    \
+                     (const uint16_t*)down_w, gate, ab, (uint16_t*)y)
+#define WM_MLP(T)                                                                                                  \
+  do {                                                                                                             \
+    if (hidden <= 512) WM_GU(T, 1);                                                                                \
+    else if (hidden <= 1024) WM_GU(T, 2);                                                                          \
+    else WM_GU(T, 4);                                                                                              \
+    check_launch("mlp_gate_up_gemv");                                                                              \
+    if (inter <= 512) WM_DN(T, 1);                                                                                 \
+    else if (inter <= 1024) WM_DN(T, 2);                                                                           \
+    else WM_DN(T, 4);                                                                                              \
+    check_launch("mlp_down_gemv");                                                                                 \
   } while (0)
       if (tokens <= 1) WM_MLP(1);
       else if (tokens <= 2) WM_MLP(2);
-      else WM_MLP(4);
+      else if (tokens <= 4) WM_MLP(4);
+      else WM_MLP(5);
 #undef WM_MLP
+#undef WM_DN
+#undef WM_GU
       return;
     }
     GemmArgs g{};
