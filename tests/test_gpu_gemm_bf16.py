@@ -27,7 +27,7 @@ def check_sums(got, x, w):
 
 # kernel for kernel: GEMV (<= 4 tokens), small, a wave per output and either side of its line, split, 64 x 64 tiles,
 # 128 x 128 tiles
-@pytest.mark.parametrize("T,K,N", [(1, 32, 1), (4, 2080, 33), (3, 1032, 4097),
+@pytest.mark.parametrize("T,K,N", [(1, 32, 1), (4, 2080, 33), (3, 1032, 4097), (2, 512, 65), (2, 520, 65),
                                    (5, 32, 1), (16, 96, 513), (17, 2592, 512), (64, 2048, 77),
                                    (17, 32, 1), (63, 1056, 65), (6000, 32, 4), (57, 8192, 32), (58, 8192, 32), (65536, 32, 1),
                                    (33, 32, 1000), (129, 160, 640), (300, 416, 520),

@@ -196,13 +196,13 @@ __device__ __forceinline__ float dot8_bf16x(uint4 a, uint4 b, float acc) {
 // not the weights, the larger read at 4 tokens); non-temporal weight loads (3% off a verify step).
 // ROWS 1, below LR_MIN_OUTPUTS: a wave per row puts four times the waves on the few rows, and
 // eight chunks of the row and of every x are in flight at once: one memory round trip for 4096
-// values (512 rows of 2560, 1 token: 2.3 us against 4.9 with 4 rows and two chunks in flight).
+// values (512 rows of 2560, 1 token: 2.3 us against 4.9 with 4 rows and two chunks in flight); one where
+// the row has no more for a lane, since those past its end are loads too (16 rows of 32: 2.6 us, 2.85 with eight).
 constexpr int LR_ROWS = 4;
 constexpr int LR_MIN_OUTPUTS = 4096;
-template <int TMAX, int ROWS>
+template <int TMAX, int ROWS, int UNROLL>
 __global__ void __launch_bounds__(256) linear_rows_kernel(const uint4* __restrict__ x, const uint4* __restrict__ w,
                                                          int tokens, int chunks, int outputs, float* __restrict__ out) {
-  constexpr int UNROLL = ROWS == 1 ? 8 : 2;
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int o0 = (blockIdx.x * 4 + wave) * ROWS;
   if (o0 >= outputs) return;
@@ -331,14 +331,19 @@ WM_EXPORT int wm_linear_bf16(const void* x, const void* w, int32_t tokens, int32
     // More: the GEMM (8 tokens of the large one 432 us streamed, 312 as a GEMM).
     if (rows16 && tokens <= (gemm ? 4 : 16)) {
       const int chunks = hidden / 8;
-#define WM_LR(T, R) hipLaunchKernelGGL((linear_rows_kernel<T, R>), dim3((outputs + 4 * R - 1) / (4 * R)), dim3(256), 0, \
-                                       as_stream(stream), (const uint4*)x, (const uint4*)w, tokens, chunks, outputs, out)
-#define WM_LRT(T) do { if (outputs < LR_MIN_OUTPUTS) WM_LR(T, 1); else WM_LR(T, LR_ROWS); } while (0)
+#define WM_LR(T, R, U) hipLaunchKernelGGL((linear_rows_kernel<T, R, U>), dim3((outputs + 4 * R - 1) / (4 * R)), dim3(256), 0, \
+                                          as_stream(stream), (const uint4*)x, (const uint4*)w, tokens, chunks, outputs, out)
+#define WM_LRT(T)                                                 \
+  do {                                                            \
+    if (outputs >= LR_MIN_OUTPUTS) WM_LR(T, LR_ROWS, 2);          \
+    else if (chunks <= 64) WM_LR(T, 1, 1);                        \
+    else WM_LR(T, 1, 8);                                          \
+  } while (0)
       if (tokens <= 1) WM_LRT(1);
       else if (tokens <= 2) WM_LRT(2);
       else if (tokens <= 4) WM_LRT(4);
-      else if (tokens <= 8) WM_LR(8, LR_ROWS);
-      else WM_LR(16, LR_ROWS);
+      else if (tokens <= 8) WM_LR(8, LR_ROWS, 2);
+      else WM_LR(16, LR_ROWS, 2);
 #undef WM_LRT
 #undef WM_LR
       check_launch("linear_rows");
