@@ -167,3 +167,15 @@ def test_residual_rmsnorm_matches_oracle(device, T, H, with_y):
     want_r = r0 + (y.float().cpu().numpy() if with_y else 0.0)
     np.testing.assert_array_equal(r.cpu().numpy(), want_r.astype(np.float32))
     check_x(x.float().cpu().numpy(), M.rms_norm(want_r, 1e-6))
+
+
+@pytest.mark.parametrize("T", [3, 40])
+def test_residual_without_y_keeps_its_bits(device, T):
+    """With no y, residual_out is the residual bit for bit, negative zeros too, in either launch form."""
+    rng = np.random.default_rng(T)
+    r = torch.from_numpy(rng.standard_normal((T, 2048)).astype(np.float32)).to(device)
+    r[:, ::7] = -0.0
+    v = torch.empty_like(r)
+    x, _, _ = wa.norm_router(r, None, bf16_tensor(rng, (64, 2048), device, 0.05), residual_out=v)
+    assert torch.equal(v.view(torch.int32), r.view(torch.int32))
+    assert bool((x[:, ::7].view(torch.int16) == -32768).all())

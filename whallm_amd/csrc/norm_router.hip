@@ -258,10 +258,12 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const float* __restr
   float ss = 0.0f;
 #pragma unroll
   for (int j = 0; j < Q; ++j) {
-    v[j].x += bf16_bits_to_f32(b[j].x & 0xffffu);
-    v[j].y += bf16_bits_to_f32(b[j].x >> 16);
-    v[j].z += bf16_bits_to_f32(b[j].y & 0xffffu);
-    v[j].w += bf16_bits_to_f32(b[j].y >> 16);
+    if (yy) {  // without y, v is r with the sign of its zeros
+      v[j].x += bf16_bits_to_f32(b[j].x & 0xffffu);
+      v[j].y += bf16_bits_to_f32(b[j].x >> 16);
+      v[j].z += bf16_bits_to_f32(b[j].y & 0xffffu);
+      v[j].w += bf16_bits_to_f32(b[j].y >> 16);
+    }
     if ((int)threadIdx.x + 256 * j < quads) ss += v[j].x * v[j].x + v[j].y * v[j].y + v[j].z * v[j].z + v[j].w * v[j].w;
   }
   ss = segment_sum<64>(ss);
