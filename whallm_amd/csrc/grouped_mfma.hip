@@ -1630,14 +1630,14 @@ static Layout layout(int tokens, int k, int experts, int hidden, int inter, bool
   return p;
 }
 
-// How a call's row tiles are made. ROWS_MIXED is the general one: it was the fastest or within 3%
-// of it at every size measured (us of a whole call, tiled weights, 128-row tiles alone / mixed):
-//   MXFP4 2048/512, 512 experts top 10, even routing: 64 tokens 273/202, 1200 402/294, 2048 416/376,
-//     4096 466/479, 16384 1278/1292; skewed (Zipf 1.1): 97/80, 200/198, 272/249, 441/405, 1230/1227
-//   MXFP4 5120/2304, 384 experts top 6: 64 1543/934, 2048 2684/2038, 4096 2922/2747; skewed 2231/2068
-//   FP8 7168/2048, 256 experts top 8: 64 2490/1507, 2048 3190/2882, 4096 4722/4750; skewed 4642/4279
-// Where it loses its 3% (64 to 128 rows for every expert) the host, which knows the mean and not the
-// counts, cannot tell it from the skewed call that gains 9%.
+// How a call's row tiles are made. ROWS_MIXED is the general one: it was the fastest or within 1%
+// of it at every size measured (us of a whole call, row layout, 128-row tiles alone / mixed, even routing, then Zipf 1.1):
+//   MXFP4 2048/512, 512 experts top 10: 64 tokens 275/183, 103/83; 2048 tokens 432/317, 288/245; 4096 tokens 488/491,
+//     393/378; 8192 tokens 844/846, 743/676
+//   MXFP4 4096/2048, 128 experts top 8: 2048 tokens 1152/1154, 1303/1073; 4096 tokens 1849/1849, 2100/1857
+//   MXFP4 2048/768, 128 experts top 8: 2048 tokens 279/281, 276/261; 8 experts of 4096/14336 top 2: 2048 tokens
+//     1924/1921, 1999/1998
+//   FP8 7168/2048, 256 experts top 8: 2048 tokens 3690/3055, 3372/2754; 4096 tokens 5479/5460, 5328/4669
 // ROWS_16, MXFP4 at up to 8 rows an expert on average. It reads an expert's weights once per 16 rows, so
 // skewed routing ends its lead as the tokens grow, the sooner the larger the experts (128-row tiles / mixed
 // / 16 rows, even routing, then Zipf 1.1; row layout):
@@ -1778,11 +1778,12 @@ static void run(const uint16_t* x, int tokens, const int32_t* indices, const flo
   if constexpr (F::Terms::E4) {
     if (how == ROWS_MIXED) {
       const dim3 all((unsigned)(std::max(cus / XCDS, 1) * XCDS));
-      hipLaunchKernelGGL((mixed_gate_up_kernel<F, Table>), all, dim3(512), 0, s, x6, x6s, row_token, L, cold, routed, sh, a6,
-                         a6s);
+      MixedArgs<Table> ma{x6, x6s, row_token, L, cold, routed, sh, a6, a6s, out_rows};
+      hipLaunchKernelGGL((mixed_gate_up_kernel<F, Table>), all, dim3(512), 0, s, ma);
       mid();
-      hipLaunchKernelGGL((mixed_down_kernel<F, Table>), all, dim3(512), 0, s, a6, (const uint8_t*)a6s, L, cold, routed, sh,
-                         out_rows);
+      ma.terms = a6;
+      ma.scales = (const uint8_t*)a6s;
+      hipLaunchKernelGGL((mixed_down_kernel<F, Table>), all, dim3(512), 0, s, ma);
     }
   }
   if (how == ROWS_128) {

@@ -592,26 +592,43 @@ template <typename F>
 constexpr int MIXED_LDS = RingMx<F, F::DA, F::DB>::BYTES > StreamOf<F>::BYTES ? RingMx<F, F::DA, F::DB>::BYTES
                                                                               : StreamOf<F>::BYTES;
 
+template <typename Table>
+struct MixedArgs {
+  const uint8_t *terms, *scales;  // x's (gate_up) or act's (down)
+  const int32_t* row_token;
+  Lists hot, cold;
+  Table routed, shared;
+  uint8_t* a8;
+  uint32_t* a8s;
+  uint16_t* out;
+};
+// The launch's arguments read again from its argument buffer. The second part's copies of pointers and table fields
+// otherwise live through the first, whose tiles then spill and reload scalar registers at each set-up.
+template <typename Args>
+__device__ __forceinline__ const Args& args_again() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Args*)p;
+}
+
 template <typename F, typename Table>
-__global__ void __launch_bounds__(512, 2) mixed_gate_up_kernel(const uint8_t* __restrict__ x8, const uint8_t* __restrict__ x8s,
-                                                               const int32_t* __restrict__ row_token, Lists hot,
-                                                               Lists cold, Table routed, Table shared,
-                                                               uint8_t* __restrict__ a8, uint32_t* __restrict__ a8s) {
+__global__ void __launch_bounds__(512, 2) mixed_gate_up_kernel(MixedArgs<Table> a) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[MIXED_LDS<F>];
-  gate_up_mx<F, F::DA, F::DB>(lds, x8, x8s, row_token, hot, routed, shared, a8, a8s);
+  gate_up_mx<F, F::DA, F::DB>(lds, a.terms, a.scales, a.row_token, a.hot, a.routed, a.shared, a.a8, a.a8s);
   ring_wait_all();  // no load into the rings and no LDS access of the first part is left
-  stream_gate_up<StreamOf<F>>(lds, x8, x8s, row_token, cold, routed, shared,
-                              active_row_tiles(hot) * ((routed.inter + F::TW / 2 - 1) / (F::TW / 2)), 0, 0, a8, (uint8_t*)a8s);
+  const MixedArgs<Table>& b = args_again<MixedArgs<Table>>();
+  stream_gate_up<StreamOf<F>>(lds, b.terms, b.scales, b.row_token, b.cold, b.routed, b.shared,
+                              active_row_tiles(b.hot) * ((b.routed.inter + F::TW / 2 - 1) / (F::TW / 2)), 0, 0, b.a8,
+                              (uint8_t*)b.a8s);
 }
 template <typename F, typename Table>
-__global__ void __launch_bounds__(512, 2) mixed_down_kernel(const uint8_t* __restrict__ a8, const uint8_t* __restrict__ a8s,
-                                                            Lists hot, Lists cold, Table routed, Table shared,
-                                                            uint16_t* __restrict__ out) {
+__global__ void __launch_bounds__(512, 2) mixed_down_kernel(MixedArgs<Table> a) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[MIXED_LDS<F>];
-  down_mx<F, F::DA, F::DB>(lds, a8, a8s, hot, routed, shared, out);
+  down_mx<F, F::DA, F::DB>(lds, a.terms, a.scales, a.hot, a.routed, a.shared, a.out);
   ring_wait_all();
-  stream_down<StreamOf<F>>(lds, a8, a8s, cold, routed, shared, active_row_tiles(hot) * ((routed.hidden + F::TW - 1) / F::TW),
-                           0, out);
+  const MixedArgs<Table>& b = args_again<MixedArgs<Table>>();
+  stream_down<StreamOf<F>>(lds, b.terms, b.scales, b.cold, b.routed, b.shared,
+                           active_row_tiles(b.hot) * ((b.routed.hidden + F::TW - 1) / F::TW), 0, b.out);
 }
 
 }  // namespace mf
