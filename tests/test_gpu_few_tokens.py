@@ -57,8 +57,8 @@ def test_few_tokens_match_oracle(device, T, k, E, H, I):
 
 
 def test_few_tokens_slots_masks_and_replays(device):
-    """Non-resident and out-of-range experts add nothing (zero rows per pair), a masked pair's row is left
-    as it is, and a captured call gives the same bits on every replay."""
+    """Non-resident and out-of-range experts add nothing (zero rows per pair), a masked pair adds nothing and leaves
+    its row of `out` as it is, and a captured call gives the same bits on every replay."""
     rng = np.random.default_rng(7)
     T, k, E, H, I = 6, 4, 12, 2560, 2048
     slots = np.arange(E, dtype=np.int32)
@@ -66,10 +66,13 @@ def test_few_tokens_slots_masks_and_replays(device):
     tab = S.experts_to_device(S.mxfp4_experts_np(rng, E, H, I), device, slots=torch.from_numpy(slots).to(device), experts=E)
     x = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (T, H)), device)
     ids = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)
-    ids[0, 0], ids[1, 1] = 5, E
-    live = (ids != 5) & (ids != E)
+    ids[0, 0], ids[1, 1], ids[2, 2] = 5, E, -1
+    live = (ids != 5) & (ids != E) & (ids >= 0)
     i_d, w_d = torch.from_numpy(ids).to(device), torch.rand(T, k, device=device) + 0.1
-    per_pair = wa.experts_mxfp4(x, i_d, tab).double()
+    per_pair = wa.experts_mxfp4(x, i_d, tab, out=torch.full((T, k, H), 3.0, dtype=torch.bfloat16, device=device))
+    assert bool((per_pair[2, 2] == 3).all())
+    per_pair[2, 2] = 0
+    per_pair = per_pair.double()
     assert bool((per_pair[torch.from_numpy(~live).to(device)] == 0).all())
     want = (per_pair * w_d.double()[..., None]).sum(1)
     got = wa.moe_mxfp4(x, i_d, w_d, tab)
@@ -160,3 +163,22 @@ def test_few_tokens_read_nothing_for_what_is_not_resident(device):
     torch.cuda.synchronize()
     assert bool((y == 0).all())
     assert int((ws == 0x5a).sum()) >= 4 * H * T * (k + 1) + 2 * I * T * (k + 1)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_few_tokens_keep_what_is_not_finite_to_its_token(device, value):
+    """A NaN or an infinity in x makes its own token's results NaN, as in 64 bits (an infinity meets weights of
+    both signs and zeros), and changes no bit of the others', in rows of the same tiles."""
+    rng = np.random.default_rng(11)
+    T, k, E, H, I = 8, 4, 6, 2560, 2048
+    tab, shared = (S.experts_to_device(S.mxfp4_experts_np(rng, n, H, I), device) for n in (E, 1))
+    x = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (T, H)), device)
+    i = torch.from_numpy(np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.int32)).to(device)
+    w = torch.rand(T, k, device=device) + 0.1
+    bad = x.clone()
+    bad[3, 100] = value
+    rest = [t for t in range(T) if t != 3]
+    for got, want in ((wa.moe_mxfp4(bad, i, w, tab, shared), wa.moe_mxfp4(x, i, w, tab, shared)),
+                      (wa.experts_mxfp4(bad, i, tab), wa.experts_mxfp4(x, i, tab))):
+        assert torch.equal(got[rest], want[rest])
+        assert bool(got[3].isnan().all())

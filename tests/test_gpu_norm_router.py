@@ -40,10 +40,10 @@ def check_dot(got, x, w):
     (1, 2560, 512, True, False, True),       # C2 decode: one token, Qwen router + shared gate
     (3, 2048, 128, True, True, True),        # ragged token block
     (40, 4096, 256, False, True, False),     # DeepSeek width, no y, no gate
-    (300, 2560, 512, True, True, True),      # MFMA path, 16-token blocks, ragged last block
-    (20, 7168, 256, True, False, True),      # MFMA path, 8-token blocks (C4 width)
-    (70, 2048, 512, True, True, True),       # MFMA path, 32-token blocks (two column blocks), ragged tail
-    (17, 1000, 64, True, True, True),        # hidden not a multiple of 32: dot-product path, 16 tokens
+    (300, 2560, 512, True, True, True),      # norm, then the GEMM: a prompt
+    (20, 7168, 256, True, False, True),      # the one launch at the DeepSeek width, blocks of 4 tokens
+    (70, 2048, 512, True, True, True),       # norm, then the GEMM: a ragged token tile
+    (17, 1000, 64, True, True, True),        # hidden not a multiple of 32: the one launch, 16 tokens
 ])
 def test_norm_router_matches_oracle(device, T, H, E, with_y, with_w, with_gate):
     rng = np.random.default_rng(T + H + E)
@@ -112,9 +112,8 @@ def test_empty_and_error_paths(device):
 @pytest.mark.parametrize("T,H,E,with_gate", [(300, 2560, 512, True), (20, 7168, 256, True), (64, 2048, 40, False),
                                              (1, 2048, 512, True)])
 def test_packed_router_is_bit_identical(device, T, H, E, with_gate):
-    """repack_router's fragment order (checked against a torch permute of the zero-padded
-    rows) feeds the prefill GEMM the same operands, so logits are bit-identical to the row
-    path; at one token (dot-product path) the packed copy is not read."""
+    """repack_router's fragment order (against a torch permute of the zero-padded rows). wm_norm_router
+    checks a packed router's size and reads the rows as stored, so passing one changes no bit."""
     rng = np.random.default_rng(T * 7 + E)
     r = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(device)
     y = bf16_tensor(rng, (T, H), device)
@@ -140,10 +139,9 @@ def test_packed_router_is_bit_identical(device, T, H, E, with_gate):
 @pytest.mark.parametrize("T,H,E", [(300, 2048, 512), (70, 7168, 256), (64, 1024, 64), (63, 2048, 128),
                                    (1, 2048, 512), (3, 7168, 1000), (4, 7168, 129280), (16, 1032, 77), (9, 2048, 64)])
 def test_linear_bf16_prefill_path(device, T, H, E):
-    """wm_linear_bf16 at 64+ tokens runs on the router GEMM's MFMA path (a tile of x as
-    given), up to 16 tokens on the row-streaming kernel (every weight row read once for all
-    tokens; the C5 LM head at 4 x 129,280), in between on the one-wave-per-output kernel:
-    each within the dot-product bound of the float64 product."""
+    """wm_linear_bf16 on its kernels (up to 4 tokens, or 16 with rows the GEMM does not take, every weight row
+    streamed once for all tokens, an LM head of 4 x 129,280 among them; the bf16 GEMM; a wave per output
+    for few weights): each within the dot-product bound of the float64 product."""
     rng = np.random.default_rng(T + E)
     x = bf16_tensor(rng, (T, H), device)
     w = bf16_tensor(rng, (E, H), device, 0.05)

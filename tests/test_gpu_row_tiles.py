@@ -5,6 +5,9 @@ of 128 rows, which test_gpu_moe.py and test_gpu_fp8.py hold against the oracle).
 Row counts at the edges of the tiles, K of an even and odd number of 128-wide steps, a last column tile
 of half its width, both layouts, a slot map with an expert that is not resident, ids out of range.
 All take the same products in the same order, so a row's bits do not depend on the tile that held it.
+The second test has more 64-row tiles than an XCD's 32 workgroups, so that each goes from tile to tile, over an odd
+number of K steps (its last weight unit is half of one), and with hot experts also through the tiles that
+the workgroups without a 128-row tile take first and the rest after them.
 """
 import numpy as np
 import pytest
@@ -29,6 +32,33 @@ def tables(form, rng, device, n, hidden, inter, **kw):
     if form == "mxfp4":
         return S.experts_to_device(S.mxfp4_experts_np(rng, n, hidden, inter), device, **kw)
     return S.fp8_experts_to_device(S.fp8_experts_np(rng, n, hidden, inter, scale_format=int(form == "fp8-32")), device, **kw)
+
+
+MANY = {  # tokens, choices, experts, Zipf exponent
+    "even": (100, 8, 64, 0.0),       # 320 tiles of 64 rows in either GEMM (MXFP4: 12.5 rows an expert)
+    "skewed": (600, 8, 256, 1.1),    # about 20 experts of more than 64 rows, 230 of fewer
+}
+
+
+@pytest.mark.parametrize("call", sorted(MANY))
+@pytest.mark.parametrize("form", FORMS)
+def test_row_tiles_agree_from_tile_to_tile(device, form, call):
+    T, k, E, skew = MANY[call]
+    hidden, inter = 1152, 640  # 9 and 5 K steps
+    rng = np.random.default_rng(T + E)
+    routed, shared = tables(form, rng, device, E, hidden, inter), tables(form, rng, device, 1, hidden, inter)
+    lot = rng.gumbel(size=(T, E)) - skew * np.log(np.arange(1, E + 1))  # the k largest: a draw without replacement
+    ids = np.argsort(-lot, axis=1)[:, :k]
+    counts = np.bincount(ids.ravel(), minlength=E)
+    assert (counts <= 64).sum() * 5 > 256 and (counts > 64).any() == (skew > 0)
+    more = np.stack([(np.arange(9 * E) + j * 5) % E for j in range(k)], 1)  # 72 rows for every expert
+    n = T + len(more)
+    x = S.bf16_bits_to_tensor(S.bf16_normal_np(rng, (n, hidden)), device)
+    i = torch.from_numpy(np.concatenate([ids, more]).astype(np.int32)).to(device)
+    w = torch.rand(n, k, device=device) + 0.1
+    moe = wa.moe_mxfp4 if form == "mxfp4" else wa.moe_fp8
+    for a, b in ((routed, shared), (wa.prefill_layout(routed), wa.prefill_layout(shared))):
+        assert torch.equal(moe(x[:T], i[:T], w[:T], a, b), moe(x, i, w, a, b)[:T])
 
 
 @pytest.mark.parametrize("hidden,inter", [(384, 384), (640, 384), (384, 640), (256, 256), (512, 1152)])
