@@ -284,8 +284,8 @@ WM_EXPORT int wm_residual_rmsnorm(float* residual, const void* y, int32_t tokens
  * (both nullable together). residual_out (nullable, must not overlap residual) receives v.
  * bf16 y [T, H], norm_weight [H], router [E, H], shared_gate [H]; every pointer 16-byte
  * aligned, hidden a multiple of 8. router_packed (nullable) is the same rows from
- * wm_repack_router, router_packed_bytes its size: accepted and checked, but the GEMM reads
- * router, whose rows it loads as fast. Replaces the norm dispatch and the router / shared-gate linears
+ * wm_repack_router, router_packed_bytes its size: accepted and its size checked, but no kernel
+ * reads it (the GEMM loads router's rows as fast); pass NULL. Replaces the norm dispatch and the router / shared-gate linears
  * before the expert step (Native/QwenNative/engine.mm:2074-2079; SparseMoE.gate and
  * shared_expert_gate, qwen4_exp.py:1000-1003); routing follows with wm_route_softmax_topk or
  * wm_route_scored on the device. */

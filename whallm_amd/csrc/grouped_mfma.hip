@@ -8,14 +8,14 @@
 // moe_combine_rows (Native/QwenNative/kernels.metal:691-765, engine.mm:2104-2162) and
 // mx.gather_qmm (qwen4_exp.py:857-897, model.py:435-501):
 //
-//   split   : every token row of x (bf16) becomes two E2M3 (fp6) terms, hi and lo, each
-//             with an E8M0 scale per 32 values, stored as the MFMA's B operand reads them
-//             (the GEMMs copy them to LDS unchanged).
+//   split   : every token row of x (bf16) becomes two terms, hi and lo, each with an E8M0
+//             scale per 32 values, stored as the MFMA's B operand reads them (the GEMMs copy
+//             them to LDS unchanged): E4M3 terms, or E2M3 (fp6) where the table asks for them.
 //   gate_up : tile = 128 permuted rows (64 or 16 where an expert has few: grouped_stream.h) x
 //             (TW / 2 gate + the matching up weight rows); per
 //             128-wide K step each wave runs its weight tiles x 2 row tiles x 2 halves of
 //             the step x 2 terms MFMAs. SwiGLU is the epilogue, which writes act straight
-//             back as E2M3 terms (the down GEMM's B operand).
+//             back as terms (the down GEMM's B operand).
 //   down    : tile = 128 permuted rows x TW output columns over K = intermediate; bf16
 //             rows in permuted order, unweighted.
 //   combine : y[t] = sum of the token's K rows times their routing weights in k order,
@@ -1997,10 +1997,10 @@ static void run_few(const uint16_t* x, int tokens, const int32_t* indices, const
 }  // namespace mf
 
 // The line to the GEMV is the bytes of weights that it would pass, T k times an expert's 1.5 H I: below
-// about 180 MB its two launches are the faster (us of a whole call, GEMV / here): 2048/512 top 10,
-// 8 tokens (126 MB) 45/55, 12 (189 MB) 62.5/62.8, 25 116/88; 2560/640 top 10, 6 (147 MB) 60/62, 8 (197 MB)
-// 78/67, 25 199/131; 4096/2048 top 8, 1 (101 MB) 53/59, 2 94/77, 8 326/146, 32 1205/296; 5120/2304 top 6,
-// 1 (106 MB) 51/56, 2 83/76, 8 288/187, 32 1098/550.
+// about 180 MB its two launches are the faster or level (us of a whole call, GEMV / here): 2048/512 top 10,
+// 6 tokens (94 MB) 39/41, 8 (126 MB) 48/50, 12 (189 MB) 68/61, 25 129/95; 2560/640 top 10, 3 (74 MB) 40/43,
+// 6 (147 MB) 64/59, 8 (197 MB) 82/66, 25 211/136; 4096/2048 top 8, 1 (101 MB) 59/58, 2 102/61, 8 346/149, 32
+// 1246/333; 5120/2304 top 6, 1 (106 MB) 60/54, 2 107/81, 8 349/197, 32 1272/580.
 constexpr int64_t FEW_WEIGHTS = 120000000;  // T k H I
 
 bool few_mxfp4_takes(int tokens, int k, const wm_mxfp4_experts& e) {

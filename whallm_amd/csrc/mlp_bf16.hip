@@ -21,7 +21,8 @@
 
 namespace wm {
 
-// The widths of the interface at 64 or more tokens.
+// The widths that the interface takes at 64 or more tokens: a bound of an earlier GEMM that held whole token
+// rows in LDS, which the present kernels do not need; lifting it is a change of the interface.
 constexpr int MLP_MAX_WIDTH = 9568;
 
 // Tokens of the GEMVs (5 tokens, GEMVs / GEMMs, us: 2048/512 9.3/13.2, 2560/640 11.8/15.3, 7168/2048 32.3/32.4,

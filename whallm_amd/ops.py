@@ -543,7 +543,8 @@ def residual_rmsnorm(residual: torch.Tensor, y: torch.Tensor | None, eps: float 
 
 def repack_router(router: torch.Tensor, shared_gate: torch.Tensor | None = None) -> torch.Tensor:
     """The router rows (+ the shared gate row) in MFMA fragment order (wm_repack_router).
-    norm_router(..., router_packed=) accepts it; it reads the rows as stored just as fast."""
+    norm_router(..., router_packed=) still accepts it and checks its size, but reads the rows as stored,
+    just as fast: new code has no use for it."""
     device = _require_device(router, shared_gate)
     router = _contig(router, torch.bfloat16, "router")
     E, H = router.shape
